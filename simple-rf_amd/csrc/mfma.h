@@ -74,6 +74,36 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
   }
 }
 
+// max(v, 0) in one instruction, NaN -> 0: the median of v, 0 and +inf (v_med3_f32 gives the least of
+// its operands that are numbers).  The infinity is opaque to the compiler, which would otherwise make
+// this the two instructions that fmaxf and a select also take.
+__device__ __forceinline__ float relu1(float v) {
+  float inf = __builtin_inff();
+  asm("" : "+s"(inf));
+  return __builtin_amdgcn_fmed3f(v, 0.f, inf);
+}
+
+typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
+typedef int16_t i16x2_t __attribute__((ext_vector_type(2)));
+
+// Shifts two pairs of flags into m: m = m << 1 | (a != 0), then the same for b, in each 16-bit half
+// (a, b: packed pairs of non-negative 16-bit floats).  Written out, since the compiler turns the
+// minimum with 1 into a comparison and a select for each half.
+__device__ __forceinline__ void push_nonzero(uint32_t& m, uint32_t a, uint32_t b) {
+  uint32_t t;
+  asm("v_pk_min_u16 %1, %2, %4\n\tv_lshl_or_b32 %0, %0, 1, %1\n\t"
+      "v_pk_min_u16 %1, %3, %4\n\tv_lshl_or_b32 %0, %0, 1, %1"
+      : "+v"(m), "=&v"(t)
+      : "v"(a), "v"(b), "s"(0x00010001u));
+}
+
+// 0xffff in every 16-bit half of m whose bit 15 - k is set, 0 in the other halves.
+template <int K>
+__device__ __forceinline__ uint32_t half_mask(uint32_t m) {
+  const i16x2_t s = __builtin_bit_cast(i16x2_t, __builtin_bit_cast(u16x2_t, m) << u16x2_t{K, K});
+  return __builtin_bit_cast(uint32_t, s >> i16x2_t{15, 15});
+}
+
 template <int P>
 __device__ __forceinline__ float unpack_lo(uint32_t v) {
   if constexpr (P == kBF16) return bf16_bits_to_f32(v & 0xffffu);

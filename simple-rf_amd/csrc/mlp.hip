@@ -67,19 +67,42 @@ __device__ inline int slot_k(int s, int g, int i) {
   return 32 * s + (i < 4 ? 4 * g + i : 16 + 4 * g + i - 4);
 }
 
+// Slots 8 idx .. 8 idx + 7 of the forward (bwd = 0) or transposed (1) image of layer l for 32x32x16
+// MFMAs (mlp16.h): 1 KB fragments of 32 rows x 16 features, lane 32 h + c of k-step 2 T + m holding row c
+// at features 32 T + 16 (i / 4) + 8 m + 4 h + i % 4.  The fragments lie k-step by k-step, the row tiles of one k-step together;
+// row tiles past the eighth (the sigma row) follow in the same order.
+__device__ void pack_fragment16(const PackArgs& a, int l, int bwd, int rows_t, int steps, unsigned idx) {
+  const Plan& p = a.p;
+  if (idx >= (unsigned)(rows_t * steps) * 64u) return;
+  const unsigned lane = idx & 63u, f = idx >> 6;
+  const unsigned mt = rows_t < 8 ? rows_t : 8, f1 = mt * steps;
+  const unsigned n = f < f1 ? mt : rows_t - mt, fl = f < f1 ? f : f - f1;
+  const unsigned s = fl / n;
+  const int T = (int)(fl - s * n) + (f < f1 ? 0 : 8);
+  const int row = 32 * T + (int)(lane & 31u), k0 = 32 * (int)(s >> 1) + 8 * (int)(s & 1u) + 4 * (int)(lane >> 5);
+  const int row_col = bwd ? ref_col(p, l, row) : 0;
+  uint32_t d[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int k = k0 + 16 * (i >> 2) + (i & 3);
+    const float v = bwd ? ref_weight(a, l, k, row_col) : ref_weight(a, l, row, ref_col(p, l, k));
+    d[i] = p.prec == SRF_PREC_BF16 ? f32_to_bf16_bits(v) : f32_to_f16_bits(v);
+  }
+  uint4* dst = reinterpret_cast<uint4*>(a.out + (bwd ? p.bwd_off[l] : p.fwd_off[l]));
+  dst[idx] = make_uint4(d[0] | d[1] << 16, d[2] | d[3] << 16, d[4] | d[5] << 16, d[6] | d[7] << 16);
+}
+
 // Element idx of the forward (bwd = 0) or transposed (bwd = 1) operand image of layer l.
 __device__ void pack_element(const PackArgs& a, int l, int bwd, long idx) {
   const Plan& p = a.p;
   const bool f32 = p.prec == SRF_PREC_F32;
   const bool split = p.prec == SRF_PREC_BF16_SPLIT;
   const int kpl = f32 ? 1 : 8;
-  int rows_t, k_tiles;
-  if (!bwd) {
-    rows_t = p.out_tiles[l];
-    k_tiles = p.reg_tiles[l] + p.comp_tiles[l];
-  } else {
-    rows_t = p.reg_tiles[l];
-    k_tiles = p.bwd_tiles[l];
+  const int rows_t = bwd ? p.bwd_rows_t[l] : p.fwd_rows_t[l];
+  const int k_tiles = bwd ? p.bwd_tiles[l] : p.reg_tiles[l] + p.comp_tiles[l];
+  if (p.row_tile == 32) {
+    pack_fragment16(a, l, bwd, rows_t, k_tiles, (unsigned)idx);
+    return;
   }
   const int ks = f32 ? 4 * k_tiles : k_tiles / 2;
   const long total = (long)rows_t * ks * 64 * kpl;
@@ -115,17 +138,13 @@ __device__ void pack_element(const PackArgs& a, int l, int bwd, long idx) {
       d16[(f * np + pl) * 512 + within] = (uint16_t)h;
       r = r - bf16_bits_to_f32(h);
     }
-  } else if (f32) {
-    reinterpret_cast<float*>(dst)[idx] = v;
-  } else if (p.prec == SRF_PREC_BF16) {
-    reinterpret_cast<uint16_t*>(dst)[idx] = (uint16_t)f32_to_bf16_bits(v);
   } else {
-    reinterpret_cast<uint16_t*>(dst)[idx] = (uint16_t)f32_to_f16_bits(v);
+    reinterpret_cast<float*>(dst)[idx] = v;
   }
 }
 
 __device__ void pack_bias_element(const PackArgs& a, int l, int o) {
-  if (o >= 16 * a.p.out_tiles[l]) return;
+  if (o >= a.p.row_tile * a.p.fwd_rows_t[l]) return;
   float v = 0.f;
   if (o < a.p.out_rows[l]) {
     int t, r;
@@ -228,12 +247,12 @@ extern "C" int srf_mlp_pack(const srf_mlp_desc* desc, const float* const* weight
     if (!p.present[l]) continue;
     for (int bwd = 0; bwd < 2; ++bwd) {
       if (bwd && l == 0) continue;
-      const int rows_t = bwd ? p.reg_tiles[l] : p.out_tiles[l];
+      const int rows_t = bwd ? p.bwd_rows_t[l] : p.fwd_rows_t[l];
       const int k_tiles = bwd ? p.bwd_tiles[l] : p.reg_tiles[l] + p.comp_tiles[l];
       const int ks = p.prec == SRF_PREC_F32 ? 4 * k_tiles : k_tiles / 2;
-      add(l, bwd, (long)rows_t * ks * 64 * kpl);
+      add(l, bwd, p.row_tile == 32 ? (long)rows_t * k_tiles * 64 : (long)rows_t * ks * 64 * kpl);
     }
-    add(l, 2, 16L * p.out_tiles[l]);
+    add(l, 2, (long)p.row_tile * p.fwd_rows_t[l]);
   }
   jobs.first_block[jobs.n_jobs] = blocks;
   hipLaunchKernelGGL(pack_all_kernel, dim3(blocks), dim3(256), 0, as_stream(stream), a, jobs);

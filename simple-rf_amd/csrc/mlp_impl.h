@@ -1,4 +1,6 @@
-// Fused positional encoding + NeRF MLP (kernel templates shared by mlp*.hip) (forward, backward, weight gradients) on gfx950 MFMA.
+// Fused positional encoding + NeRF MLP on gfx950 MFMA (templates shared by mlp*.hip): forward and backward
+// chain on FP32 activations (FP32 and split-BF16 operands; mlp16.h has those for 16-bit operands) and the
+// weight gradients of every precision.
 //
 // Reference semantics: MLP.forward / get_view_independent_outputs / get_view_dependent_outputs
 // and PositionalEncoder (src/models/SimpleNeRF17.py:581-785), driven by run_network/batchify
@@ -7,7 +9,7 @@
 //   points-augmented  trunk PE 21,  view layer input [feature, PE_xyz[21:63], PE_dir] = 325
 //   views-augmented   trunk PE 63,  head: 4 channels (sigma, rgb) straight from the trunk
 //
-// Design (one 64-lane wave owns 16*CB points, CB = 4 for 16-bit operands, 2 for FP32):
+// Design (one 64-lane wave owns 16*CB = 32 points; 64 in mlp16.h):
 //   * The MLP is evaluated "transposed": each layer computes H_out^T = W H_in^T with the
 //     weights as the MFMA A operand and the points as the N dimension.  With the slot map of
 //     mfma.h, the D tiles of one layer are, bit for bit, the B operand of the next layer, so
@@ -49,19 +51,21 @@ constexpr int kParams = SRF_MLP_NUM_PARAMS;
 constexpr int kMaskSlots = 9;      // ReLU masks of layers 0-7 and the view layer
 constexpr int kWaves = 4;          // waves per block
 constexpr int kMaxJobs = 16;
-// padded biases of the largest model: trunk 8 x 256, head 272, view 128, rgb 16
-constexpr int kMaxBiasFloats = 8 * 256 + 272 + 128 + 16;
+// padded biases of the largest model: trunk 8 x 256, head 288, view 128, rgb 32
+constexpr int kMaxBiasFloats = 8 * 256 + 288 + 128 + 32;
 
 // ----------------------------------------------------------------------------- plan
 struct Plan {
   int prec, view_dep, softplus, trunk_pe, pts_deg, dir_deg;
   int extra;  // computed inputs of the view layer: [PE_xyz[trunk_pe:], PE_dir]
   int elem;   // bytes per stored value
-  // bytes of the forward and of the transposed (backward) operand image per (output tile, input
-  // tile): 16 x 16 values, times the BF16 planes of the split precision
+  int row_tile;  // rows of a weight fragment: 32 for 16-bit operands (mlp16.h), else 16
+  // bytes of the forward and of the transposed (backward) operand image per (row tile, 16 input
+  // features): row_tile x 16 values, times the BF16 planes of the split precision
   int fwd_tile_bytes, bwd_tile_bytes;
   int out_rows[kLayers], out_tiles[kLayers], reg_tiles[kLayers], comp_feats[kLayers],
       comp_tiles[kLayers], bwd_tiles[kLayers], present[kLayers];
+  int fwd_rows_t[kLayers], bwd_rows_t[kLayers];  // row tiles of the forward / transposed image
   int bias_floats;  // padded biases of every present layer, contiguous from bias_off[0]
   size_t fwd_off[kLayers], bwd_off[kLayers], bias_off[kLayers], packed_bytes;
 };
@@ -85,12 +89,15 @@ inline bool make_plan(const srf_mlp_desc* d, Plan* p) {
   const bool split = d->prec == SRF_PREC_BF16_SPLIT;
   p->elem = (d->prec == SRF_PREC_F32 || split) ? 4 : 2;
   // split: forward image in three BF16 planes, transposed image in two
-  p->fwd_tile_bytes = split ? 3 * 512 : 256 * p->elem;
-  p->bwd_tile_bytes = split ? 2 * 512 : 256 * p->elem;
+  p->row_tile = p->elem == 2 ? 32 : 16;
+  p->fwd_tile_bytes = split ? 3 * 512 : 16 * p->row_tile * p->elem;
+  p->bwd_tile_bytes = split ? 2 * 512 : 16 * p->row_tile * p->elem;
   p->extra = p->view_dep ? (pts_dim - d->trunk_pe) + 3 * (2 * d->dirs_pe_degree + 1) : 0;
   if (p->extra > 96) return false;
   if (!p->view_dep && pts_dim != d->trunk_pe) return false;
-  const int pe_tiles = round_up(round_up(d->trunk_pe, 16) / 16, 2);
+  // 16-bit operands: always four (a trunk PE of at most 32 features is padded with zero weights), so that
+  // layers 0 and 5 have one form
+  const int pe_tiles = p->elem == 2 ? 4 : round_up(round_up(d->trunk_pe, 16) / 16, 2);
   const int ex_tiles = round_up(round_up(p->extra, 16) / 16, 2);
   for (int l = 0; l < kLayers; ++l) p->present[l] = (l <= 8) || p->view_dep;
   for (int l = 0; l < 8; ++l) {
@@ -113,21 +120,25 @@ inline bool make_plan(const srf_mlp_desc* d, Plan* p) {
   for (int l = 0; l < kLayers; ++l) {
     if (!p->present[l]) continue;
     p->out_tiles[l] = (p->out_rows[l] + 15) / 16;
-    p->bwd_tiles[l] = round_up(p->out_tiles[l], 2);
+    // reduction tiles of the transposed product: one MFMA k-step is 32 features on 16-row tiles, 16 on
+    // 32-row ones
+    p->bwd_tiles[l] = p->row_tile == 32 ? p->out_tiles[l] : round_up(p->out_tiles[l], 2);
+    p->fwd_rows_t[l] = (p->out_rows[l] + p->row_tile - 1) / p->row_tile;
+    p->bwd_rows_t[l] = 16 * p->reg_tiles[l] / p->row_tile;
     const int in_tiles = p->reg_tiles[l] + p->comp_tiles[l];
     p->fwd_off[l] = off;
-    off += (size_t)p->out_tiles[l] * in_tiles * p->fwd_tile_bytes;
+    off += (size_t)p->fwd_rows_t[l] * in_tiles * p->fwd_tile_bytes;
   }
   for (int l = 1; l < kLayers; ++l) {
     if (!p->present[l]) continue;
     p->bwd_off[l] = off;
-    off += (size_t)p->reg_tiles[l] * p->bwd_tiles[l] * p->bwd_tile_bytes;
+    off += (size_t)p->bwd_rows_t[l] * p->bwd_tiles[l] * p->bwd_tile_bytes;
   }
   for (int l = 0; l < kLayers; ++l) {
     if (!p->present[l]) continue;
     p->bias_off[l] = off;
-    off += (size_t)p->out_tiles[l] * 16 * sizeof(float);
-    p->bias_floats += p->out_tiles[l] * 16;
+    off += (size_t)p->fwd_rows_t[l] * p->row_tile * sizeof(float);
+    p->bias_floats += p->fwd_rows_t[l] * p->row_tile;
   }
   p->packed_bytes = round_up((int)off, 256);
   return true;
@@ -191,12 +202,10 @@ struct Tr;
 template <>
 struct Tr<kBF16> {
   static constexpr int CB = 4;
-  using Act = u32x2;
 };
 template <>
 struct Tr<kF16> {
   static constexpr int CB = 4;
-  using Act = u32x2;
 };
 template <>
 struct Tr<kF32> {
@@ -211,37 +220,10 @@ template <>
 struct Tr<kBFS1> : Tr<kF32> {};
 
 template <int P>
-__device__ __forceinline__ typename Tr<P>::Act to_act(const f32x4& v) {
-  if constexpr (f32_layout<P>()) {
-    return v;
-  } else {
-    u32x2 a;
-    a.x = pack2<P>(v[0], v[1]);
-    a.y = pack2<P>(v[2], v[3]);
-    return a;
-  }
-}
+__device__ __forceinline__ typename Tr<P>::Act zero_act() { return f32x4{0.f, 0.f, 0.f, 0.f}; }
 
-template <int P>
-__device__ __forceinline__ typename Tr<P>::Act zero_act() {
-  typename Tr<P>::Act a;
-  if constexpr (f32_layout<P>()) a = f32x4{0.f, 0.f, 0.f, 0.f};
-  else a = u32x2{0u, 0u};
-  return a;
-}
-
-template <int P>
-__device__ __forceinline__ uint32_t act_elem_bits(const typename Tr<P>::Act& a, int r) {
-  if constexpr (f32_layout<P>()) return __float_as_uint(a[r]);
-  else return (r < 2 ? a.x : a.y) >> (16 * (r & 1)) & 0xffffu;
-}
-
-// A wave's 16 activation tiles x CB column blocks in registers, one Act per tile (ActTiles) or,
-// for 16-bit operands, tiles 2u and 2u + 1 of a column block in one 128-bit register quad
-// (ActQuads), which is exactly the MFMA B operand of k-unit u, so that no register copies
-// assemble it.  Measured on gfx950: the quads make the training forward 8 % faster and the
-// inference forward 20 % slower (register allocation differs), so each uses its own.  Indices
-// are compile-time constants after unrolling (the arrays stay in VGPRs).
+// A wave's 16 activation tiles x CB column blocks in registers, one Act per tile.  Indices are
+// compile-time constants after unrolling (the arrays stay in VGPRs).
 template <int P>
 struct ActTiles {
   using Act = typename Tr<P>::Act;
@@ -249,30 +231,6 @@ struct ActTiles {
   __device__ SRF_AI Act get(int t, int cb) const { return q[t][cb]; }
   __device__ SRF_AI void set(int t, int cb, Act a) { q[t][cb] = a; }
 };
-template <int P>
-struct ActQuads {
-  using Act = typename Tr<P>::Act;
-  u32x4 q[8][Tr<P>::CB];
-  __device__ SRF_AI Act get(int t, int cb) const {
-    const u32x4 v = q[t >> 1][cb];
-    return (t & 1) ? u32x2{v.z, v.w} : u32x2{v.x, v.y};
-  }
-  __device__ SRF_AI void set(int t, int cb, Act a) {
-    if (t & 1) {
-      q[t >> 1][cb].z = a.x;
-      q[t >> 1][cb].w = a.y;
-    } else {
-      q[t >> 1][cb].x = a.x;
-      q[t >> 1][cb].y = a.y;
-    }
-  }
-};
-template <>
-struct ActQuads<kF32> : ActTiles<kF32> {};
-template <>
-struct ActQuads<kBFS3> : ActTiles<kBFS3> {};
-template <>
-struct ActQuads<kBFS2> : ActTiles<kBFS2> {};
 
 // sin and cos of x for |x| up to ~1e4 (positional-encoding arguments are |2^m x| < 1e3):
 // Cody-Waite reduction x = k pi/2 + r with pi/2 split into three floats applied by fma, then
@@ -309,20 +267,16 @@ struct PeRows {
   static constexpr int kParts = 64 / kNpt;     // lanes per point (FP32: two, levels split)
   static constexpr int kStride = 100;          // elements per row: up to 96 features, and
                                                // conflict-free 8 (16)-byte gathers
-  static constexpr int kBytes = kNpt * kStride * (f32_layout<P>() ? 4 : 2);
-  using E = std::conditional_t<f32_layout<P>(), float, uint16_t>;
+  static constexpr int kBytes = kNpt * kStride * 4;
+  using E = float;
 
-  __device__ static SRF_AI E cvt(float v) {
-    if constexpr (f32_layout<P>()) return v;
-    else return (uint16_t)(pack2<P>(v, 0.f) & 0xffffu);
-  }
   // Features f in [f_lo, f_hi) of PE_L(x), written at row[f - shift]; this lane computes the
   // levels m = part, part + kParts, ...
   __device__ static SRF_AI void write(E* row, const float (&x)[3], int L, int f_lo, int f_hi, int shift, int part) {
     if (part == 0)
 #pragma unroll
       for (int c = 0; c < 3; ++c)
-        if (c >= f_lo && c < f_hi) row[c - shift] = cvt(x[c]);
+        if (c >= f_lo && c < f_hi) row[c - shift] = x[c];
     for (int m = part; m < L; m += kParts) {
       if (8 + 6 * m < f_lo || 3 + 6 * m >= f_hi) continue;
 #pragma unroll
@@ -330,8 +284,8 @@ struct PeRows {
         float sn, cs;
         pe_sincos(ldexpf(x[c], m), &sn, &cs);
         const int fs = 3 + 6 * m + c, fc = 6 + 6 * m + c;
-        if (fs >= f_lo && fs < f_hi) row[fs - shift] = cvt(sn);
-        if (fc >= f_lo && fc < f_hi) row[fc - shift] = cvt(cs);
+        if (fs >= f_lo && fs < f_hi) row[fs - shift] = sn;
+        if (fc >= f_lo && fc < f_hi) row[fc - shift] = cs;
       }
     }
   }
@@ -341,17 +295,10 @@ struct PeRows {
     const int lane = threadIdx.x & 63, g = lane >> 4, j = lane & 15;
     const int c0 = 16 * t + 4 * g;
     const E* src = rows + (16 * cb + j) * kStride + c0;
-    if constexpr (f32_layout<P>()) {
-      f32x4 v = *reinterpret_cast<const f32x4*>(src);
+    f32x4 v = *reinterpret_cast<const f32x4*>(src);
 #pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = c0 + r < n_valid ? v[r] : 0.f;
-      return v;
-    } else {
-      u32x2 v = *reinterpret_cast<const u32x2*>(src);
-      v.x &= (c0 + 0 < n_valid ? 0x0000ffffu : 0u) | (c0 + 1 < n_valid ? 0xffff0000u : 0u);
-      v.y &= (c0 + 2 < n_valid ? 0x0000ffffu : 0u) | (c0 + 3 < n_valid ? 0xffff0000u : 0u);
-      return v;
-    }
+    for (int r = 0; r < 4; ++r) v[r] = c0 + r < n_valid ? v[r] : 0.f;
+    return v;
   }
 };
 
@@ -540,7 +487,8 @@ __device__ __forceinline__ void mma_tiles(f32x4 (&acc)[OUT][Tr<P>::CB], const ui
             for (int cb = 0; cb < CB; ++cb) acc[to][cb] = mfma32(a, b[cb][r], acc[to][cb]);
           }
         }
-      } else if constexpr (split_prec<P>()) {
+      } else {
+        static_assert(split_prec<P>(), "16-bit operands: mlp16.h");
         // Split BF16: the FP32 input tiles 2u, 2u + 1 of each column block become NPL BF16 B
         // operands (slot order of the 16-bit map), the weight fragments are already split into
         // NPL planes (stage layout: plane pl of (to, kc) at ((to KC + kc) NPL + pl) KB), and each
@@ -592,40 +540,6 @@ __device__ __forceinline__ void mma_tiles(f32x4 (&acc)[OUT][Tr<P>::CB], const ui
           for (int q = 0; q < kG; ++q)
 #pragma unroll
             for (int pl = 0; pl < NPL; ++pl) a_cur[q][pl] = a_nxt[q][pl];
-        });
-      } else {
-        u32x4 b[CB];
-#pragma unroll
-        for (int cb = 0; cb < CB; ++cb) {
-          const u32x2 x0 = fin(2 * u, cb), x1 = fin(2 * u + 1, cb);
-          b[cb] = u32x4{x0.x, x0.y, x1.x, x1.y};
-        }
-        // Output tiles in groups of kG: the A fragments of group g+1 are read from LDS while
-        // the MFMAs of group g run; scheduling barriers keep the compiler from hoisting every
-        // fragment read of the chunk (which would exhaust the arch VGPRs).
-        constexpr int kG = 4;
-        constexpr int NG = (OUT + kG - 1) / kG;
-        auto read_a = [&](auto GI, u32x4 (&a)[kG]) SRF_AI {
-          constexpr int gi = decltype(GI)::value;
-#pragma unroll
-          for (int q = 0; q < kG; ++q)
-            if (gi * kG + q < OUT)
-              a[q] = *reinterpret_cast<const u32x4*>(cur + ((gi * kG + q) * KC + kc) * 1024 + lane * 16);
-        };
-        u32x4 a_cur[kG], a_nxt[kG];
-        read_a(std::integral_constant<int, 0>{}, a_cur);
-        static_for<0, NG>([&](auto GI) SRF_AI {
-          constexpr int gi = decltype(GI)::value;
-          if constexpr (gi + 1 < NG) read_a(std::integral_constant<int, gi + 1>{}, a_nxt);
-#pragma unroll
-          for (int q = 0; q < kG; ++q)
-            if (gi * kG + q < OUT)
-#pragma unroll
-              for (int cb = 0; cb < CB; ++cb)
-                acc[gi * kG + q][cb] = mfma16<P>(a_cur[q], b[cb], acc[gi * kG + q][cb]);
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int q = 0; q < kG; ++q) a_cur[q] = a_nxt[q];
         });
       }
     });
@@ -738,57 +652,42 @@ __device__ __forceinline__ uint32_t tile_block(int t, int ldP, int elem, int p0)
   return (uint32_t)t * 16u * (uint32_t)ldP * (uint32_t)elem + (uint32_t)(p0 / (16 * Tr<P>::CB)) * 2048u;
 }
 
-// Writes one 16-feature tile of the wave's points in the paired tile layout read by the weight-
-// gradient GEMM: the 2 KB block at byte offset blk (tile_block) of the array described by dst.
+// Writes one 16-feature tile of the wave's points in the tile layout read by the weight-gradient
+// GEMM: the 2 KB block at byte offset blk (tile_block) of the array described by dst.
 // A tile of the whole workspace array occupies the bytes of 16 feature-major rows;
 // inside it, the wave owning points p0 .. p0 + 16 CB - 1 writes one 2 KB block of 64 lane records,
-// each two 16 B chunks.  The lanes of a pair (j = 2m, 2m + 1) first swap half of their D-tile
-// values (swap_adjacent), so that record (g, 2m + e) holds features 4 g + 2 e + c (c = 0, 1), each
-// as one 16 B chunk of that feature at the points 16 cb + 2 m and 16 cb + 2 m + 1 (cb = 0 ..
-// CB - 1), in point order.  A 16 B chunk is then exactly one lane's MFMA operand slice of one
-// feature, so the GEMM reads fragments with plain 16 B copies.  The block is chunk-major: chunk c
-// of record r sits at byte 1024 c + 16 r, so each of the two stores writes 1 KB of whole
-// contiguous lines (a record-major block would leave every line half written between them).
+// each two 16 B chunks.  The block is chunk-major: chunk c of record r sits at byte 1024 c + 16 r, so
+// each of the two stores writes 1 KB of whole contiguous lines (a record-major block would leave
+// every line half written between them).
+// The lanes of a pair (j = 2m, 2m + 1) first swap half of their D-tile values (swap_adjacent), so that
+// record (g, 2m + e) holds features 4 g + 2 e + c (c = 0, 1), each as one 16 B chunk of that feature at the
+// points 16 cb + 2 m and 16 cb + 2 m + 1 (cb = 0, 1), in point order: one lane's operand slice of one
+// feature.  (mlp16.h: store_tile16.)
 // The stores are non-temporal: a layer's tiles of all the CUs of an XCD (~4 MB) would otherwise
 // displace the streamed weights from that XCD's L2, and they are read back only by the backward.
 template <int P>
 __device__ __forceinline__ void store_tile(Rsrc dst, uint32_t blk, const typename Tr<P>::Act (&v)[Tr<P>::CB]) {
   constexpr int CB = Tr<P>::CB;
   const uint32_t rec = lane_here() * 16u;
-  if constexpr (f32_layout<P>()) {
-    // v[cb] = features 4g + 0..3 at point 16 cb + j; even lanes keep r0, r1 and take the
-    // partner's; odd lanes keep r2, r3
-    float rc[CB][2];
+  // v[cb] = features 4g + 0..3 at point 16 cb + j; even lanes keep r0, r1 and take the
+  // partner's; odd lanes keep r2, r3
+  float rc[CB][2];
 #pragma unroll
-    for (int cb = 0; cb < CB; ++cb) {
-      rc[cb][0] = swap_adjacent(sel_odd(v[cb][0], v[cb][2]));
-      rc[cb][1] = swap_adjacent(sel_odd(v[cb][1], v[cb][3]));
-    }
-    f32x4 c0, c1;
-#pragma unroll
-    for (int cb = 0; cb < CB; ++cb) {
-      const float own0 = sel_odd(v[cb][2], v[cb][0]), own1 = sel_odd(v[cb][3], v[cb][1]);
-      c0[2 * cb + 0] = sel_odd(rc[cb][0], own0);
-      c0[2 * cb + 1] = sel_odd(own0, rc[cb][0]);
-      c1[2 * cb + 0] = sel_odd(rc[cb][1], own1);
-      c1[2 * cb + 1] = sel_odd(own1, rc[cb][1]);
-    }
-    store_nt16(dst, rec, blk, __builtin_bit_cast(u32x4, c0));
-    store_nt16(dst, rec, blk + 1024, __builtin_bit_cast(u32x4, c1));
-  } else {
-    // v[cb] = {bf16 (r0, r1), bf16 (r2, r3)} at point 16 cb + j
-    u32x4 c0, c1;
-#pragma unroll
-    for (int cb = 0; cb < CB; ++cb) {
-      const uint32_t recv = swap_adjacent(sel_odd(v[cb][0], v[cb][1]));
-      const uint32_t own = sel_odd(v[cb][1], v[cb][0]);
-      const uint32_t first = sel_odd(recv, own), second = sel_odd(own, recv);  // points 2m, 2m + 1
-      c0[cb] = (first & 0xffffu) | (second << 16);
-      c1[cb] = (first >> 16) | (second & 0xffff0000u);
-    }
-    store_nt16(dst, rec, blk, c0);
-    store_nt16(dst, rec, blk + 1024, c1);
+  for (int cb = 0; cb < CB; ++cb) {
+    rc[cb][0] = swap_adjacent(sel_odd(v[cb][0], v[cb][2]));
+    rc[cb][1] = swap_adjacent(sel_odd(v[cb][1], v[cb][3]));
   }
+  f32x4 c0, c1;
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb) {
+    const float own0 = sel_odd(v[cb][2], v[cb][0]), own1 = sel_odd(v[cb][3], v[cb][1]);
+    c0[2 * cb + 0] = sel_odd(rc[cb][0], own0);
+    c0[2 * cb + 1] = sel_odd(own0, rc[cb][0]);
+    c1[2 * cb + 0] = sel_odd(rc[cb][1], own1);
+    c1[2 * cb + 1] = sel_odd(own1, rc[cb][1]);
+  }
+  store_nt16(dst, rec, blk, __builtin_bit_cast(u32x4, c0));
+  store_nt16(dst, rec, blk + 1024, __builtin_bit_cast(u32x4, c1));
 }
 
 // Inverse of store_tile for FP32 tiles (CB = 2): the lane's D-tile values (v[cb][r] = feature 4 g + r
@@ -835,7 +734,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 
   auto valid = [&](int cb) SRF_AI { return p0 + 16 * cb + j < a.n; };
 
-  std::conditional_t<TRAIN, ActQuads<P>, ActTiles<P>> h;
+  ActTiles<P> h;
   uint32_t mbits[CB][2];  // ReLU mask bits 4T+r of tiles 0-7 (word 0) and 8-15 (word 1)
 
   // trunk PE tiles -> pe_lds (training stores them for the weight gradients during layer 0)
@@ -917,7 +816,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
         v[r] = pos ? v[r] : 0.f;
         mbits[cb][T >> 3] |= pos ? (1u << (4 * (T & 7) + r)) : 0u;
       }
-      h.set(T, cb, to_act<P>(v));
+      h.set(T, cb, v);
     }
   };
   // Deferred training stores (mma_tiles' side items) of the tiles the layer being computed
@@ -1011,7 +910,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     }, stage, bias_of(8), side_of(I16{}, a.w.h[7], I0{}, 0, 7));
     run_layer<P, 16, 16, 0>(a.packed + pl.fwd_off[8], fin_h, [&](int T, f32x4(&acc)[CB]) SRF_AI {
 #pragma unroll
-      for (int cb = 0; cb < CB; ++cb) h.set(T, cb, to_act<P>(acc[cb]));
+      for (int cb = 0; cb < CB; ++cb) h.set(T, cb, acc[cb]);
     }, stage, bias_of(8));
     // view layer input extras: [PE_xyz[trunk_pe:], PE_dir], one row per point (the feature
     // layer's product ended with a block barrier, so the stage is free)
@@ -1145,7 +1044,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
       f32x4 v = acc[cb];
 #pragma unroll
       for (int r = 0; r < 4; ++r) v[r] = (mb[cb][T >> 3] & (1u << (4 * (T & 7) + r))) ? v[r] : 0.f;
-      z[T][cb] = to_act<P>(v);
+      z[T][cb] = v;
     }
   };
   auto fin_z = [&](int t, int cb) SRF_AI { return z[t][cb]; };
@@ -1157,7 +1056,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
       for (int cb = 0; cb < CB; ++cb) {
         f32x4 v = {0.f, 0.f, 0.f, 0.f};
         if (g == 0) v = f32x4{drr[cb][0], drr[cb][1], drr[cb][2], 0.f};
-        z[0][cb] = to_act<P>(v);
+        z[0][cb] = v;
         z[1][cb] = zero_act<P>();
       }
     }
@@ -1166,14 +1065,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     // dF = W9^T dZ9 (feature part, identity activation) -> dZ8 rows 0..255 (z[0..15]); stores dZ9
     run_layer<P, 8, 16, 0, 8>(a.packed + pl.bwd_off[9], fin_z, [&](int T, f32x4(&acc)[CB]) SRF_AI {
 #pragma unroll
-      for (int cb = 0; cb < CB; ++cb) z[T][cb] = to_act<P>(acc[cb]);
+      for (int cb = 0; cb < CB; ++cb) z[T][cb] = acc[cb];
     }, stage, nullptr, dz_side(9, I0{}));
     {
 #pragma unroll
       for (int cb = 0; cb < CB; ++cb) {
         f32x4 v = {0.f, 0.f, 0.f, 0.f};
         if (g == 0) v[0] = dsr[cb];
-        z[16][cb] = to_act<P>(v);
+        z[16][cb] = v;
         z[17][cb] = zero_act<P>();
       }
     }
@@ -1188,7 +1087,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
       for (int cb = 0; cb < CB; ++cb) {
         f32x4 v = {0.f, 0.f, 0.f, 0.f};
         if (g == 0) v = f32x4{dsr[cb], drr[cb][0], drr[cb][1], drr[cb][2]};
-        z[0][cb] = to_act<P>(v);
+        z[0][cb] = v;
         z[1][cb] = zero_act<P>();
       }
     }
@@ -1363,16 +1262,22 @@ __global__ __launch_bounds__(64 * kDwWaves) void mlp_dw_kernel(DwArgs a) {
       if (a.paired) {
         // lane (g, j) takes feature j's chunk of the record pair m = 4 u + g of the 2 KB block of
         // the points' wave (see store_tile): record (j >> 2, 2 m + ((j >> 1) & 1)), chunk j & 1
+        // 16-bit values (store_tile16): LDS position l of the fragment takes chunk (l >> 1) & 1 of record
+        // (h = l & 1, c = 16 u + 4 ((l >> 2) & 3) + (l >> 4)), so that operand lane (g', j') finds
+        // feature j' at the points c, 32 + c of c = 16 u + 4 g' + i as dword i (frag16: 4 B at 4 lane +
+        // 256 i, contiguous over the wave).
         constexpr int PPW = F32L ? 32 : 64;  // points per stored wave block
         const int wb = p / PPW, u = (p % PPW) / KPTS;
-        const int rec = 16 * (j >> 2) + 2 * (4 * u + g) + ((j >> 1) & 1);
+        const int rec = F32L ? 16 * (j >> 2) + 2 * (4 * u + g) + ((j >> 1) & 1)
+                             : 32 * (lane & 1) + 16 * u + 4 * ((lane >> 2) & 3) + (lane >> 4);
+        const int piece = F32L ? j & 1 : (lane >> 1) & 1;
         // the wide tilings read tile-major blocks (tile t's blocks span 16 rows of ldP points, the MLP
         // workspace); the narrow one point-block-major blocks (the array's tiles of one wave block
         // adjacent, 2 KB each: the colour network's workspace)
         size_t blk;
         if constexpr (kRowWaves) blk = ((size_t)wb * ((is_a ? jb.dz_rows : jb.x_rows) / 16) + row0 / 16) * 2048;
         else blk = (size_t)row0 * ldP * ELEM + (size_t)wb * 2048;
-        src = base + blk + (j & 1) * 1024 + rec * 16;
+        src = base + blk + piece * 1024 + rec * 16;
       } else {
         const int pg = F32L ? 4 * g : 8 * g;
         src = base + (((size_t)(row0 + j)) * ldP + p + pg) * ELEM;
@@ -1380,6 +1285,11 @@ __global__ __launch_bounds__(64 * kDwWaves) void mlp_dw_kernel(DwArgs a) {
       __builtin_amdgcn_global_load_lds((const void*)src,
                                        (__attribute__((address_space(3))) void*)(buf + f * 1024), 16, 0, 0);
     }
+  };
+  // one operand fragment of 16-bit values (see dma_unit)
+  auto frag16 = [&](const uint8_t* f) SRF_AI {
+    const uint32_t* v = reinterpret_cast<const uint32_t*>(f) + lane;
+    return u32x4{v[0], v[64], v[128], v[192]};
   };
   f32x4 acc[RM][NC];
   float rs[RM];
@@ -1456,9 +1366,9 @@ __global__ __launch_bounds__(64 * kDwWaves) void mlp_dw_kernel(DwArgs a) {
       } else {
         u32x4 av[RM], bv[NC];
 #pragma unroll
-        for (int i = 0; i < RM; ++i) av[i] = *reinterpret_cast<const u32x4*>(fr + (qm + i) * 1024 + lane * 16);
+        for (int i = 0; i < RM; ++i) av[i] = frag16(fr + (qm + i) * 1024);
 #pragma unroll
-        for (int k = 0; k < NC; ++k) bv[k] = *reinterpret_cast<const u32x4*>(fr + (16 + qn + k) * 1024 + lane * 16);
+        for (int k = 0; k < NC; ++k) bv[k] = frag16(fr + (16 + qn + k) * 1024);
         // every tile's product, valid or not (the epilogue stores the valid ones; the slot holds a
         // whole k-unit either way): no branch between the MFMAs
 #pragma unroll
