@@ -86,14 +86,15 @@ __device__ __forceinline__ float relu1(float v) {
 typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
 typedef int16_t i16x2_t __attribute__((ext_vector_type(2)));
 
-// Shifts two pairs of flags into m: m = m << 1 | (a != 0), then the same for b, in each 16-bit half
-// (a, b: packed pairs of non-negative 16-bit floats).  Written out, since the compiler turns the
-// minimum with 1 into a comparison and a select for each half.
-__device__ __forceinline__ void push_nonzero(uint32_t& m, uint32_t a, uint32_t b) {
-  uint32_t t;
+// Shifts the flags of two packed pairs of non-negative 16-bit floats into m: m = m << 1 | (a != 0) in each
+// 16-bit half, then the same for b.  Written out, since the compiler turns the minimum with 1 into a
+// comparison and a select for each half.  Both registers written here are read-write operands (t: any
+// value, kept by the caller), so neither can be one that an MFMA still in flight is about to write, which
+// the compiler does not check for written-out instructions.
+__device__ __forceinline__ void push_nonzero(uint32_t& m, uint32_t& t, uint32_t a, uint32_t b) {
   asm("v_pk_min_u16 %1, %2, %4\n\tv_lshl_or_b32 %0, %0, 1, %1\n\t"
       "v_pk_min_u16 %1, %3, %4\n\tv_lshl_or_b32 %0, %0, 1, %1"
-      : "+v"(m), "=&v"(t)
+      : "+v"(m), "+&v"(t)
       : "v"(a), "v"(b), "s"(0x00010001u));
 }
 
@@ -155,6 +156,20 @@ __device__ __forceinline__ void lds_dma_1k(const uint8_t* src, uint8_t* lds_base
   const int lane = threadIdx.x & 63;
   __builtin_amdgcn_global_load_lds((const void*)(src + 16 * lane),
                                    (__attribute__((address_space(3))) void*)lds_base, 16, 0, 0);
+}
+
+// The same copy (src and lds_offset wave-uniform, lane16 = 16 lane) without the compiler's knowledge: it makes every LDS read that follows the builtin wait for all vector-memory operations
+// (it cannot tell the buffers of a ring apart), which undoes a copy ahead of its use.  The caller waits
+// for the copy (s_waitcnt vmcnt) and synchronises before it is read.
+__device__ __forceinline__ void lds_dma_1k_ahead(const uint8_t* src, uint32_t lds_offset, uint32_t lane16) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :
+               : "s"(lds_offset), "v"(lane16), "s"(src)
+               : "memory", "m0");
+}
+// Offset of an LDS object, as lds_dma_1k_ahead takes it.
+__device__ __forceinline__ uint32_t lds_offset(const void* p) {
+  return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)p);
 }
 
 // Wait for every outstanding vector-memory operation of this wave (LDS DMA included).

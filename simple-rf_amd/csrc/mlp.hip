@@ -69,16 +69,14 @@ __device__ inline int slot_k(int s, int g, int i) {
 
 // Slots 8 idx .. 8 idx + 7 of the forward (bwd = 0) or transposed (1) image of layer l for 32x32x16
 // MFMAs (mlp16.h): 1 KB fragments of 32 rows x 16 features, lane 32 h + c of k-step 2 T + m holding row c
-// at features 32 T + 16 (i / 4) + 8 m + 4 h + i % 4.  The fragments lie k-step by k-step, the row tiles of one k-step together;
-// row tiles past the eighth (the sigma row) follow in the same order.
+// at features 32 T + 16 (i / 4) + 8 m + 4 h + i % 4; the fragments of one row tile together, padded with
+// zeros to whole units of four.
 __device__ void pack_fragment16(const PackArgs& a, int l, int bwd, int rows_t, int steps, unsigned idx) {
   const Plan& p = a.p;
   if (idx >= (unsigned)(rows_t * steps) * 64u) return;
   const unsigned lane = idx & 63u, f = idx >> 6;
-  const unsigned mt = rows_t < 8 ? rows_t : 8, f1 = mt * steps;
-  const unsigned n = f < f1 ? mt : rows_t - mt, fl = f < f1 ? f : f - f1;
-  const unsigned s = fl / n;
-  const int T = (int)(fl - s * n) + (f < f1 ? 0 : 8);
+  const int T = (int)(f / (unsigned)steps);
+  const unsigned s = f - (unsigned)T * (unsigned)steps;
   const int row = 32 * T + (int)(lane & 31u), k0 = 32 * (int)(s >> 1) + 8 * (int)(s & 1u) + 4 * (int)(lane >> 5);
   const int row_col = bwd ? ref_col(p, l, row) : 0;
   uint32_t d[8];
@@ -101,7 +99,7 @@ __device__ void pack_element(const PackArgs& a, int l, int bwd, long idx) {
   const int rows_t = bwd ? p.bwd_rows_t[l] : p.fwd_rows_t[l];
   const int k_tiles = bwd ? p.bwd_tiles[l] : p.reg_tiles[l] + p.comp_tiles[l];
   if (p.row_tile == 32) {
-    pack_fragment16(a, l, bwd, rows_t, k_tiles, (unsigned)idx);
+    pack_fragment16(a, l, bwd, rows_t, bwd ? p.bwd_steps[l] : p.fwd_steps[l], (unsigned)idx);
     return;
   }
   const int ks = f32 ? 4 * k_tiles : k_tiles / 2;
@@ -250,7 +248,7 @@ extern "C" int srf_mlp_pack(const srf_mlp_desc* desc, const float* const* weight
       const int rows_t = bwd ? p.bwd_rows_t[l] : p.fwd_rows_t[l];
       const int k_tiles = bwd ? p.bwd_tiles[l] : p.reg_tiles[l] + p.comp_tiles[l];
       const int ks = p.prec == SRF_PREC_F32 ? 4 * k_tiles : k_tiles / 2;
-      add(l, bwd, p.row_tile == 32 ? (long)rows_t * k_tiles * 64 : (long)rows_t * ks * 64 * kpl);
+      add(l, bwd, p.row_tile == 32 ? (long)rows_t * (bwd ? p.bwd_steps[l] : p.fwd_steps[l]) * 64 : (long)rows_t * ks * 64 * kpl);
     }
     add(l, 2, (long)p.row_tile * p.fwd_rows_t[l]);
   }

@@ -5,9 +5,10 @@
 // independent 16x16x32 MFMAs on random operands reaches 1.40-1.50 PFLOP/s on this chip, the same
 // products as 32x32x16 MFMAs 1.79 PFLOP/s (1.58 and 2.49 on zeros: the larger shape also draws less
 // power per product).  4,096 rays x 192 samples, main model: training forward 1,705 us on 16x16x32 tiles,
-// 1,214 us here; backward chain 1,339 -> 1,078 us; inference of 16,384 x 192 points 3,981 -> 3,444 us.
-// Part of it is the epilogue: ReLU by v_med3, masks from packed pairs, tile records without a lane exchange
-// (2,700 -> 1,100 vector operations a layer).
+// 1,034 us here; backward chain 1,339 -> 898 us; inference of 16,384 x 192 points 3,985 -> 3,107 us.
+// The kernels are bound by the MFMAs (a 256 x 256 layer of 256 points: 3.5 us at the full clock, 4.8 us at
+// the clock that random operands leave), their operand reads from LDS (half of its rate) and, in training,
+// the stores (5.5 and 5.2 KB a point: 630 us at a fill's rate for 786,432 points).
 //
 // Lane layout (lane = 32 h + c, h = 0, 1):
 //   A operand (32 x 16): row c, eight reduction slots i = 0 .. 7
@@ -38,124 +39,129 @@ __device__ __forceinline__ f32x16 mfma32x32(const u32x4& a, const u32x4& b, cons
                                                   0, 0);
 }
 
-// Weight stage: two buffers of one chunk each.  The packed image of a product lists its 1 KB
-// fragments k-step by k-step (all OUT row tiles of k-step 0, then of k-step 1, ...), so a chunk of
-// kChunk / OUT k-steps is one linear copy and the wave reads its fragments in the order they lie.
-constexpr int kChunk = 32;  // fragments of a chunk (32 KB)
-struct Stage16 {
-  uint8_t* base;
-  uint32_t off;  // byte offset of the buffer that holds the next product's first chunk (0 or 32 KB)
-};
+// Weight stream.  The packed images of a kernel's products lie in the order of their use, each row tile's
+// fragments (1 KB, one per k-step, padded to whole units) together: a product runs row tile by row tile,
+// all its k-steps, so that only two tiles' accumulators are live, a tile's epilogue runs between the
+// MFMAs of the next one, and the layer's outputs fit the AGPRs beside its inputs.  (The earlier form held
+// all eight tiles' accumulators and ran its epilogues, 1,100 vector operations a layer, after them.)
+// The stream goes through a ring of units of four fragments, copied global -> LDS by the block's four
+// waves (one fragment each) and read by all of them one unit ahead of its use.  Every unit used copies the
+// one kAhead units further on, so the copies need no schedule; the last ones of a kernel run past its
+// images (into what follows them, or the buffer's pad) and are waited for at its end.
+// A group is at most six units between two synchronisations.  At its start (sync) all its units and the
+// next one have landed, and the waves have read all earlier units, so that at most kAhead + 6 units of
+// the ring are in use.
+constexpr int kUnit = 4096;
+constexpr int kRingUnits = 24;   // 96 KB
+constexpr int kAhead = 16;
+static_assert((kAhead + 1) * kUnit <= kPackPad, "the copies past the last image stay in the buffer");
+struct Stream16 {
+  const uint8_t* src;   // this wave's fragment of the next unit to copy
+  const uint8_t* ring;
+  uint32_t lds;         // LDS offset of this wave's fragment of the ring's first unit
+  uint32_t wr, rd;      // byte offsets of the unit to copy / in a
+  u32x4 a[4];           // the fragments of the current unit
 
-// The first chunk of the product that follows: n fragments (0: none) at src.
-struct NextChunk {
-  const uint8_t* src;
-  int n;
-};
-
-// Copies n fragments (n <= kChunk, uniform) at src into the buffer at dst, by the block's waves together.
-__device__ __forceinline__ void dma_frags(const uint8_t* __restrict__ src, int n, uint8_t* dst) {
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  __device__ SRF_AI Stream16(const uint8_t* image, const uint8_t* ring_) {
+    const uint32_t frag = 1024u * (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    src = image + frag;
+    ring = ring_;
+    lds = lds_offset(ring_) + frag;
+    wr = rd = 0;
 #pragma unroll
-  for (int i = 0; i < kChunk / kWaves; ++i) {
-    const int f = w + kWaves * i;
-    if (f < n) lds_dma_1k(src + (size_t)f * 1024, dst + f * 1024);
+    for (int i = 0; i < kAhead; ++i) copy();
   }
-}
-
-__device__ __forceinline__ void block_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
-// acc[T][cb] (+)= rows 32 T .. of the image at img times the NK k-steps that fin(s, cb) returns; the
-// sum starts from the bias of those rows (kBias), from zero (kZero) or from acc (kAdd).
-// On entry the first chunk lies in the stage (st.off); every wave of the block must come here.  While
-// a chunk is multiplied the next one is copied, and while the last one is, the first chunk of the
-// product that follows (next): its latency hides behind this product's epilogue.
-// Deferred stores: side(i), i in [0, NSIDE), issues at least two vector-memory operations each (the
-// training copies of the tiles that this product reads).  They are spread over the groups of MFMAs, and
-// a chunk waits with vmcnt(operations issued after its copy), since these complete in issue order.
-enum { kZero, kBias, kAdd };
-template <int P, int NB, int NK, int OUT, int INIT, int NSIDE = 0, typename FIn, typename Side = NoSide>
-__device__ __forceinline__ void product(f32x16 (&acc)[OUT][NB], const uint8_t* __restrict__ img, const float* bias,
-                                        FIn&& fin, Stage16& st, NextChunk next, Side&& side = Side{}) {
-  constexpr int KC = kChunk / OUT < NK ? kChunk / OUT : NK;  // k-steps per chunk
-  constexpr int NCH = (NK + KC - 1) / KC;
-  constexpr int kPer = (NSIDE + NCH - 1) / NCH;               // side items per chunk
-  constexpr int kG = 4;                                       // fragments per group
-  const int lane = threadIdx.x & 63;
-  const float* bias_h = bias + 4 * (lane >> 5);
-  static_for<0, NCH>([&](auto CI) SRF_AI {
-    constexpr int c = decltype(CI)::value;
-    constexpr int kn = NK - c * KC < KC ? NK - c * KC : KC;
-    constexpr int NF = kn * OUT, NG = (NF + kG - 1) / kG;
-    const uint8_t* cur = st.base + st.off;
-    st.off ^= kChunk * 1024;
-    if constexpr (c + 1 < NCH) {
-      constexpr int kn1 = NK - (c + 1) * KC < KC ? NK - (c + 1) * KC : KC;
-      dma_frags(img + (size_t)(c + 1) * KC * OUT * 1024, kn1 * OUT, st.base + st.off);
-    } else if (next.n) {
-      dma_frags(next.src, next.n, st.base + st.off);
-    }
+  __device__ SRF_AI static uint32_t next(uint32_t o) { return o + kUnit == kRingUnits * kUnit ? 0u : o + kUnit; }
+  __device__ SRF_AI void copy() {
+    lds_dma_1k_ahead(src, lds + wr, (threadIdx.x & 63) * 16);
+    src += kUnit;
+    wr = next(wr);
+  }
+  __device__ SRF_AI u32x4 read(uint32_t off, int i) const {
+    return *reinterpret_cast<const u32x4*>(ring + off + i * 1024 + (threadIdx.x & 63) * 16);
+  }
+  // The first unit, once the prologue has waited for the copies.
+  __device__ SRF_AI void begin() {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a[i] = read(0, i);
+  }
+  // Start of a group.  This wave's copies of the group's units and the next one were issued at least nine
+  // copies and kStores stores ago, and vector-memory operations complete in issue order.
+  template <int kStores>
+  __device__ SRF_AI void sync() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(vmcnt_only(kAhead - 7 + kStores));
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
-    constexpr int i0 = c * kPer < NSIDE ? c * kPer : NSIDE;
-    constexpr int i1 = (c + 1) * kPer < NSIDE ? (c + 1) * kPer : NSIDE;
-    constexpr int per_group = (i1 - i0 + NG - 1) / NG;
-    auto read_a = [&](auto GI, u32x4 (&a)[kG]) SRF_AI {
-      constexpr int g = decltype(GI)::value;
-#pragma unroll
-      for (int q = 0; q < kG; ++q)
-        if (g * kG + q < NF) a[q] = *reinterpret_cast<const u32x4*>(cur + (g * kG + q) * 1024 + lane * 16);
-    };
-    // the fragments of group g + 1 are read from LDS while the MFMAs of group g run; the scheduling
-    // barriers keep the compiler from hoisting every read of the chunk
-    u32x4 a_cur[kG], a_nxt[kG];
-    read_a(std::integral_constant<int, 0>{}, a_cur);
-    static_for<0, NG>([&](auto GI) SRF_AI {
-      constexpr int g = decltype(GI)::value;
-      if constexpr (g + 1 < NG) read_a(std::integral_constant<int, g + 1>{}, a_nxt);
-      static_for<0, kG>([&](auto QI) SRF_AI {
-        constexpr int f = g * kG + decltype(QI)::value;
-        if constexpr (f < NF) {
-          constexpr int s = c * KC + f / OUT, T = f % OUT;
-          f32x16 init;
-          if constexpr (s == 0 && INIT == kBias) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const f32x4 b = *reinterpret_cast<const f32x4*>(bias_h + 32 * T + 8 * q);
-#pragma unroll
-              for (int r = 0; r < 4; ++r) init[4 * q + r] = b[r];
-            }
-          } else if constexpr (s == 0 && INIT == kZero) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) init[r] = 0.f;
-          }
-#pragma unroll
-          for (int cb = 0; cb < NB; ++cb) {
-            if constexpr (s == 0 && INIT != kAdd) acc[T][cb] = mfma32x32<P>(a_cur[decltype(QI)::value], fin(s, cb), init);
-            else acc[T][cb] = mfma32x32<P>(a_cur[decltype(QI)::value], fin(s, cb), acc[T][cb]);
-          }
-        }
-      });
-      static_for<0, per_group>([&](auto KI) SRF_AI {
-        constexpr int i = i0 + g * per_group + decltype(KI)::value;
-        if constexpr (i < i1) side(std::integral_constant<int, i>{});
-      });
+  }
+  // One unit: f(i, fragment) for its four fragments, reading the next unit's meanwhile.
+  template <typename F>
+  __device__ SRF_AI void unit(F&& f) {
+    rd = next(rd);
+    static_for<0, 4>([&](auto II) SRF_AI {
+      constexpr int i = decltype(II)::value;
+      f(II, a[i]);
+      a[i] = read(rd, i);
+      if constexpr (i == 1) copy();
       __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int q = 0; q < kG; ++q) a_cur[q] = a_nxt[q];
     });
-    // the copy has landed once at most the 2 (i1 - i0) operations issued after it are outstanding; the
-    // barrier also frees the buffer that this chunk read (its reads were consumed by the MFMAs above)
-    if (c + 1 < NCH || next.n) {
-      constexpr int after = 2 * (i1 - i0);
-      __builtin_amdgcn_s_waitcnt(vmcnt_only(after < 63 ? after : 63));
+  }
+};
+
+// A value in an accumulation register (the MFMAs read their operands from there; vector operations
+// cannot).  No MFMA of these kernels writes accumulation registers.
+__device__ __forceinline__ uint32_t to_agpr(uint32_t x) {
+  uint32_t r;
+  asm("v_accvgpr_write_b32 %0, %1" : "=a"(r) : "v"(x));
+  return r;
+}
+
+// Epilogue of one 32-row tile in 16 pieces (q, i): pair p = i % 2 of registers 4 q .. 4 q + 3 of column
+// block i / 2, packed into dword 2 (q / 2) + p of quad q % 2 of the tile.  pack(q, i, v0, v1)
+// returns the packed pair (after the ReLU or the mask); done(q, e) gets the four dwords e[cb][p] of q.
+struct NoPiece {
+  template <typename Q, typename I>
+  __device__ SRF_AI void operator()(Q, I) const {}
+};
+template <int NB, typename Pack, typename Done>
+struct TileEpi {
+  f32x16 (&v)[NB];
+  u32x4 (&lo)[NB];   // quad 2 T
+  u32x4 (&hi)[NB];   // quad 2 T + 1
+  Pack pack;
+  Done done;
+  uint32_t (&e)[2][2][2];  // [q % 2]: two pieces may be under way
+  template <typename Q, typename I>
+  __device__ SRF_AI void operator()(Q QI, I) const {
+    constexpr int q = Q::value, cb = I::value >> 1, p = I::value & 1;
+    if constexpr (cb < NB) {
+      const uint32_t d = pack(QI, I{}, v[cb][4 * q + 2 * p], v[cb][4 * q + 2 * p + 1]);
+      e[q & 1][cb][p] = d;
+      (q & 1 ? hi : lo)[cb][2 * (q >> 1) + p] = to_agpr(d);
     }
-    block_barrier();
-  });
+    if constexpr (I::value == 3) done(QI, e[q & 1]);
+  }
+};
+
+// The pieces that go with k-step i of unit u: kPieces = 1: piece (u, i) in units 0 .. 3; 2: pieces (2 u, i)
+// and (2 u + 1, i) in units 0 and 1; 4: pieces (i, 0 .. 3) in unit 0.
+template <int kPieces, int u, int i, typename Epi>
+__device__ __forceinline__ void pieces(const Epi& epi) {
+  using std::integral_constant;
+  if constexpr (kPieces == 1 && u < 4) {
+    epi(integral_constant<int, u>{}, integral_constant<int, i>{});
+  } else if constexpr (kPieces == 2 && u < 2) {
+    epi(integral_constant<int, 2 * u>{}, integral_constant<int, i>{});
+    epi(integral_constant<int, 2 * u + 1>{}, integral_constant<int, i>{});
+  } else if constexpr (kPieces == 4 && u == 0) {
+    static_for<0, 4>([&](auto J) SRF_AI { epi(integral_constant<int, i>{}, J); });
+  }
+}
+template <typename Epi>
+__device__ __forceinline__ void all_pieces(const Epi& epi) {
+  static_for<0, 4>([&](auto Q) SRF_AI { static_for<0, 4>([&](auto I) SRF_AI { epi(Q, I); }); });
 }
 
 // Stores 16-feature tile t of the wave's 64 points as the 2 KB block that the weight-gradient GEMM
@@ -163,38 +169,35 @@ __device__ __forceinline__ void product(f32x16 (&acc)[OUT][NB], const uint8_t* _
 // r (r = 0 .. 3, one dword each) at the lane's own points c and 32 + c.  Chunk k comes from quad k of the
 // tile's pair (its k-steps 2 (t / 2) + k) in both column blocks.  One byte permutation a dword, no lane
 // exchange, and each of the two stores writes 1 KB of whole lines.  Non-temporal, as store_tile's.
-template <int T>
-__device__ __forceinline__ u32x4 tile_chunk(const u32x4& a, const u32x4& b) {
+__device__ __forceinline__ u32x4 tile_chunk(uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1) {
   constexpr uint32_t kLo = 0x05040100, kHi = 0x07060302;  // the low / high halves of two dwords
-  constexpr int d = 2 * (T & 1);
-  const uint32_t a0 = a[d], a1 = a[d + 1], b0 = b[d], b1 = b[d + 1];
   return u32x4{__builtin_amdgcn_perm(b0, a0, kLo), __builtin_amdgcn_perm(b0, a0, kHi),
                __builtin_amdgcn_perm(b1, a1, kLo), __builtin_amdgcn_perm(b1, a1, kHi)};
 }
+// Chunk k of tile t from its quads 2 (t / 2) + k.
 template <int T>
 __device__ __forceinline__ void store_tile16(Rsrc dst, uint32_t blk, const u32x4 (&q0)[2], const u32x4 (&q1)[2]) {
-  const uint32_t rec = lane_here() * 16u;
-  store_nt16(dst, rec, blk, tile_chunk<T>(q0[0], q0[1]));
-  store_nt16(dst, rec, blk + 1024, tile_chunk<T>(q1[0], q1[1]));
+  const uint32_t rec = (threadIdx.x & 63) * 16u;
+  constexpr int d = 2 * (T & 1);
+  store_nt16(dst, rec, blk, tile_chunk(q0[0][d], q0[0][d + 1], q0[1][d], q0[1][d + 1]));
+  store_nt16(dst, rec, blk + 1024, tile_chunk(q1[0][d], q1[0][d + 1], q1[1][d], q1[1][d + 1]));
 }
-
-// The two quads of 32 rows (one D tile) from their eight packed pairs d[2 q + p].
-__device__ __forceinline__ u32x4 quad_of(const uint32_t (&d)[8], int m) { return u32x4{d[2 * m], d[2 * m + 1], d[4 + 2 * m], d[5 + 2 * m]}; }
 
 // Positional encoding straight into B-operand quads (lane = point of the wave).
 template <int P, int NB>
 struct PeQuads {
-  // features [f_lo, f_hi) of PE_L(x) at columns f - shift of the wave's quads
   __device__ static SRF_AI void put(uint8_t* quads, int col, float v) {
     const int pt = (threadIdx.x & 63) % (32 * NB);
-    const int step = 2 * (col >> 5) + ((col >> 3) & 1);
-    const int at = (step * NB + (pt >> 5)) * 1024 + (((col >> 2) & 1) * 32 + (pt & 31)) * 16 +
-                   (((col >> 4) & 1) * 4 + (col & 3)) * 2;
-    *reinterpret_cast<uint16_t*>(quads + at) = (uint16_t)(pack2<P>(v, 0.f) & 0xffffu);
+    // the point's part of the address, and the column's
+    const int at_pt = (pt >> 5) * 1024 + (pt & 31) * 16;
+    const int at_col = (2 * (col >> 5) + ((col >> 3) & 1)) * NB * 1024 + ((col >> 2) & 1) * 512 +
+                       (((col >> 4) & 1) * 4 + (col & 3)) * 2;
+    *reinterpret_cast<uint16_t*>(quads + at_pt + at_col) = (uint16_t)(pack2<P>(v, 0.f) & 0xffffu);
   }
+  // features [f_lo, f_hi) of PE_L(x) at columns f - shift of the wave's quads
   __device__ static SRF_AI void write(uint8_t* quads, const float (&x)[3], int L, int f_lo, int f_hi, int shift) {
-    // NB = 1: two lanes per point share its levels
-    const int part = (threadIdx.x & 63) / (32 * NB), parts = 2 / NB;
+    // NB = 1: two lanes per point share its levels (NB = 2: m, and so the columns, are uniform)
+    const int part = NB == 2 ? 0 : (threadIdx.x & 63) / 32, parts = 2 / NB;
     if (part == 0)
 #pragma unroll
       for (int c = 0; c < 3; ++c)
@@ -222,9 +225,9 @@ struct PeQuads {
 template <int P, bool VD, bool TRAIN, int NB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void mlp16_fwd_kernel(FwdArgs a) {
   static_assert(!TRAIN || NB == 2, "the training layout is that of 64-point waves");
-  __shared__ __attribute__((aligned(16))) uint8_t stage[2 * kChunk * 1024];
-  // computed input features of each wave's points (trunk PE for layers 0 and 5, then the view layer's
-  // [PE_xyz[trunk_pe:], PE_dir]) as B-operand quads, written and read by the wave alone
+  __shared__ __attribute__((aligned(16))) uint8_t ring[kRingUnits * kUnit];
+  // computed input features of each wave's points (the trunk PE, then the view layer's [PE_xyz[trunk_pe:],
+  // PE_dir]) as B-operand quads, written and read by the wave alone
   __shared__ __attribute__((aligned(16))) u32x4 pe_lds[kWaves][6][NB][64];
   __shared__ __attribute__((aligned(16))) float bias_lds[kMaxBiasFloats];
   const int lane = threadIdx.x & 63, h = lane >> 5, cl = lane & 31;
@@ -233,17 +236,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   const int p0 = wave * 32 * NB;
   const Plan& pl = a.p;
   const int ldP = a.w.ldP;
-  Stage16 st{stage, 0};
   uint8_t* quads = reinterpret_cast<uint8_t*>(&pe_lds[wv][0][0][0]);
   using PE = PeQuads<P, NB>;
-  auto image = [&](int l, int kstep_frags = 0) SRF_AI { return a.packed + pl.fwd_off[l] + (size_t)kstep_frags * 1024; };
 
-  dma_frags(image(0), kChunk, stage);  // layer 0's only chunk
-  {
-    const float* src = reinterpret_cast<const float*>(a.packed + pl.bias_off[0]);
-    for (int i = threadIdx.x; i < pl.bias_floats; i += 64 * kWaves) bias_lds[i] = src[i];
-  }
-  auto bias_of = [&](int l) SRF_AI { return bias_lds + (pl.bias_off[l] - pl.bias_off[0]) / 4; };
+  Stream16 st(a.packed + pl.fwd_off[0], ring);
+  static_assert(kMaxBiasFloats % 256 == 0, "copied as whole fragments");
+#pragma unroll
+  for (int i = 0; i < (kMaxBiasFloats / 256 + kWaves - 1) / kWaves; ++i)
+    if (i * kWaves + wv < kMaxBiasFloats / 256)
+      lds_dma_1k_ahead(a.packed + pl.bias_off[0] + (i * kWaves + wv) * 1024,
+                       lds_offset(bias_lds) + (i * kWaves + wv) * 1024, lane * 16);
 
   // the lane's point (PE): stored, or rays_o[..., None, :] + rays_d[..., None, :] * z[..., :, None] of
   // its ray (src/models/SimpleNeRF17.py:213-215, :266-268; two rounded FP32 operations)
@@ -265,201 +267,253 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 #pragma unroll
     for (int c = 0; c < 3; ++c) v[c] = pe_in ? a.dirs[3 * r + c] : 0.f;
   };
-  {
-    float x[3];
-    load_xyz(x);
-    PE::write(quads, x, pl.pts_deg, 0, pl.trunk_pe, 0);
-    PE::pad(quads, pl.trunk_pe, 4);
-  }
-
-  u32x4 q[16][NB];       // the layer input: quad s, column block cb
-  uint32_t mbits[NB][4];  // ReLU mask: word T / 2, see relu_epi
-  auto fin_q = [&](int s, int cb) SRF_AI { return q[s][cb]; };
-  auto fin_pe = [&](int s, int cb) SRF_AI { return pe_lds[wv][s][cb][lane]; };
-  // ReLU, packing and (training) the mask from the packed pairs: both bits of pair 8 (T % 2) + 2 qq + p
-  // of word T / 2 lie at 15 minus that in the word's halves (push_nonzero)
-  auto relu_epi = [&](auto TI, f32x16(&v)[NB]) SRF_AI {
-    constexpr int T = decltype(TI)::value;
-#pragma unroll
-    for (int cb = 0; cb < NB; ++cb) {
-      uint32_t d[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) d[i] = pack2<P>(relu1(v[cb][2 * i]), relu1(v[cb][2 * i + 1]));
-      q[2 * T][cb] = quad_of(d, 0);
-      q[2 * T + 1][cb] = quad_of(d, 1);
-      if constexpr (TRAIN) {
-        if ((T & 1) == 0) mbits[cb][T >> 1] = 0;
-#pragma unroll
-        for (int i = 0; i < 8; i += 2) push_nonzero(mbits[cb][T >> 1], d[i], d[i + 1]);
-      }
-    }
-  };
-  // Deferred stores of the tiles that a product reads: NQ quads of q at ws offset q_off, then NPE PE
-  // quads at pe_off, then (slot >= 0) the ReLU mask of the layer that produced q.
-  constexpr int kT = TRAIN ? 1 : 0;
-  auto side_of = [&](auto NQI, size_t q_off, auto NPEI, size_t pe_off, int slot) SRF_AI {
-    constexpr int nq = decltype(NQI)::value, npe = decltype(NPEI)::value;
-    const Rsrc rq = uniform_rsrc(a.ws + q_off), rpe = uniform_rsrc(a.ws + pe_off);
-    const Rsrc rm = uniform_rsrc(a.ws + a.w.mask + (size_t)(slot < 0 ? 0 : slot) * ldP * 32);
-    return [&, rq, rpe, rm](auto II) SRF_AI {
-      constexpr int i = decltype(II)::value;
-      if constexpr (NB == 2) {
-        if constexpr (i < nq) {
-          store_tile16<i>(rq, tile_block<P>(i, ldP, pl.elem, p0), q[i & ~1], q[i | 1]);
-        } else if constexpr (i < nq + npe) {
-          constexpr int t = i - nq;
-          u32x4 e[2][2];
-#pragma unroll
-          for (int k = 0; k < 2; ++k)
-#pragma unroll
-            for (int cb = 0; cb < 2; ++cb) e[k][cb] = pe_lds[wv][(t & ~1) + k][cb][lane];
-          store_tile16<t>(rpe, tile_block<P>(t, ldP, pl.elem, p0), e[0], e[1]);
-        } else {
-#pragma unroll
-          for (int cb = 0; cb < 2; ++cb)
-            store_nt16(rm, lane_here() * 16u, (uint32_t)wave * 2048u + cb * 1024u,
-                       u32x4{mbits[cb][0], mbits[cb][1], mbits[cb][2], mbits[cb][3]});
-        }
-      }
-    };
-  };
-  using I0 = std::integral_constant<int, 0>;
-  using I16 = std::integral_constant<int, 16>;
-
+  float x[3], vdir[3] = {0.f, 0.f, 0.f};
+  load_xyz(x);
+  if constexpr (VD) load_dir(vdir);
+  PE::write(quads, x, pl.pts_deg, 0, pl.trunk_pe, 0);
+  PE::pad(quads, pl.trunk_pe, 4);
   wait_vmem();
-  __syncthreads();  // layer 0's weights, the biases and the PE quads
+  __syncthreads();  // the first units, the biases and the PE quads
 
-  // ---- layer 0: PE(trunk) -> 256 (stores the PE tiles)
-  {
-    f32x16 acc[8][NB];
-    product<P, NB, 4, 8, kBias, 4 * kT>(acc, image(0), bias_of(0), fin_pe, st, NextChunk{image(1), kChunk},
-                                        side_of(I0{}, 0, std::integral_constant<int, 4>{}, a.w.x0, -1));
-    static_for<0, 8>([&](auto TI) SRF_AI { relu_epi(TI, acc[decltype(TI)::value]); });
-  }
-  // ---- layers 1..7 in place in q; layer 5 adds the trunk PE (storing layer l - 1's output and mask)
-  // (three copies of the layer body: with layer 5's extra product behind a branch in one loop, the
-  // accumulators meet at its join and the compiler spills and copies them)
-  auto trunk_layer = [&](int l, auto SKIP) SRF_AI {
-    constexpr bool skip = decltype(SKIP)::value;
-    f32x16 acc[8][NB];
-    // what comes after layer 7: the sigma tile (stored behind the feature tiles) or the 4-channel head
-    const NextChunk nx = skip ? NextChunk{image(5, 16 * 8), kChunk}
-                         : l < 7 ? NextChunk{image(l + 1), kChunk}
-                                 : NextChunk{image(8, VD ? 16 * 8 : 0), 16};
-    product<P, NB, 16, 8, kBias, 17 * kT>(acc, image(l), bias_of(l), fin_q, st, nx,
-                                          side_of(I16{}, a.w.h[l - 1], I0{}, 0, l - 1));
-    if constexpr (skip) {
-      product<P, NB, 4, 8, kAdd>(acc, image(5, 16 * 8), nullptr, fin_pe, st, NextChunk{image(6), kChunk});
+  u32x4 qa[16][NB], qb[16][NB];  // a layer's input and output quads (AGPRs), in turns
+  u32x4 pe[4][NB];               // the trunk PE's
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+#pragma unroll
+    for (int cb = 0; cb < NB; ++cb) pe[s][cb] = pe_lds[wv][s][cb][lane];
+  f32x16 acc[2][NB];      // accumulators of tile T in acc[T % 2], the other one's epilogue running
+  uint32_t mbits[NB][4];  // ReLU mask: word T / 2
+  uint32_t flag = 0;      // push_nonzero's
+  uint32_t e[2][2][2];    // the epilogue pieces' dwords
+
+  // biases of the tiles in the order of the products, one tile ahead
+  const float* bp = bias_lds + 4 * h;
+  f32x16 bias;
+  auto next_bias = [&]() SRF_AI {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const f32x4 b = *reinterpret_cast<const f32x4*>(bp + 8 * q);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) bias[4 * q + r] = b[r];
     }
-    static_for<0, 8>([&](auto TI) SRF_AI { relu_epi(TI, acc[decltype(TI)::value]); });
+    bp += 32;
+  };
+  next_bias();
+  st.begin();
+
+  constexpr int kSt = TRAIN ? 8 : 0;  // stores of two tiles
+  using IC0 = std::integral_constant<int, 0>;
+  const Rsrc rmask = uniform_rsrc(a.ws + a.w.mask);
+  // The epilogue of tile T: ReLU (or not), packing, the mask from the packed pairs (both bits of pair
+  // 8 (T % 2) + 2 q + p of word T / 2 at 15 minus that in the word's halves), and the tile's record.
+  auto epi = [&](auto TI, auto RELU, u32x4 (&dst)[16][NB], Rsrc out) SRF_AI {
+    constexpr int T = decltype(TI)::value;
+    constexpr bool relu = decltype(RELU)::value;
+    auto pack = [&](auto QI, auto II, float v0, float v1) SRF_AI {
+      constexpr int cb = decltype(II)::value >> 1, p = decltype(II)::value & 1;
+      const uint32_t d = relu ? pack2<P>(relu1(v0), relu1(v1)) : pack2<P>(v0, v1);
+      if constexpr (TRAIN && relu && p == 1) {
+        if constexpr (decltype(QI)::value == 0 && (T & 1) == 0) mbits[cb][T >> 1] = 0;
+        push_nonzero(mbits[cb][T >> 1], flag, e[decltype(QI)::value & 1][cb][0], d);
+      }
+      return d;
+    };
+    auto done = [&, out](auto QI, const uint32_t (&d)[2][2]) SRF_AI {
+      constexpr int q = decltype(QI)::value;
+      if constexpr (TRAIN)
+        store_nt16(out, lane * 16u, tile_block<P>(2 * T + (q >> 1), ldP, pl.elem, p0) + 1024u * (q & 1),
+                   tile_chunk(d[0][0], d[0][1], d[1][0], d[1][1]));
+    };
+    return TileEpi<NB, decltype(pack), decltype(done)>{acc[T & 1], dst[2 * T], dst[2 * T + 1], pack, done, e};
+  };
+  auto out_of = [&](size_t off) SRF_AI { return uniform_rsrc(a.ws + off); };
+  auto store_mask = [&](int slot) SRF_AI {
+    if constexpr (TRAIN)
+#pragma unroll
+      for (int cb = 0; cb < NB; ++cb)
+        store_nt16(rmask, lane * 16u, (uint32_t)slot * (uint32_t)ldP * 32u + (uint32_t)wave * 2048u + cb * 1024u,
+                   u32x4{mbits[cb][0], mbits[cb][1], mbits[cb][2], mbits[cb][3]});
+  };
+  // One unit of tile accumulators ac: k-steps s0 .. s0 + n - 1 with operand quads src, pieces of the
+  // previous tile's epilogue in between.
+  auto unit = [&](auto UI, auto NI, auto PIECES, f32x16(&ac)[NB], auto&& src, const auto& prev) SRF_AI {
+    constexpr int u = decltype(UI)::value, n = decltype(NI)::value;
+    st.unit([&](auto II, const u32x4& w) SRF_AI {
+      constexpr int i = decltype(II)::value;
+      if constexpr (i < n) {
+#pragma unroll
+        for (int cb = 0; cb < NB; ++cb) ac[cb] = mfma32x32<P>(w, src(4 * u + i, cb), u == 0 && i == 0 ? bias : ac[cb]);
+        if constexpr (u == 0 && i == 0) next_bias();
+      }
+      pieces<decltype(PIECES)::value, u, i>(prev);
+    });
+  };
+  using I1 = std::integral_constant<int, 1>;
+  using I2 = std::integral_constant<int, 2>;
+  using I4 = std::integral_constant<int, 4>;
+  using Yes = std::true_type;
+  using No = std::false_type;
+  // the four units of a 256-input tile
+  auto tile = [&](auto PIECES, f32x16(&ac)[NB], const u32x4 (&src)[16][NB], const auto& prev) SRF_AI {
+    static_for<0, 4>([&](auto UI) SRF_AI {
+      unit(UI, I4{}, PIECES, ac, [&](int s, int cb) SRF_AI { return src[s][cb]; }, prev);
+    });
+  };
+
+  // ---- layer 0: PE(trunk) -> qa
+  if constexpr (TRAIN) {
+    const Rsrc rx = out_of(a.w.x0);
+    static_for<0, 4>([&](auto TI) SRF_AI {
+      constexpr int t = decltype(TI)::value;
+      store_tile16<t>(rx, tile_block<P>(t, ldP, pl.elem, p0), pe[t & ~1], pe[t | 1]);
+    });
+  }
+  {
+    const Rsrc out = out_of(a.w.h[0]);
+    static_for<0, 8>([&](auto TI) SRF_AI {
+      constexpr int T = decltype(TI)::value;
+      if constexpr (T == 4) st.template sync<0>();
+      auto src = [&](int s, int cb) SRF_AI { return pe[s][cb]; };
+      if constexpr (T == 0) unit(IC0{}, I4{}, I4{}, acc[0], src, NoPiece{});
+      else unit(IC0{}, I4{}, I4{}, acc[T & 1], src, epi(std::integral_constant<int, T - 1>{}, Yes{}, qa, out));
+    });
+  }
+  // ---- layers 1-7: src -> dst.  The first tile finishes the previous layer's last one (whose quads its
+  // last two k-steps read), which leaves out of layer l - 1 stored.
+  auto layer = [&](int l, u32x4 (&src)[16][NB], u32x4 (&dst)[16][NB], auto FIVE) SRF_AI {
+    const Rsrc prev = out_of(a.w.h[l - 1]), out = out_of(a.w.h[l]);
+    static_for<0, 8>([&](auto TI) SRF_AI {
+      constexpr int T = decltype(TI)::value;
+      st.template sync<kSt>();
+      if constexpr (T == 0) {
+        tile(I2{}, acc[0], src, epi(std::integral_constant<int, 7>{}, Yes{}, src, prev));
+        store_mask(l - 1);
+      } else {
+        tile(I1{}, acc[T & 1], src, epi(std::integral_constant<int, T - 1>{}, Yes{}, dst, out));
+      }
+      if constexpr (decltype(FIVE)::value)
+        if (l == 5)
+          unit(I4{}, I4{}, I4{}, acc[T & 1], [&](int s, int cb) SRF_AI { return pe[s & 3][cb]; }, NoPiece{});
+    });
   };
 #pragma unroll 1
-  for (int l = 1; l < 5; ++l) trunk_layer(l, std::false_type{});
-  trunk_layer(5, std::true_type{});
-#pragma unroll 1
-  for (int l = 6; l < 8; ++l) trunk_layer(l, std::false_type{});
+  for (int l = 1;; l += 2) {
+    layer(l, qa, qb, Yes{});
+    if (l == 7) break;
+    layer(l + 1, qb, qa, No{});
+  }
 
   // ---- heads (their rows lie in the lanes h = 0)
   auto head_sigma = [&](int p, float raw) SRF_AI {
     if (a.noise) raw = raw + a.noise[p];
     a.sigma[p] = pl.softplus ? softplusf_(raw) : (raw > 0.f ? raw : 0.f);
   };
-  f32x16 hd[1][NB];
+  const Rsrc out7 = out_of(a.w.h[7]);
+  const auto last7 = epi(std::integral_constant<int, 7>{}, Yes{}, qb, out7);
   if constexpr (!VD) {
-    // 4-channel output: sigma, rgb (src/models/SimpleNeRF17.py:735-750); stores layer 7
-    product<P, NB, 16, 1, kBias, 17 * kT>(hd, image(8), bias_of(8), fin_q, st, NextChunk{nullptr, 0},
-                                          side_of(I16{}, a.w.h[7], I0{}, 0, 7));
+    // 4-channel output: sigma, rgb (src/models/SimpleNeRF17.py:735-750)
+    st.template sync<kSt>();
+    tile(I2{}, acc[0], qb, last7);
+    store_mask(7);
 #pragma unroll
     for (int cb = 0; cb < NB; ++cb) {
       const int p = p0 + 32 * cb + cl;
       if (h == 0 && p < a.n) {
-        head_sigma(p, hd[0][cb][0]);
+        head_sigma(p, acc[0][cb][0]);
 #pragma unroll
-        for (int c = 0; c < 3; ++c) a.rgb[3 * p + c] = sigmoidf_(hd[0][cb][1 + c]);
+        for (int c = 0; c < 3; ++c) a.rgb[3 * p + c] = sigmoidf_(acc[0][cb][1 + c]);
       }
     }
   } else {
-    product<P, NB, 16, 1, kBias>(hd, image(8, 16 * 8), bias_of(8) + 256, fin_q, st, NextChunk{image(8), kChunk});
+    // feature rows 0..255 (no activation) -> qa, then the sigma row
+    const Rsrc out = out_of(a.w.f);
+    static_for<0, 9>([&](auto TI) SRF_AI {
+      constexpr int T = decltype(TI)::value;
+      st.template sync<kSt>();
+      if constexpr (T == 0) {
+        tile(I2{}, acc[0], qb, last7);
+        store_mask(7);
+      } else {
+        tile(I1{}, acc[T & 1], qb, epi(std::integral_constant<int, T - 1>{}, No{}, qa, out));
+      }
+    });
 #pragma unroll
     for (int cb = 0; cb < NB; ++cb) {
       const int p = p0 + 32 * cb + cl;
-      if (h == 0 && p < a.n) head_sigma(p, hd[0][cb][0]);
-    }
-    {
-      // feature rows 0..255 (no activation) in place in q; stores layer 7
-      f32x16 acc[8][NB];
-      product<P, NB, 16, 8, kBias, 17 * kT>(acc, image(8), bias_of(8), fin_q, st, NextChunk{image(9), kChunk},
-                                            side_of(I16{}, a.w.h[7], I0{}, 0, 7));
-      static_for<0, 8>([&](auto TI) SRF_AI {
-        constexpr int T = decltype(TI)::value;
-#pragma unroll
-        for (int cb = 0; cb < NB; ++cb) {
-          uint32_t d[8];
-#pragma unroll
-          for (int i = 0; i < 8; ++i) d[i] = pack2<P>(acc[T][cb][2 * i], acc[T][cb][2 * i + 1]);
-          q[2 * T][cb] = quad_of(d, 0);
-          q[2 * T + 1][cb] = quad_of(d, 1);
-        }
-      });
+      if (h == 0 && p < a.n) head_sigma(p, acc[0][cb][0]);
     }
     // the view layer's computed inputs [PE_xyz[trunk_pe:], PE_dir]
+    const int ct = pl.comp_tiles[9];  // 2, 4 or 6
     {
       const int pts_dim = 3 * (2 * pl.pts_deg + 1), n_hi = pts_dim - pl.trunk_pe;
-      float x[3], d[3];
-      load_xyz(x);
-      load_dir(d);
       if (n_hi > 0) PE::write(quads, x, pl.pts_deg, pl.trunk_pe, pts_dim, pl.trunk_pe);
-      PE::write(quads, d, pl.dir_deg, 0, pl.extra - n_hi, -n_hi);
-      PE::pad(quads, pl.extra, pl.comp_tiles[9]);
+      PE::write(quads, vdir, pl.dir_deg, 0, pl.extra - n_hi, -n_hi);
+      PE::pad(quads, pl.extra, ct);
       wave_lds_sync();
     }
-    // view layer [feature, extras] -> 128, in place into q[0..7]; stores the feature tiles and the extras
-    auto fin_qe = [&](int s, int cb) SRF_AI { return s < 16 ? q[s < 16 ? s : 0][cb] : pe_lds[wv][s < 16 ? 0 : s - 16][cb][lane]; };
-    {
-      f32x16 acc[4][NB];
-      const NextChunk nx{image(10), 8};
-      if (pl.comp_tiles[9] == 2)
-        product<P, NB, 18, 4, kBias, 18 * kT>(acc, image(9), bias_of(9), fin_qe, st, nx,
-                                              side_of(I16{}, a.w.f, std::integral_constant<int, 2>{}, a.w.ex, -1));
-      else if (pl.comp_tiles[9] == 4)
-        product<P, NB, 20, 4, kBias, 20 * kT>(acc, image(9), bias_of(9), fin_qe, st, nx,
-                                              side_of(I16{}, a.w.f, std::integral_constant<int, 4>{}, a.w.ex, -1));
-      else
-        product<P, NB, 22, 4, kBias, 22 * kT>(acc, image(9), bias_of(9), fin_qe, st, nx,
-                                              side_of(I16{}, a.w.f, std::integral_constant<int, 6>{}, a.w.ex, -1));
-      static_for<0, 4>([&](auto TI) SRF_AI { relu_epi(TI, acc[decltype(TI)::value]); });
-      if constexpr (TRAIN)
+    u32x4 ex[6][NB];
+    static_for<0, 6>([&](auto SI) SRF_AI {
+      constexpr int s = decltype(SI)::value;
 #pragma unroll
-        for (int cb = 0; cb < NB; ++cb) mbits[cb][2] = mbits[cb][3] = 0;
+      for (int cb = 0; cb < NB; ++cb) ex[s][cb] = s < ct ? pe_lds[wv][s][cb][lane] : u32x4{0u, 0u, 0u, 0u};
+    });
+    if constexpr (TRAIN) {
+      const Rsrc rx = out_of(a.w.ex);
+      static_for<0, 6>([&](auto TI) SRF_AI {
+        constexpr int t = decltype(TI)::value;
+        if (t < ct) store_tile16<t>(rx, tile_block<P>(t, ldP, pl.elem, p0), ex[t & ~1], ex[t | 1]);
+      });
     }
-    // rgb head 128 -> 3, sigmoid (stores the view layer's output and mask)
-    product<P, NB, 8, 1, kBias, 9 * kT>(hd, image(10), bias_of(10), fin_q, st, NextChunk{nullptr, 0},
-                                        side_of(std::integral_constant<int, 8>{}, a.w.v, I0{}, 0, 8));
+    // view layer [feature, extras] -> 128 in qb[0..7].  The fragments that pad a tile to whole units are
+    // zero, and so are the extra quads they meet.
+    const Rsrc outv = out_of(a.w.v);
+    static_for<0, 4>([&](auto TI) SRF_AI {
+      constexpr int T = decltype(TI)::value;
+      st.template sync<0>();
+      auto src = [&](int s, int cb) SRF_AI { return s < 16 ? qa[s & 15][cb] : ex[s < 16 ? 0 : s - 16][cb]; };
+      auto run = [&](const auto& prev) SRF_AI {
+        static_for<0, 4>([&](auto UI) SRF_AI { unit(UI, I4{}, I1{}, acc[T & 1], src, prev); });
+      };
+      if constexpr (T == 0) run(NoPiece{});
+      else run(epi(std::integral_constant<int, T - 1>{}, Yes{}, qb, outv));
+      unit(I4{}, I4{}, I1{}, acc[T & 1], src, NoPiece{});
+      if (ct > 4) unit(std::integral_constant<int, 5>{}, I2{}, I1{}, acc[T & 1], src, NoPiece{});
+    });
+    all_pieces(epi(std::integral_constant<int, 3>{}, Yes{}, qb, outv));
+    if constexpr (TRAIN) {
+#pragma unroll
+      for (int cb = 0; cb < NB; ++cb) mbits[cb][2] = mbits[cb][3] = 0;
+      store_mask(8);
+    }
+    // rgb head 128 -> 3, sigmoid
+    st.template sync<0>();
+    static_for<0, 2>([&](auto UI) SRF_AI {
+      unit(UI, I4{}, I1{}, acc[0], [&](int s, int cb) SRF_AI { return qb[s][cb]; }, NoPiece{});
+    });
 #pragma unroll
     for (int cb = 0; cb < NB; ++cb) {
       const int p = p0 + 32 * cb + cl;
       if (h == 0 && p < a.n)
 #pragma unroll
-        for (int c = 0; c < 3; ++c) a.rgb[3 * p + c] = sigmoidf_(hd[0][cb][c]);
+        for (int c = 0; c < 3; ++c) a.rgb[3 * p + c] = sigmoidf_(acc[0][cb][c]);
     }
   }
+  wait_vmem();  // the copies past the last unit
 }
 
 // ------------------------------------------------------------------- backward chain
 template <int P, bool VD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void mlp16_bwd_kernel(BwdArgs a) {
   constexpr int NB = 2;
-  __shared__ __attribute__((aligned(16))) uint8_t stage[2 * kChunk * 1024];
+  __shared__ __attribute__((aligned(16))) uint8_t ring[kRingUnits * kUnit];
   const int lane = threadIdx.x & 63, h = lane >> 5, cl = lane & 31;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wave = blockIdx.x * kWaves + wv;
   const int p0 = wave * 32 * NB;
   const Plan& pl = a.p;
   const int ldP = a.w.ldP;
-  Stage16 st{stage, 0};
-  auto image = [&](int l) SRF_AI { return a.packed + pl.bwd_off[l]; };
-  dma_frags(image(VD ? 10 : 8), VD ? 4 : 8, stage);  // the first product's only chunk
 
+  Stream16 st(a.packed + pl.bwd_off[VD ? 10 : 8], ring);
   float dsr[NB], drr[NB][3];  // head pre-activation gradients
 #pragma unroll
   for (int cb = 0; cb < NB; ++cb) {
@@ -473,107 +527,152 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
       drr[cb][c] = dr * (1.0f - y) * y;
     }
   }
+  wait_vmem();
+  __syncthreads();
+  st.begin();
 
-  // z holds the current layer's pre-activation gradients as B-operand quads; every product writes in
-  // place, and the next one stores what it reads for the weight gradients (deferred stores).
-  u32x4 z[18][NB];  // (z[17]: zero padding)
-  uint32_t mb[NB][4];
-  auto fin_z = [&](int s, int cb) SRF_AI { return z[s][cb]; };
-  // item 0 (slot >= 0): the ReLU masks of that slot, for the epilogue of the product they are loaded in;
-  // then the quads of z as tiles of dZ_l
-  auto side_of = [&](auto MI, int slot, int l) SRF_AI {
-    constexpr int nm = decltype(MI)::value;
-    const Rsrc rz = uniform_rsrc(a.ws + a.w.dz[l]);
-    const Rsrc rm = uniform_rsrc(a.ws + a.w.mask + (size_t)(slot < 0 ? 0 : slot) * ldP * 32);
-    return [&, rz, rm](auto II) SRF_AI {
-      constexpr int i = decltype(II)::value;
-      if constexpr (i < nm) {
+  u32x4 za[16][NB], zb[16][NB];  // pre-activation gradients as B-operand quads (AGPRs), in turns
+  f32x16 acc[2][NB];
+  uint32_t e[2][2][2];
+  uint32_t mb[NB][4];  // ReLU masks of the layer whose gradient is being computed
+  uint32_t mlast[NB];  // the last word of the previous one's, for its last tile
+  const Rsrc rmask = uniform_rsrc(a.ws + a.w.mask);
+  auto load_masks = [&](int slot) SRF_AI {
 #pragma unroll
-        for (int cb = 0; cb < NB; ++cb) {
-          const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rm, lane * 16u, (uint32_t)wave * 2048u + cb * 1024u, 0);
+    for (int cb = 0; cb < NB; ++cb) {
+      const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(
+          rmask, lane * 16u, (uint32_t)slot * (uint32_t)ldP * 32u + (uint32_t)wave * 2048u + cb * 1024u, 0);
 #pragma unroll
-          for (int k = 0; k < 4; ++k) mb[cb][k] = v[k];
-        }
-      } else {
-        constexpr int t = i - nm;
-        store_tile16<t>(rz, tile_block<P>(t, ldP, pl.elem, p0), z[t & ~1], z[t | 1]);
-      }
+      for (int k = 0; k < 4; ++k) mb[cb][k] = v[k];
+    }
+  };
+  auto out_of = [&](int l) SRF_AI { return uniform_rsrc(a.ws + a.w.dz[l]); };
+  // Epilogue of tile T: packed, masked (kMask 1: by mb, 2: by mlast, 0: not), stored as dZ tiles.
+  auto epi = [&](auto TI, auto MASK, u32x4 (&dst)[16][NB], Rsrc out) SRF_AI {
+    constexpr int T = decltype(TI)::value, mask = decltype(MASK)::value;
+    auto pack = [&](auto QI, auto II, float v0, float v1) SRF_AI {
+      constexpr int cb = decltype(II)::value >> 1, k = 8 * (T & 1) + 2 * decltype(QI)::value + (decltype(II)::value & 1);
+      const uint32_t d = pack2<P>(v0, v1);
+      if constexpr (mask == 1) return d & half_mask<k>(mb[cb][T >> 1]);
+      else if constexpr (mask == 2) return d & half_mask<k>(mlast[cb]);
+      else return d;
     };
+    auto done = [&, out](auto QI, const uint32_t (&d)[2][2]) SRF_AI {
+      constexpr int q = decltype(QI)::value;
+      store_nt16(out, lane * 16u, tile_block<P>(2 * T + (q >> 1), ldP, pl.elem, p0) + 1024u * (q & 1),
+                 tile_chunk(d[0][0], d[0][1], d[1][0], d[1][1]));
+    };
+    return TileEpi<NB, decltype(pack), decltype(done)>{acc[T & 1], dst[2 * T], dst[2 * T + 1], pack, done, e};
   };
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
-  // ReLU-masked gradient into z (the forward's bit order, mlp16_fwd_kernel's relu_epi)
-  auto masked_epi = [&](auto TI, f32x16(&v)[NB]) SRF_AI {
-    constexpr int T = decltype(TI)::value;
+  using I2 = std::integral_constant<int, 2>;
+  using I4 = std::integral_constant<int, 4>;
+  using I7 = std::integral_constant<int, 7>;
+  using I8 = std::integral_constant<int, 8>;
+  auto unit = [&](auto UI, auto NI, auto PIECES, f32x16(&ac)[NB], auto&& src, const auto& prev) SRF_AI {
+    constexpr int u = decltype(UI)::value, n = decltype(NI)::value;
+    st.unit([&](auto II, const u32x4& w) SRF_AI {
+      constexpr int i = decltype(II)::value;
+      if constexpr (i < n) {
+        f32x16 zero;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) zero[r] = 0.f;
+#pragma unroll
+        for (int cb = 0; cb < NB; ++cb) ac[cb] = mfma32x32<P>(w, src(4 * u + i, cb), u == 0 && i == 0 ? zero : ac[cb]);
+      }
+      pieces<decltype(PIECES)::value, u, i>(prev);
+    });
+  };
+  auto tile = [&](auto PIECES, f32x16(&ac)[NB], const u32x4 (&src)[16][NB], const auto& prev) SRF_AI {
+    static_for<0, 4>([&](auto UI) SRF_AI {
+      unit(UI, I4{}, PIECES, ac, [&](int s, int cb) SRF_AI { return src[s][cb]; }, prev);
+    });
+  };
+  // A head's gradient rows 0..3 as the one quad that holds them, and their 16-row tile t of dZ_l
+  // (rows 4.. of it are zero).
+  u32x4 head[NB];
+  auto set_head = [&](auto rows, Rsrc out, int t) SRF_AI {
 #pragma unroll
     for (int cb = 0; cb < NB; ++cb) {
-      uint32_t d[8];
-      static_for<0, 8>([&](auto KI) SRF_AI {
-        constexpr int i = decltype(KI)::value;
-        d[i] = pack2<P>(v[cb][2 * i], v[cb][2 * i + 1]) & half_mask<8 * (T & 1) + i>(mb[cb][T >> 1]);
-      });
-      z[2 * T][cb] = quad_of(d, 0);
-      z[2 * T + 1][cb] = quad_of(d, 1);
+      const f32x4 v = rows(cb);
+      head[cb] = h == 0 ? u32x4{pack2<P>(v[0], v[1]), pack2<P>(v[2], v[3]), 0u, 0u} : u32x4{0u, 0u, 0u, 0u};
     }
+    const u32x4 none[2] = {u32x4{0u, 0u, 0u, 0u}, u32x4{0u, 0u, 0u, 0u}};
+    store_tile16<0>(out, tile_block<P>(t, ldP, pl.elem, p0), head, none);
   };
-  // a head's gradient rows 0..3 as quads s, s + 1
-  auto head_quad = [&](int s, int cb, float r0, float r1, float r2, float r3) SRF_AI {
-    z[s][cb] = h == 0 ? u32x4{pack2<P>(r0, r1), pack2<P>(r2, r3), 0u, 0u} : u32x4{0u, 0u, 0u, 0u};
-    z[s + 1][cb] = u32x4{0u, 0u, 0u, 0u};
+  // A product over one k-step (a head's quad): tile T from fragment T, the epilogue of tile T - 1 behind it.
+  auto from_head = [&](auto TILES, u32x4 (&dst)[16][NB], Rsrc out) SRF_AI {
+    constexpr int tiles = decltype(TILES)::value;
+    static_for<0, tiles / 4>([&](auto UI) SRF_AI {
+      st.unit([&](auto II, const u32x4& w) SRF_AI {
+        constexpr int T = 4 * decltype(UI)::value + decltype(II)::value;
+        f32x16 zero;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) zero[r] = 0.f;
+#pragma unroll
+        for (int cb = 0; cb < NB; ++cb) acc[T & 1][cb] = mfma32x32<P>(w, head[cb], zero);
+        if constexpr (T > 0) all_pieces(epi(std::integral_constant<int, T - 1>{}, I1{}, dst, out));
+      });
+    });
   };
-  wait_vmem();
-  __syncthreads();
+  constexpr int kSt = 8;  // stores of two tiles
 
   if constexpr (VD) {
-#pragma unroll
-    for (int cb = 0; cb < NB; ++cb) head_quad(0, cb, drr[cb][0], drr[cb][1], drr[cb][2], 0.f);
-    {
-      // dV = W10^T dZ10, masked by the view-layer ReLU -> dZ9 (z[0..7]); stores dZ10
-      f32x16 acc[4][NB];
-      product<P, NB, 1, 4, kZero, 2>(acc, image(10), nullptr, fin_z, st, NextChunk{image(9), kChunk}, side_of(I1{}, 8, 10));
-      static_for<0, 4>([&](auto TI) SRF_AI { masked_epi(TI, acc[decltype(TI)::value]); });
-    }
-    {
-      // dF = W9^T dZ9 (feature part, no activation) -> dZ8 rows 0..255 (z[0..15]); stores dZ9
-      f32x16 acc[8][NB];
-      product<P, NB, 8, 8, kZero, 8>(acc, image(9), nullptr, fin_z, st, NextChunk{image(8), kChunk}, side_of(I0{}, -1, 9));
-      static_for<0, 8>([&](auto TI) SRF_AI {
-        constexpr int T = decltype(TI)::value;
-#pragma unroll
-        for (int cb = 0; cb < NB; ++cb) {
-          uint32_t d[8];
-#pragma unroll
-          for (int i = 0; i < 8; ++i) d[i] = pack2<P>(acc[T][cb][2 * i], acc[T][cb][2 * i + 1]);
-          z[2 * T][cb] = quad_of(d, 0);
-          z[2 * T + 1][cb] = quad_of(d, 1);
-        }
+    // dV = W10^T dZ10, masked by the view layer's ReLU -> dZ9 (zb[0..7])
+    load_masks(8);
+    set_head([&](int cb) SRF_AI { return f32x4{drr[cb][0], drr[cb][1], drr[cb][2], 0.f}; }, out_of(10), 0);
+    const Rsrc out9 = out_of(9), out8 = out_of(8);
+    from_head(I4{}, zb, out9);
+    all_pieces(epi(std::integral_constant<int, 3>{}, I1{}, zb, out9));
+    // dF = W9^T dZ9 (feature part, no activation) -> dZ8 rows 0..255 (za)
+    load_masks(7);
+    static_for<0, 8>([&](auto TI) SRF_AI {
+      constexpr int T = decltype(TI)::value;
+      if constexpr ((T & 1) == 0) st.template sync<0>();
+      static_for<0, 2>([&](auto UI) SRF_AI {
+        auto src = [&](int s, int cb) SRF_AI { return zb[s][cb]; };
+        if constexpr (T == 0) unit(UI, I4{}, I2{}, acc[0], src, NoPiece{});
+        else unit(UI, I4{}, I2{}, acc[T & 1], src, epi(std::integral_constant<int, T - 1>{}, I0{}, za, out8));
       });
-    }
-#pragma unroll
-    for (int cb = 0; cb < NB; ++cb) head_quad(16, cb, dsr[cb], 0.f, 0.f, 0.f);
-    f32x16 acc[8][NB];
-    product<P, NB, 17, 8, kZero, 18>(acc, image(8), nullptr, fin_z, st, NextChunk{image(7), kChunk}, side_of(I1{}, 7, 8));
-    static_for<0, 8>([&](auto TI) SRF_AI { masked_epi(TI, acc[decltype(TI)::value]); });
+    });
+    // dH7 = W8^T dZ8 (feature rows and the sigma row), masked -> dZ7 (zb)
+    set_head([&](int cb) SRF_AI { return f32x4{dsr[cb], 0.f, 0.f, 0.f}; }, out8, 16);
+    const Rsrc out7 = out_of(7);
+    static_for<0, 8>([&](auto TI) SRF_AI {
+      constexpr int T = decltype(TI)::value;
+      st.template sync<0>();
+      if constexpr (T == 0) tile(I2{}, acc[0], za, epi(I7{}, I0{}, za, out8));
+      else tile(I1{}, acc[T & 1], za, epi(std::integral_constant<int, T - 1>{}, I1{}, zb, out7));
+      unit(I4{}, I1{}, I4{}, acc[T & 1], [&](int, int cb) SRF_AI { return head[cb]; }, NoPiece{});
+    });
   } else {
+    // dH7 = W8^T dZ8 (four channels), masked -> dZ7 (zb)
+    load_masks(7);
+    set_head([&](int cb) SRF_AI { return f32x4{dsr[cb], drr[cb][0], drr[cb][1], drr[cb][2]}; }, out_of(8), 0);
+    from_head(I8{}, zb, out_of(7));
+  }
+  // trunk: dH_{l-1} = W_l^T dZ_l, masked -> dZ_{l-1}
+  auto layer = [&](int l, u32x4 (&src)[16][NB], u32x4 (&dst)[16][NB]) SRF_AI {
+    const Rsrc prev = out_of(l), out = out_of(l - 1);
 #pragma unroll
-    for (int cb = 0; cb < NB; ++cb) head_quad(0, cb, dsr[cb], drr[cb][0], drr[cb][1], drr[cb][2]);
-    f32x16 acc[8][NB];
-    product<P, NB, 1, 8, kZero, 2>(acc, image(8), nullptr, fin_z, st, NextChunk{image(7), kChunk}, side_of(I1{}, 7, 8));
-    static_for<0, 8>([&](auto TI) SRF_AI { masked_epi(TI, acc[decltype(TI)::value]); });
+    for (int cb = 0; cb < NB; ++cb) mlast[cb] = mb[cb][3];
+    load_masks(l - 1);
+    static_for<0, 8>([&](auto TI) SRF_AI {
+      constexpr int T = decltype(TI)::value;
+      st.template sync<kSt>();
+      if constexpr (T == 0) tile(I2{}, acc[0], src, epi(I7{}, I2{}, src, prev));
+      else tile(I1{}, acc[T & 1], src, epi(std::integral_constant<int, T - 1>{}, I1{}, dst, out));
+    });
+  };
+#pragma unroll 1
+  for (int l = 7;; l -= 2) {
+    layer(l, zb, za);
+    if (l == 1) break;
+    layer(l - 1, za, zb);
   }
-  // trunk: z holds dZ_l; dH_{l-1} = W_l^T dZ_l, masked -> dZ_{l-1}, in place (storing dZ_l)
-  for (int l = 7; l >= 1; --l) {
-    f32x16 acc[8][NB];
-    product<P, NB, 16, 8, kZero, 17>(acc, image(l), nullptr, fin_z, st, NextChunk{image(l > 1 ? l - 1 : 1), l > 1 ? kChunk : 0},
-                                     side_of(I1{}, l - 1, l));
-    static_for<0, 8>([&](auto TI) SRF_AI { masked_epi(TI, acc[decltype(TI)::value]); });
-  }
-  // dZ0: no product follows
-  const Rsrc rz = uniform_rsrc(a.ws + a.w.dz[0]);
-  static_for<0, 16>([&](auto TI) SRF_AI {
-    constexpr int t = decltype(TI)::value;
-    store_tile16<t>(rz, tile_block<P>(t, ldP, pl.elem, p0), z[t & ~1], z[t | 1]);
-  });
+  all_pieces(epi(I7{}, I1{}, za, out_of(0)));
+  wait_vmem();  // the copies past the last unit
 }
 
 template <int P, bool VD, bool TRAIN, int NB>

@@ -51,8 +51,10 @@ constexpr int kParams = SRF_MLP_NUM_PARAMS;
 constexpr int kMaskSlots = 9;      // ReLU masks of layers 0-7 and the view layer
 constexpr int kWaves = 4;          // waves per block
 constexpr int kMaxJobs = 16;
-// padded biases of the largest model: trunk 8 x 256, head 288, view 128, rgb 32
-constexpr int kMaxBiasFloats = 8 * 256 + 288 + 128 + 32;
+// padded biases of the largest model (trunk 8 x 256, head 288, view 128, rgb 32), in whole KB
+constexpr int kMaxBiasFloats = 2560;
+static_assert(kMaxBiasFloats >= 8 * 256 + 288 + 128 + 32, "");
+constexpr int kPackPad = 17 * 4096;  // bytes past the packed image that the 16-bit kernels may copy (mlp16.h)
 
 // ----------------------------------------------------------------------------- plan
 struct Plan {
@@ -66,6 +68,7 @@ struct Plan {
   int out_rows[kLayers], out_tiles[kLayers], reg_tiles[kLayers], comp_feats[kLayers],
       comp_tiles[kLayers], bwd_tiles[kLayers], present[kLayers];
   int fwd_rows_t[kLayers], bwd_rows_t[kLayers];  // row tiles of the forward / transposed image
+  int fwd_steps[kLayers], bwd_steps[kLayers];    // 32-row tiles: fragments of a row tile (mlp16.h)
   int bias_floats;  // padded biases of every present layer, contiguous from bias_off[0]
   size_t fwd_off[kLayers], bwd_off[kLayers], bias_off[kLayers], packed_bytes;
 };
@@ -127,12 +130,17 @@ inline bool make_plan(const srf_mlp_desc* d, Plan* p) {
     p->bwd_rows_t[l] = 16 * p->reg_tiles[l] / p->row_tile;
     const int in_tiles = p->reg_tiles[l] + p->comp_tiles[l];
     p->fwd_off[l] = off;
-    off += (size_t)p->fwd_rows_t[l] * in_tiles * p->fwd_tile_bytes;
+    // 32-row tiles: whole units of four fragments a tile (one, where the product has a single k-step)
+    const auto padded = [](int steps) { return steps < 4 ? steps : round_up(steps, 4); };
+    p->fwd_steps[l] = padded(in_tiles);
+    p->bwd_steps[l] = padded(p->bwd_tiles[l]);
+    off += (size_t)p->fwd_rows_t[l] * (p->row_tile == 32 ? p->fwd_steps[l] : in_tiles) * p->fwd_tile_bytes;
   }
-  for (int l = 1; l < kLayers; ++l) {
+  // the transposed images in the order of their use, from the heads to layer 1
+  for (int l = kLayers - 1; l >= 1; --l) {
     if (!p->present[l]) continue;
     p->bwd_off[l] = off;
-    off += (size_t)p->bwd_rows_t[l] * p->bwd_tiles[l] * p->bwd_tile_bytes;
+    off += (size_t)p->bwd_rows_t[l] * (p->row_tile == 32 ? p->bwd_steps[l] : p->bwd_tiles[l]) * p->bwd_tile_bytes;
   }
   for (int l = 0; l < kLayers; ++l) {
     if (!p->present[l]) continue;
@@ -140,7 +148,7 @@ inline bool make_plan(const srf_mlp_desc* d, Plan* p) {
     off += (size_t)p->fwd_rows_t[l] * p->row_tile * sizeof(float);
     p->bias_floats += p->fwd_rows_t[l] * p->row_tile;
   }
-  p->packed_bytes = round_up((int)off, 256);
+  p->packed_bytes = round_up((int)off, 256) + (p->row_tile == 32 ? kPackPad : 0);
   return true;
 }
 

@@ -33,6 +33,10 @@ HIPCC_FLAGS = [
     f'-I{REPO_DIR / "include"}',
 ]
 
+# flags of single sources: the 16-bit MLP kernels keep their accumulators in vector registers, which their
+# epilogues read directly, and the activations in the accumulation registers (csrc/mlp16.h)
+SOURCE_FLAGS = {name: ['-mllvm', '-amdgpu-mfma-vgpr-form'] for name in ('mlp_bf16', 'mlp_f16')}
+
 
 def _hipcc() -> str:
     for cand in (shutil.which('hipcc'), '/opt/rocm/bin/hipcc'):
@@ -56,7 +60,7 @@ def _compile(src: Path, extra: list[str], incremental: bool = False) -> Path:
     obj = OBJ_DIR / (src.stem + '.o')
     if incremental and _up_to_date(src, obj):
         return obj
-    cmd = [_hipcc(), *HIPCC_FLAGS, *extra, '-c', str(src), '-o', str(obj)]
+    cmd = [_hipcc(), *HIPCC_FLAGS, *SOURCE_FLAGS.get(src.stem, []), *extra, '-c', str(src), '-o', str(obj)]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f'hipcc failed for {src.name}:\n{" ".join(cmd)}\n{res.stdout}\n{res.stderr}')
