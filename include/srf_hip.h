@@ -477,8 +477,10 @@ int srf_adam_step(int n_tensors, float* const* params, const float* const* grads
  * built-in choice; results are the same for every value up to the order of FP32 atomic
  * additions.  Launches read the table when they are issued, so a captured graph keeps the
  * values it was captured with. */
-#define SRF_TUNE_DW_CHUNK 0       /* points per work item of the MLP weight-gradient GEMM (srf_mlp_weight_grads):
-                                     0 = about 1024 work items; else 2048..262144, a multiple of 256 */
+#define SRF_TUNE_DW_CHUNK 0       /* points per work item of the MLP weight-gradient GEMM (srf_mlp_weight_grads;
+                                     16-bit operands: of a 256 x 256 layer, the others in proportion):
+                                     0 = whole rounds of the compute units; else 2048..262144, a multiple of
+                                     256 */
 #define SRF_TUNE_COLOR_DW_CHUNK 1 /* the same for the colour network's weight gradients (srf_color_backward):
                                      0 = adaptive; else 2048..65536, a multiple of 256 */
 #define SRF_TUNE_GATHER_BLOCKS 2  /* grid cap of the factor-gather kernels (srf_vm_*, srf_cp_*): 0 = 8192;

@@ -172,6 +172,13 @@ __device__ __forceinline__ uint32_t lds_offset(const void* p) {
   return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)p);
 }
 
+// A block barrier that waits for no memory operation (__syncthreads would drain the copies in flight).
+__device__ __forceinline__ void block_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
 // Wait for every outstanding vector-memory operation of this wave (LDS DMA included).
 __device__ __forceinline__ void wait_vmem() { __builtin_amdgcn_s_waitcnt(0); }
 

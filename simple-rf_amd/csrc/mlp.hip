@@ -3,6 +3,7 @@
 #include <string.h>
 
 #include "mlp_impl.h"
+#include "mlp16_dw.h"
 
 namespace srf {
 namespace mlp {
@@ -192,7 +193,6 @@ int bwd_launch(int prec, const BwdArgs& a, bool vd, hipStream_t s) {
 int dw_launch(int prec, const DwArgs& d, hipStream_t s) {
   switch (prec) {
     case SRF_PREC_F32: return dw_f32(d, s);
-    case SRF_PREC_BF16: return dw_bf16(d, s);
     case SRF_PREC_BF16_SPLIT: return dw_bf16s(d, s);
     default: return SRF_EUNSUPPORTED;
   }
@@ -302,6 +302,86 @@ extern "C" int srf_mlp_forward_rays(const srf_mlp_desc* desc, const void* packed
                           noise, sigma, rgb, workspace, stream);
 }
 
+// The weight gradients of 16-bit operands (mlp16_dw.h): the jobs, and for each the points of a block.
+static int weight_grads16(const Plan& p, const Ws& w, uint8_t* ws, float* const* d_weights, float* const* d_biases,
+                          hipStream_t s) {
+  Dw16Args d;
+  memset(&d, 0, sizeof(d));
+  d.ldP = w.ldP;
+  d.cols = w.cols;
+  const int D = p.trunk_pe, pe_tiles = round_up(D, 32) / 16;
+  auto job = [&](int kind, int l, int n_dz, size_t x, int n_x, int M, int N, float* dw, int ld, float* db) -> Dw16Job& {
+    Dw16Job& j = d.jobs[d.n_jobs++];
+    j.kind = kind;
+    j.dz = ws + w.dz[l];
+    j.n_dz = n_dz;
+    j.x = ws + x;
+    j.n_x = n_x;
+    j.M = M;
+    j.N = N;
+    j.dw = dw;
+    j.ld = ld;
+    j.db = db;
+    return j;
+  };
+  job(kDwNarrow, 0, 16, w.x0, pe_tiles, 256, D, d_weights[0], D, d_biases[0]);
+  for (int l = 1; l < 8; ++l) {
+    if (l == 5) {
+      Dw16Job& j = job(kDwWide, 5, 16, w.h[4], 16, 256, 256, d_weights[5] + D, D + 256, d_biases[5]);
+      j.x2 = ws + w.x0;
+      j.n_x2 = pe_tiles;
+      j.N2 = D;
+      j.dw2 = d_weights[5];
+    } else {
+      job(kDwFull, l, 16, w.h[l - 1], 16, 256, 256, d_weights[l], 256, d_biases[l]);
+    }
+  }
+  if (p.view_dep) {
+    Dw16Job& t = job(kDwTall, 8, 17, w.h[7], 16, 256, 256, d_weights[8], 256, d_biases[8]);
+    t.dw_row = d_weights[9];
+    t.db_row = d_biases[9];
+    Dw16Job& v = job(kDwHalf, 9, 8, w.f, 16, 128, 256, d_weights[10], 256 + p.extra, d_biases[10]);
+    v.x2 = ws + w.ex;
+    v.n_x2 = round_up(p.extra, 32) / 16;
+    v.N2 = p.extra;
+    v.dw2 = d_weights[10] + 256;
+    job(kDwRow, 10, 1, w.v, 8, 3, 128, d_weights[11], 128, d_biases[11]);
+  } else {
+    job(kDwRow, 8, 1, w.h[7], 16, 4, 256, d_weights[9], 256, d_biases[9]);
+  }
+  // Points of a block: a unit of 32 points costs about its fragments (KB to read) and the step itself, worth
+  // kStep of them, and every block gets the same cost: one block to each compute unit (the ring takes its
+  // LDS), or two where a block of a 256 x 256 layer would reduce more than kLong points, and at least kLeast
+  // points.  Measured (main model): 65,536 points 170 us in one round, 199 in two, 231 in three (each block
+  // adds 256 KB with atomics); 262,144 points 517, 523, 550; 786,432 points 1,495, 1,440, 1,436 (a second
+  // round evens out the compute units).  16,384 points 87 us with 512 points a block, 79 with 1,024, 82
+  // with 1,536.
+  constexpr int kStep = 6, kLeast = 1024, kLong = 20000;
+  auto cost = [](const Dw16Job& j) { return j.n_dz + j.n_x + j.n_x2 + kStep; };
+  const int64_t tuned = tune_value(SRF_TUNE_DW_CHUNK);  // points of a block of a 256 x 256 layer
+  double per_block = 0.;                                // points x cost
+  for (int i = 0; i < d.n_jobs; ++i) per_block += (double)w.cols * cost(d.jobs[i]);
+  const int cus = device_compute_units();
+  const int rounds = per_block / cus > (double)kLong * (32 + kStep) ? 2 : 1;
+  per_block /= (double)rounds * cus;
+  if (tuned) per_block = (double)tuned * (32 + kStep);
+  int blocks = 0;
+  for (int pass = 0;; ++pass) {
+    blocks = 0;
+    for (int i = 0; i < d.n_jobs; ++i) {
+      Dw16Job& j = d.jobs[i];
+      j.first_block = blocks;
+      j.chunk = (int)(per_block / cost(j)) / 64 * 64;
+      if (j.chunk < kLeast) j.chunk = kLeast;
+      blocks += (w.cols + j.chunk - 1) / j.chunk;
+    }
+    // (the jobs' last, partly filled blocks: no more than whole rounds)
+    if (tuned || pass == 40 || blocks <= rounds * cus) break;
+    per_block *= 1.005;
+  }
+  return dw16_launch(d, blocks, s);
+}
+
 static int mlp_backward_impl(const srf_mlp_desc* desc, const void* packed, int n_points,
                              const float* sigma, const float* rgb, const float* d_sigma,
                              const float* d_rgb, void* workspace, float* const* d_weights,
@@ -336,6 +416,7 @@ static int mlp_backward_impl(const srf_mlp_desc* desc, const void* packed, int n
     const int st = bwd_launch(p.prec, b, p.view_dep, s);
     if (st != SRF_OK || !weights) return st;
   }
+  if (p.prec == SRF_PREC_BF16) return weight_grads16(p, w, ws, d_weights, d_biases, s);
   // grouped weight-gradient GEMM
   const size_t rb = (size_t)w.ldP * p.elem;  // bytes per stored row
   DwArgs d;

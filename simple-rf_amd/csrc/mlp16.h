@@ -91,9 +91,7 @@ struct Stream16 {
   __device__ SRF_AI void sync() {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(vmcnt_only(kAhead - 7 + kStores));
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
+    block_barrier();
     __builtin_amdgcn_sched_barrier(0);
   }
   // One unit: f(i, fragment) for its four fragments, reading the next unit's meanwhile.

@@ -13,7 +13,5 @@ int bwd_bf16(const BwdArgs& a, bool vd, hipStream_t s) {
   return vd ? launch_bwd16<kBF16, true>(a, s) : launch_bwd16<kBF16, false>(a, s);
 }
 
-int dw_bf16(const DwArgs& d, hipStream_t s) { return launch_dw<kBF16>(d, s); }
-
 }  // namespace mlp
 }  // namespace srf

@@ -1178,7 +1178,7 @@ __device__ __forceinline__ int dw_cols(const DwArgs& a) {
 // One block of 8 waves reduces a 256 x 256 tile of dW = dZ X^T (a whole layer of the MLP) over a
 // chunk of points, so every dZ and X row of the chunk is read from HBM once; the reduction over
 // points streams at the HBM rate (a 256 x 256 layer does 128 FLOP per byte of dZ and X, below
-// the MFMA:HBM balance of the chip).  Per k-unit (32 points for 16-bit operands, 16 for FP32)
+// the MFMA:HBM balance of the chip).  Per k-unit (16 points)
 // the 16 dZ-row and 16 X-row fragments of the tile (1 KB each, gathered from the feature-major
 // arrays by per-lane addresses) are copied global -> LDS by the eight waves into a ring of four
 // k-unit slots, three k-units ahead of the one being multiplied (96 KB in flight per CU to cover
@@ -1221,9 +1221,9 @@ __global__ __launch_bounds__(64 * kDwWaves) void mlp_dw_kernel(DwArgs a) {
   const int pe = min(pb + a.chunk, dw_cols(a));
   if (pb >= pe) return;  // the chunk lies past the device-side count (uniform over the block)
   const size_t ldP = a.ldP;
-  constexpr bool F32L = f32_layout<P>();
-  constexpr int ELEM = F32L ? 4 : 2;
-  constexpr int KPTS = F32L ? 16 : 32;  // points per k-unit (split BF16: two units per MFMA k-step)
+  static_assert(P == kF32, "16-bit operands: mlp16_dw.h; split BF16: mlp_dw_split_kernel");
+  constexpr int ELEM = 4;
+  constexpr int KPTS = 16;  // points per k-unit
   const int qm = kRowWaves ? w : RM * (w >> 1), qn = kRowWaves ? 0 : 8 * (w & 1);
   bool mv[RM], nv[NC];
 #pragma unroll
@@ -1270,34 +1270,22 @@ __global__ __launch_bounds__(64 * kDwWaves) void mlp_dw_kernel(DwArgs a) {
       if (a.paired) {
         // lane (g, j) takes feature j's chunk of the record pair m = 4 u + g of the 2 KB block of
         // the points' wave (see store_tile): record (j >> 2, 2 m + ((j >> 1) & 1)), chunk j & 1
-        // 16-bit values (store_tile16): LDS position l of the fragment takes chunk (l >> 1) & 1 of record
-        // (h = l & 1, c = 16 u + 4 ((l >> 2) & 3) + (l >> 4)), so that operand lane (g', j') finds
-        // feature j' at the points c, 32 + c of c = 16 u + 4 g' + i as dword i (frag16: 4 B at 4 lane +
-        // 256 i, contiguous over the wave).
-        constexpr int PPW = F32L ? 32 : 64;  // points per stored wave block
+        constexpr int PPW = 32;  // points per stored wave block
         const int wb = p / PPW, u = (p % PPW) / KPTS;
-        const int rec = F32L ? 16 * (j >> 2) + 2 * (4 * u + g) + ((j >> 1) & 1)
-                             : 32 * (lane & 1) + 16 * u + 4 * ((lane >> 2) & 3) + (lane >> 4);
-        const int piece = F32L ? j & 1 : (lane >> 1) & 1;
+        const int rec = 16 * (j >> 2) + 2 * (4 * u + g) + ((j >> 1) & 1);
         // the wide tilings read tile-major blocks (tile t's blocks span 16 rows of ldP points, the MLP
         // workspace); the narrow one point-block-major blocks (the array's tiles of one wave block
         // adjacent, 2 KB each: the colour network's workspace)
         size_t blk;
         if constexpr (kRowWaves) blk = ((size_t)wb * ((is_a ? jb.dz_rows : jb.x_rows) / 16) + row0 / 16) * 2048;
         else blk = (size_t)row0 * ldP * ELEM + (size_t)wb * 2048;
-        src = base + blk + piece * 1024 + rec * 16;
+        src = base + blk + (j & 1) * 1024 + rec * 16;
       } else {
-        const int pg = F32L ? 4 * g : 8 * g;
-        src = base + (((size_t)(row0 + j)) * ldP + p + pg) * ELEM;
+        src = base + (((size_t)(row0 + j)) * ldP + p + 4 * g) * ELEM;
       }
       __builtin_amdgcn_global_load_lds((const void*)src,
                                        (__attribute__((address_space(3))) void*)(buf + f * 1024), 16, 0, 0);
     }
-  };
-  // one operand fragment of 16-bit values (see dma_unit)
-  auto frag16 = [&](const uint8_t* f) SRF_AI {
-    const uint32_t* v = reinterpret_cast<const uint32_t*>(f) + lane;
-    return u32x4{v[0], v[64], v[128], v[192]};
   };
   f32x4 acc[RM][NC];
   float rs[RM];
@@ -1345,50 +1333,31 @@ __global__ __launch_bounds__(64 * kDwWaves) void mlp_dw_kernel(DwArgs a) {
       // per k-unit.  Wide tilings: every tile's product runs (a tile past the job's rows multiplies
       // the re-read first row tile; the epilogue stores only the valid tiles), since a second,
       // unguarded copy of their products spills.
-      if constexpr (P == kF32) {
-        f32x4 av[RM], bv[NC];
+      f32x4 av[RM], bv[NC];
 #pragma unroll
-        for (int i = 0; i < RM; ++i) av[i] = *reinterpret_cast<const f32x4*>(fr + (qm + i) * 1024 + lane * 16);
+      for (int i = 0; i < RM; ++i) av[i] = *reinterpret_cast<const f32x4*>(fr + (qm + i) * 1024 + lane * 16);
 #pragma unroll
-        for (int k = 0; k < NC; ++k) bv[k] = *reinterpret_cast<const f32x4*>(fr + (16 + qn + k) * 1024 + lane * 16);
-        auto prod = [&](auto NRI, auto NVI) SRF_AI {
-          constexpr int NR = decltype(NRI)::value, NV = decltype(NVI)::value;
+      for (int k = 0; k < NC; ++k) bv[k] = *reinterpret_cast<const f32x4*>(fr + (16 + qn + k) * 1024 + lane * 16);
+      auto prod = [&](auto NRI, auto NVI) SRF_AI {
+        constexpr int NR = decltype(NRI)::value, NV = decltype(NVI)::value;
 #pragma unroll
-          for (int q = 0; q < 4; ++q)
+        for (int q = 0; q < 4; ++q)
 #pragma unroll
-            for (int i = 0; i < NR; ++i)
+          for (int i = 0; i < NR; ++i)
 #pragma unroll
-              for (int k = 0; k < NV; ++k) acc[i][k] = mfma32(av[i][q], bv[k][q], acc[i][k]);
-        };
-        if constexpr (kRowWaves) {
-          if (nmv == RM)
-            static_for<1, NC + 1>([&](auto VI) SRF_AI {
-              if (nnv == decltype(VI)::value) prod(std::integral_constant<int, RM>{}, VI);
-            });
-        } else {
-          prod(std::integral_constant<int, RM>{}, std::integral_constant<int, NC>{});  // as the 16-bit tiling
-        }
-        if (do_db)
-#pragma unroll
-          for (int i = 0; i < RM; ++i) rs[i] += (av[i][0] + av[i][1]) + (av[i][2] + av[i][3]);
+            for (int k = 0; k < NV; ++k) acc[i][k] = mfma32(av[i][q], bv[k][q], acc[i][k]);
+      };
+      if constexpr (kRowWaves) {
+        if (nmv == RM)
+          static_for<1, NC + 1>([&](auto VI) SRF_AI {
+            if (nnv == decltype(VI)::value) prod(std::integral_constant<int, RM>{}, VI);
+          });
       } else {
-        u32x4 av[RM], bv[NC];
-#pragma unroll
-        for (int i = 0; i < RM; ++i) av[i] = frag16(fr + (qm + i) * 1024);
-#pragma unroll
-        for (int k = 0; k < NC; ++k) bv[k] = frag16(fr + (16 + qn + k) * 1024);
-        // every tile's product, valid or not (the epilogue stores the valid ones; the slot holds a
-        // whole k-unit either way): no branch between the MFMAs
-#pragma unroll
-        for (int i = 0; i < RM; ++i)
-#pragma unroll
-          for (int k = 0; k < NC; ++k) acc[i][k] = mfma16<P>(av[i], bv[k], acc[i][k]);
-        if (do_db)
-#pragma unroll
-          for (int i = 0; i < RM; ++i)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) rs[i] += unpack_lo<P>(av[i][q]) + unpack_hi<P>(av[i][q]);
+        prod(std::integral_constant<int, RM>{}, std::integral_constant<int, NC>{});
       }
+      if (do_db)
+#pragma unroll
+        for (int i = 0; i < RM; ++i) rs[i] += (av[i][0] + av[i][1]) + (av[i][2] + av[i][3]);
     }
   }
 #pragma unroll
@@ -1593,7 +1562,6 @@ int fwd_f16(const FwdArgs& a, bool vd, bool tr, hipStream_t s);
 int bwd_f32(const BwdArgs& a, bool vd, hipStream_t s);
 int bwd_bf16(const BwdArgs& a, bool vd, hipStream_t s);
 int dw_f32(const DwArgs& d, hipStream_t s);
-int dw_bf16(const DwArgs& d, hipStream_t s);
 int dw_f32_narrow(const DwArgs& d, hipStream_t s);  // 128 x 160 tiles (kDwNarrowRows x kDwNarrowCols)
 int fwd_bf16s(const FwdArgs& a, bool vd, bool tr, hipStream_t s);  // split BF16 (mlp_bf16s.hip)
 int bwd_bf16s(const BwdArgs& a, bool vd, hipStream_t s);

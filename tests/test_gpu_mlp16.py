@@ -61,3 +61,23 @@ def test_gradients_of_a_prefix(cuda, variant, n):
     part = torch.autograd.grad(hm.mlp_forward(spec, w, b, pts[:n], dirs[:n]), p, (gs[:n], gc[:n]))
     for x, y in zip(part, full):
         assert (x - y).norm() <= 3.6e-5 * y.norm(), n
+
+
+@pytest.mark.parametrize('variant', list(VARIANTS))
+@pytest.mark.parametrize('n,cut', [(1025, 1024), (5000, 2437), (20011, 64)])
+def test_gradients_add_up(cuda, variant, n, cut):
+    """The weight gradients over several blocks' ranges of points: a call's are the sum of its two parts',
+    up to the FP32 sum of n terms (n 2^-24)."""
+    spec = hm.MLPSpec(prec='bf16', **VARIANTS[variant]['spec'])
+    w, b = leaves(spec, cuda)
+    p = [t.requires_grad_(True) for t in w + b if t is not None]
+    pts, dirs = (t.to(cuda) for t in points(n, 26))
+    g = torch.Generator().manual_seed(27)
+    gs = torch.rand(n, generator=g).to(cuda)
+    gc = torch.rand(n, 3, generator=g).to(cuda)
+
+    def grads(q):
+        return torch.autograd.grad(hm.mlp_forward(spec, w, b, pts[q], dirs[q]), p, (gs[q], gc[q]))
+    whole, one, two = grads(slice(0, n)), grads(slice(0, cut)), grads(slice(cut, n))
+    for x, y, z in zip(whole, one, two):
+        assert (x - (y + z)).norm() <= n * 2.0 ** -24 * x.norm()
