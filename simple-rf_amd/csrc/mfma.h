@@ -149,18 +149,12 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t (&out)[NP]
   }
 }
 
-// Direct global -> LDS copy of one 1 KB fragment by a whole wave (gfx950
-// global_load_lds_dwordx4): lane l's 16 bytes at src + 16 l land at lds_base + 16 l.  src is
-// the fragment base, lds_base must be wave-uniform.  Completion is tracked by vmcnt.
-__device__ __forceinline__ void lds_dma_1k(const uint8_t* src, uint8_t* lds_base) {
-  const int lane = threadIdx.x & 63;
-  __builtin_amdgcn_global_load_lds((const void*)(src + 16 * lane),
-                                   (__attribute__((address_space(3))) void*)lds_base, 16, 0, 0);
-}
-
-// The same copy (src and lds_offset wave-uniform, lane16 = 16 lane) without the compiler's knowledge: it makes every LDS read that follows the builtin wait for all vector-memory operations
-// (it cannot tell the buffers of a ring apart), which undoes a copy ahead of its use.  The caller waits
-// for the copy (s_waitcnt vmcnt) and synchronises before it is read.
+// Direct global -> LDS copy of one 1 KB fragment by a whole wave (gfx950 global_load_lds_dwordx4): lane l's
+// 16 bytes at src + (lane16 of lane l) land at lds_offset + 16 l.  src and lds_offset are wave-uniform.
+// Completion is tracked by vmcnt.  Written out, without the compiler's knowledge: it makes the first LDS
+// read that follows the builtin wait for all vector-memory operations (it cannot tell the buffers of a
+// stage or ring apart), which undoes a copy ahead of its use and drains the stores behind it.  The caller
+// waits for the copy (s_waitcnt vmcnt) and synchronises before it is read.
 __device__ __forceinline__ void lds_dma_1k_ahead(const uint8_t* src, uint32_t lds_offset, uint32_t lane16) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                :
@@ -170,6 +164,13 @@ __device__ __forceinline__ void lds_dma_1k_ahead(const uint8_t* src, uint32_t ld
 // Offset of an LDS object, as lds_dma_1k_ahead takes it.
 __device__ __forceinline__ uint32_t lds_offset(const void* p) {
   return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)p);
+}
+// The same for a fragment that lies in lane order at src.
+__device__ __forceinline__ void lds_dma_1k(const uint8_t* src, uint8_t* lds_base) {
+  const uint64_t v = reinterpret_cast<uint64_t>(src);
+  const uint64_t u = (uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(v >> 32)) << 32 |
+                     (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)v);
+  lds_dma_1k_ahead(reinterpret_cast<const uint8_t*>(u), lds_offset(lds_base), (threadIdx.x & 63) * 16);
 }
 
 // A block barrier that waits for no memory operation (__syncthreads would drain the copies in flight).
