@@ -14,8 +14,7 @@
 // streamed global -> LDS by the four waves of a block (double-buffered, as in mlp::mma_tiles) and
 // shared by them.  The basis output F and the view directions go through a per-wave LDS tile from
 // which every lane builds its positional-encoding inputs.  Training stores the layer inputs and
-// output gradients as FP32 tile blocks (store_tile_rows) for the weight-gradient GEMMs: the MLP's
-// FP32 grouped GEMM (mlp_dw_kernel, 128 x 160 tiles) or color_dw_kernel.
+// output gradients as FP32 tile blocks (store_tile_rows) for the weight-gradient kernel (color_dw.h).
 //
 // Operand precision (desc->prec).  Activations, accumulators and the stored layer inputs are FP32
 // in every mode; the products of the forward and of the backward chain multiply
@@ -25,10 +24,13 @@
 //                         backward chain (three products), as the NeRF MLP's split mode
 //   SRF_PREC_BF16         BF16 operands rounded from the FP32 activations and weights (one plane)
 // Reduction depths are padded to whole k-units (32 features for the BF16 modes) with zeros.  The
-// weight gradients reduce the stored FP32 tiles with the FP32 GEMM (SRF_PREC_F32) or the split-BF16
-// one, two planes per operand (both BF16 modes).
+// weight gradients reduce the stored FP32 tiles with FP32 products (SRF_PREC_F32) or split-BF16
+// ones, two planes per operand (both BF16 modes).
 #include <string.h>
 
+#include <algorithm>
+
+#include "color_dw.h"
 #include "mlp_impl.h"
 
 namespace srf {
@@ -737,195 +739,6 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
 
 __global__ __launch_bounds__(64 * kWaves) void color_bwd_split_kernel(BwdArgs a) { color_bwd_body<kBFS2>(a); }
 
-// ------------------------------------------------------------------- weight gradients
-// dW = dZ X^T (+ db = row sums of dZ) of the four colour jobs (W1, W2, W3, basis) over the stored
-// FP32 tile blocks, in the BF16 modes (FP32: the MLP's FP32 GEMM, mlp_dw_kernel).  A work item is one
-// job over one chunk of points; its block copies, per 16-point unit, only the job's own fragments
-// (nA dZ and nB X row tiles, one contiguous 1 KB each) global -> LDS into a ring whose slot holds two
-// units, 2 (nA + nB) KB, so a job of 9-24 fragments keeps 4-14 units in flight in the 160 KB of LDS
-// with one barrier per two units (10 % faster than one per unit on the 300^2 step).  The
-// products are split-BF16 32x32x16 MFMAs (dZ_hi X_hi + dZ_hi X_lo + dZ_lo X_hi, as
-// mlp_dw_split_kernel); wave w multiplies row block w & 3 (32 rows) by column blocks 4 (w >> 2) .. + 3
-// (32 columns each).  Partial sums go to dW with FP32 atomics.
-constexpr int kCdwWaves = 8;
-constexpr int kCdwRingKB = 160;
-constexpr int kCdwMaxSlots = 8;
-constexpr int kCdwMaxA = 8, kCdwMaxB = 16;  // row tiles: dZ <= 128 rows, X <= 256 rows
-
-struct CdwJob {
-  const uint8_t* dz;
-  const uint8_t* x;
-  int nA, nB;  // 16-row tiles of dZ and X (the tiles of their arrays)
-  int M, N;    // valid rows and columns of dW
-  float* dw;
-  int ld_dw;
-  float* db;
-};
-
-struct CdwArgs {
-  CdwJob jobs[4];
-  int n_jobs, cols, chunk;
-  const int32_t* cols_dev;
-};
-
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-// s_waitcnt vmcnt(n) for a wave-uniform n in 0..47.
-__device__ __forceinline__ void wait_vmem_le(int n) {
-  switch (n) {
-#define SRF_WAIT_CASE(k) case k: __builtin_amdgcn_s_waitcnt(mlp::vmcnt_only(k)); break;
-    SRF_WAIT_CASE(0) SRF_WAIT_CASE(1) SRF_WAIT_CASE(2) SRF_WAIT_CASE(3) SRF_WAIT_CASE(4) SRF_WAIT_CASE(5)
-    SRF_WAIT_CASE(6) SRF_WAIT_CASE(7) SRF_WAIT_CASE(8) SRF_WAIT_CASE(9) SRF_WAIT_CASE(10) SRF_WAIT_CASE(11)
-    SRF_WAIT_CASE(12) SRF_WAIT_CASE(13) SRF_WAIT_CASE(14) SRF_WAIT_CASE(15) SRF_WAIT_CASE(16) SRF_WAIT_CASE(17)
-    SRF_WAIT_CASE(18) SRF_WAIT_CASE(19) SRF_WAIT_CASE(20) SRF_WAIT_CASE(21) SRF_WAIT_CASE(22) SRF_WAIT_CASE(23)
-    SRF_WAIT_CASE(24) SRF_WAIT_CASE(25) SRF_WAIT_CASE(26) SRF_WAIT_CASE(27) SRF_WAIT_CASE(28) SRF_WAIT_CASE(29)
-    SRF_WAIT_CASE(30) SRF_WAIT_CASE(31) SRF_WAIT_CASE(32) SRF_WAIT_CASE(33) SRF_WAIT_CASE(34) SRF_WAIT_CASE(35)
-    SRF_WAIT_CASE(36) SRF_WAIT_CASE(37) SRF_WAIT_CASE(38) SRF_WAIT_CASE(39) SRF_WAIT_CASE(40) SRF_WAIT_CASE(41)
-    SRF_WAIT_CASE(42) SRF_WAIT_CASE(43) SRF_WAIT_CASE(44) SRF_WAIT_CASE(45) SRF_WAIT_CASE(46)
-#undef SRF_WAIT_CASE
-    default: __builtin_amdgcn_s_waitcnt(mlp::vmcnt_only(47)); break;
-  }
-}
-
-__global__ __launch_bounds__(64 * kCdwWaves) void color_dw_kernel(CdwArgs a) {
-  __shared__ __attribute__((aligned(16))) uint8_t ring[kCdwRingKB * 1024];
-  const int lane = threadIdx.x & 63, g = lane >> 4, j = lane & 15;
-  const int h = lane >> 5, i32 = lane & 31;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // items are chunk-major, so that the items with points (the first chunks) of all jobs come first
-  const int job = blockIdx.x % a.n_jobs, chunk = blockIdx.x / a.n_jobs;
-  const CdwJob& jb = a.jobs[job];
-  const int cols = a.cols_dev ? min(a.cols, (*a.cols_dev + 255) / 256 * 256) : a.cols;
-  const int pb = chunk * a.chunk;
-  const int pe = min(pb + a.chunk, cols);
-  if (pb >= pe) return;  // past the device-side count (uniform over the block)
-  const int nA = jb.nA, nB = jb.nB, nf = nA + nB;
-  const int nslots = min(kCdwMaxSlots, kCdwRingKB / (2 * nf));  // two-unit slots
-  const int dma_n = (nf - w + kCdwWaves - 1) / kCdwWaves;  // this wave's fragments per unit (<= 3)
-  // unit at point p: fragment f < nA is dZ row tile f, else X row tile f - nA; lane (g, j) copies
-  // the 16 B of feature j at the four points of lane group g (the record of mlp::store_tile), to
-  // slot byte f KB + 16 lane
-  // the job's array bases, read from the kernel arguments once (wave-uniform, scalar registers)
-  const uint8_t* const dz_base = jb.dz;
-  const uint8_t* const x_base = jb.x;
-  auto dma_unit = [&](int p, uint8_t* buf) {
-    const int u = (p & 31) >> 4;
-    const int rec = 16 * (j >> 2) + 2 * (4 * u + g) + ((j >> 1) & 1);
-    const uint32_t in_blk = (j & 1) * 1024 + rec * 16;
-    for (int q = 0; q < 3; ++q) {
-      const int f = w + kCdwWaves * q;
-      if (f >= nf) break;
-      const uint8_t* src = f < nA ? dz_base + blk_off(nA, f, p) : x_base + blk_off(nB, f - nA, p);
-      __builtin_amdgcn_global_load_lds((const void*)(src + in_blk),
-                                       (__attribute__((address_space(3))) void*)(buf + f * 1024), 16, 0, 0);
-    }
-  };
-  // row block rb (32 rows), column blocks cq .. cq + 3
-  const int rb = w & 3, cq = 4 * (w >> 2);
-  const bool row_ok = 2 * rb < nA;
-  bool col_ok[4];
-  bool any_col = false;
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    col_ok[c] = 2 * (cq + c) < nB;
-    any_col |= col_ok[c];
-  }
-  const bool do_db = jb.db != nullptr && cq == 0;
-  const bool busy = row_ok && (any_col || do_db);
-  // the fragments this lane's half (i32 >> 4) reads: a 32-row block's second tile past the job's
-  // rows repeats the first (rows past M are not stored)
-  const int fa = min(2 * rb + (i32 >> 4), nA - 1);
-  int fb[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) fb[c] = nA + min(2 * (cq + c) + (i32 >> 4), nB - 1);
-  f32x16 acc[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[c][r] = 0.f;
-  float rs = 0.f;
-  // the two BF16 planes of the eight FP32 values lane (h, i) takes from fragment f: records of lane
-  // groups 2h and 2h + 1 of its row i mod 16
-  auto planes = [&](const uint8_t* fr, int f, u32x4& hi, u32x4& lo, bool sum) {
-    const int jj = i32 & 15;
-    const f32x4 v0 = *reinterpret_cast<const f32x4*>(fr + f * 1024 + ((2 * h) * 16 + jj) * 16);
-    const f32x4 v1 = *reinterpret_cast<const f32x4*>(fr + f * 1024 + ((2 * h + 1) * 16 + jj) * 16);
-    uint32_t t[4][2];
-    split_pair<2>(v0[0], v0[1], t[0]);
-    split_pair<2>(v0[2], v0[3], t[1]);
-    split_pair<2>(v1[0], v1[1], t[2]);
-    split_pair<2>(v1[2], v1[3], t[3]);
-    hi = u32x4{t[0][0], t[1][0], t[2][0], t[3][0]};
-    lo = u32x4{t[0][1], t[1][1], t[2][1], t[3][1]};
-    if (sum) rs += ((v0[0] + v0[1]) + (v0[2] + v0[3])) + ((v1[0] + v1[1]) + (v1[2] + v1[3]));
-  };
-  // The ring advances by steps of two units (one 32-point tile block, both halves): one barrier and one
-  // wait per step.
-  const int n_steps = (pe - pb) / 32;
-  const int slot = 2 * nf * 1024;
-  auto dma_step = [&](int p, uint8_t* buf) {
-    dma_unit(p, buf);
-    dma_unit(p + 16, buf + nf * 1024);
-  };
-  // the valid column blocks are a prefix (ncol of them, uniform over the wave): the products run as
-  // straight-line code for that count, one uniform choice per unit instead of a branch per MFMA
-  int ncol = 0;
-#pragma unroll
-  for (int c = 0; c < 4; ++c) ncol += col_ok[c] ? 1 : 0;
-  ncol = __builtin_amdgcn_readfirstlane(ncol);
-  auto unit_products = [&](const uint8_t* fr) {
-    u32x4 ah, al, bh[4], bl[4];
-    planes(fr, fa, ah, al, do_db);
-    mlp::static_for<1, 5>([&](auto NI) {
-      constexpr int NCOL = decltype(NI)::value;
-      if (ncol != NCOL) return;
-#pragma unroll
-      for (int c = 0; c < NCOL; ++c) planes(fr, fb[c], bh[c], bl[c], false);
-#pragma unroll
-      for (int pr = 0; pr < 3; ++pr)
-#pragma unroll
-        for (int c = 0; c < NCOL; ++c)
-          acc[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, pr == 0 ? al : ah),
-                                                           __builtin_bit_cast(bf16x8, pr == 1 ? bl[c] : bh[c]),
-                                                           acc[c], 0, 0, 0);
-    });
-  };
-  for (int st = 0; st < nslots - 1 && st < n_steps; ++st) dma_step(pb + 32 * st, ring + st * slot);
-  for (int st = 0; st < n_steps; ++st) {
-    // step st has landed once at most (steps issued after it) x 2 dma_n loads are outstanding
-    wait_vmem_le(min(nslots - 2, n_steps - 1 - st) * 2 * dma_n);
-    // every wave's part of step st is in LDS, and slot (st - 1) mod nslots is free (the waves consumed
-    // their reads of it in the MFMAs of iteration st - 1); compiler-only fences around a plain
-    // s_barrier, which would otherwise drain the prefetches (vmcnt(0))
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (st + nslots - 1 < n_steps)
-      dma_step(pb + 32 * (st + nslots - 1), ring + ((st + nslots - 1) % nslots) * slot);
-    if (!busy) continue;
-    const uint8_t* fr = ring + (st % nslots) * slot;
-    unit_products(fr);
-    unit_products(fr + nf * 1024);
-  }
-  if (!row_ok) return;
-  // 32x32 D layout: lane l, register r holds row 8 (r / 4) + 4 (l / 32) + (r mod 4), column l mod 32
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    if (!col_ok[c]) continue;
-    const int col = 32 * (cq + c) + i32;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int o = 32 * rb + 8 * (r >> 2) + 4 * h + (r & 3);
-      if (o < jb.M && col < jb.N) unsafeAtomicAdd(jb.dw + (size_t)o * jb.ld_dw + col, acc[c][r]);
-    }
-  }
-  if (do_db) {
-    const float sr = rs + __shfl_xor(rs, 32, 64);
-    const int o = 32 * rb + i32;
-    if (h == 0 && o < jb.M) unsafeAtomicAdd(jb.db + o, sr);
-  }
-}
-
 }  // namespace
 }  // namespace color
 }  // namespace srf
@@ -1076,50 +889,7 @@ extern "C" int srf_color_backward(const srf_color_desc* desc, const void* packed
     return SRF_EINVAL;
   c.cols = w.cols;
   c.cols_dev = point_count;
-  // 3840-point chunks by default (the items of the capacity's chunks past the device-side count
-  // exit at once; measured within 2048-8448 on the 300^2 step, whose times differ by their last
-  // partial round of blocks), or the autotuned size
-  const long long tuned = tune_value(SRF_TUNE_COLOR_DW_CHUNK);
-  c.chunk = tuned ? (int)tuned : 3840;
-  if (g.prec != SRF_PREC_F32) {
-    hipLaunchKernelGGL(color_dw_kernel, dim3(c.n_jobs * ((w.cols + c.chunk - 1) / c.chunk)), dim3(64 * kCdwWaves), 0,
-                       s, c);
-    return launch_status();
-  }
-  // FP32: the MLP's grouped FP32 GEMM on 128 x 160 tiles (one tile per job), whose fixed ring of
-  // four k-units in flight keeps its MFMA-bound blocks busy
-  mlp::DwArgs d;
-  memset(&d, 0, sizeof(d));
-  d.ldP = w.ld;
-  d.cols = w.cols;
-  d.cols_dev = point_count;
-  d.paired = 1;  // tile blocks (point-block-major, as the narrow tiling reads them)
-  d.n_jobs = c.n_jobs;
-  for (int i = 0; i < c.n_jobs; ++i) {
-    mlp::DwJob& jb = d.jobs[i];
-    const CdwJob& cj = c.jobs[i];
-    jb.dz = cj.dz;
-    jb.dz_rows = 16 * cj.nA;
-    jb.x = cj.x;
-    jb.x_rows = 16 * cj.nB;
-    jb.M = cj.M;
-    jb.N = cj.N;
-    jb.dw = cj.dw;
-    jb.ld_dw = cj.ld_dw;
-    jb.db = cj.db;
-    jb.mblocks = (cj.M + mlp::kDwNarrowRows - 1) / mlp::kDwNarrowRows;
-    jb.nblocks = (cj.N + mlp::kDwNarrowCols - 1) / mlp::kDwNarrowCols;
-  }
-  long long target = mlp::dw_default_chunk(w.cols, d.n_jobs, mlp::device_compute_units());
-  if (tuned) target = tuned;
-  d.chunk = (int)(target < 2048 ? 2048 : (target > 65536 ? 65536 : target));
-  d.n_chunks = (w.cols + d.chunk - 1) / d.chunk;
-  int work = 0;
-  for (int i = 0; i < d.n_jobs; ++i) {
-    d.jobs[i].work_begin = work;
-    d.jobs[i].work_count = d.jobs[i].mblocks * d.jobs[i].nblocks * d.n_chunks;
-    work += d.jobs[i].work_count;
-  }
-  d.total_work = work;
-  return mlp::dw_f32_narrow(d, s);
+  c.chunk = (int)tune_value(SRF_TUNE_COLOR_DW_CHUNK);  // the autotuned points of a block, or 0
+  c.cus = std::max(8, mlp::device_compute_units());
+  return cdw_launch(c, g.prec != SRF_PREC_F32, s);
 }

@@ -1161,8 +1161,7 @@ inline int device_compute_units() {
 struct DwArgs {
   DwJob jobs[kMaxJobs];
   int n_jobs, ldP, cols, chunk, n_chunks, total_work;
-  // dZ / X layout: 0 plain feature-major rows; 1 the paired tile blocks of store_tile (tile-major
-  // for the wide tilings, point-block-major for the narrow one; see mlp_dw_kernel)
+  // dZ / X layout: 0 plain feature-major rows; 1 the paired tile blocks of store_tile
   int paired;
   // optional device-side point count: only the columns below it, rounded up to whole 256-point
   // blocks, are reduced (the chunks past it exit); the columns up to that bound must hold finite
@@ -1190,21 +1189,12 @@ constexpr int kDwWaves = 8;
 constexpr int kDwFrags = 32;              // 16 dZ + 16 X fragments per k-unit
 constexpr int kDwSlot = kDwFrags * 1024;  // one k-unit
 constexpr int kDwSlots = 5;               // ring depth (prefetch distance kDwSlots - 1): 160 KB of LDS
-constexpr int kDwNarrowRows = 128, kDwNarrowCols = 160;  // tile of the RM = 1, NC = 10 wave tiling
 
 
-// Wave tiling: RM row tiles x NC column tiles per wave.  NC = 8: the waves split the tile into
-// four row groups x two column halves, RM = 4 giving 256 x 256 tiles (the NeRF layers) and RM = 2
-// 128 x 256 tiles.  RM = 1, NC = 10: wave w takes row tile w and column tiles 0..9 of a 128 x 160
-// tile, which keeps all eight waves (and all four SIMDs) busy on jobs of at most 128 rows and 160
-// columns (the TensoRF colour network), where the half-tile split left half of them idle.  The
-// DMA is the same for all (16 dZ and 16 X row tiles from m0 / n0).
-template <int P, int RM = 4, int NC = 8>
+template <int P>
 __global__ __launch_bounds__(64 * kDwWaves) void mlp_dw_kernel(DwArgs a) {
-  static_assert((NC == 8 && (RM == 4 || RM == 2)) || (RM == 1 && NC == 10), "supported wave tilings");
-  constexpr bool kRowWaves = NC != 8;
-  constexpr int kTM = kRowWaves ? 16 * kDwWaves : 64 * RM;  // tile rows
-  constexpr int kTN = kRowWaves ? 16 * NC : kDwTile;         // tile columns
+  constexpr int RM = 4, NC = 8;                       // row and column tiles of a wave
+  constexpr int kTM = 64 * RM, kTN = kDwTile;  // rows and columns of the tile
   __shared__ __attribute__((aligned(16))) uint8_t ring[kDwSlots * kDwSlot];
   const int lane = threadIdx.x & 63, g = lane >> 4, j = lane & 15;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1224,7 +1214,7 @@ __global__ __launch_bounds__(64 * kDwWaves) void mlp_dw_kernel(DwArgs a) {
   static_assert(P == kF32, "16-bit operands: mlp16_dw.h; split BF16: mlp_dw_split_kernel");
   constexpr int ELEM = 4;
   constexpr int KPTS = 16;  // points per k-unit
-  const int qm = kRowWaves ? w : RM * (w >> 1), qn = kRowWaves ? 0 : 8 * (w & 1);
+  const int qm = RM * (w >> 1), qn = NC * (w & 1);
   bool mv[RM], nv[NC];
 #pragma unroll
   for (int i = 0; i < RM; ++i) mv[i] = m0 + 16 * (qm + i) < jb.dz_rows;
@@ -1235,32 +1225,14 @@ __global__ __launch_bounds__(64 * kDwWaves) void mlp_dw_kernel(DwArgs a) {
   for (int i = 0; i < RM; ++i) any_m |= mv[i];
 #pragma unroll
   for (int k = 0; k < NC; ++k) any_n |= nv[k];
-  // valid row and column tiles of this wave (prefixes of the tile lists)
-  int nmv = 0, nnv = 0;
-#pragma unroll
-  for (int i = 0; i < RM; ++i) nmv += mv[i] ? 1 : 0;
-#pragma unroll
-  for (int k = 0; k < NC; ++k) nnv += nv[k] ? 1 : 0;
-  nmv = __builtin_amdgcn_readfirstlane(nmv);
-  nnv = __builtin_amdgcn_readfirstlane(nnv);
   // DMA of the 32 fragments of the k-unit at point p into a ring slot: fragment f < 16 is dZ row
   // tile f, f >= 16 is X row tile f - 16; wave w copies f = w, w + 8, w + 16, w + 24.  Every wave
   // issues exactly four loads per k-unit (a tile beyond the job's rows re-reads its first row
   // tile into the unused slot), so the vmcnt waits below count whole k-units.
-  // Narrow tiling: only the fragments the tile uses are copied, nA dZ row tiles and nB X row
-  // tiles (nA <= 8, nB <= 10), fragment f of the list going to wave f % 8; each wave waits for
-  // its own count (dma_n per k-unit).
-  const int nA = kRowWaves ? min(8, (jb.dz_rows - m0 + 15) / 16) : 16;
-  const int nB = kRowWaves ? min(NC, (jb.x_rows - n0 + 15) / 16) : 16;
-  const int dma_n = kRowWaves ? (nA + nB - w + kDwWaves - 1) / kDwWaves : 4;
   auto dma_unit = [&](int p, uint8_t* buf) SRF_AI {
 #pragma unroll
-    for (int q = 0; q < (kRowWaves ? 3 : 4); ++q) {
-      int f = w + kDwWaves * q;
-      if (kRowWaves) {
-        if (f >= nA + nB) break;
-        f = f < nA ? f : 16 + (f - nA);  // slot: dZ tile f or X tile 16 + k, as the MFMA loop reads
-      }
+    for (int q = 0; q < 4; ++q) {
+      const int f = w + kDwWaves * q;
       const bool is_a = f < 16;
       const int rt = is_a ? f : f - 16;
       int row0 = (is_a ? m0 : n0) + 16 * rt;
@@ -1273,12 +1245,8 @@ __global__ __launch_bounds__(64 * kDwWaves) void mlp_dw_kernel(DwArgs a) {
         constexpr int PPW = 32;  // points per stored wave block
         const int wb = p / PPW, u = (p % PPW) / KPTS;
         const int rec = 16 * (j >> 2) + 2 * (4 * u + g) + ((j >> 1) & 1);
-        // the wide tilings read tile-major blocks (tile t's blocks span 16 rows of ldP points, the MLP
-        // workspace); the narrow one point-block-major blocks (the array's tiles of one wave block
-        // adjacent, 2 KB each: the colour network's workspace)
-        size_t blk;
-        if constexpr (kRowWaves) blk = ((size_t)wb * ((is_a ? jb.dz_rows : jb.x_rows) / 16) + row0 / 16) * 2048;
-        else blk = (size_t)row0 * ldP * ELEM + (size_t)wb * 2048;
+        // tile-major blocks: tile t's blocks span 16 rows of ldP points
+        const size_t blk = (size_t)row0 * ldP * ELEM + (size_t)wb * 2048;
         src = base + blk + (j & 1) * 1024 + rec * 16;
       } else {
         src = base + (((size_t)(row0 + j)) * ldP + p + 4 * g) * ELEM;
@@ -1307,14 +1275,10 @@ __global__ __launch_bounds__(64 * kDwWaves) void mlp_dw_kernel(DwArgs a) {
     // k-unit u has landed once at most (issued after it) k-units' loads are outstanding
     const int after = min(kDwSlots - 2, n_units - 1 - u);
     static_assert(kDwSlots <= 5, "waits below cover up to three k-units in flight after u");
-    if constexpr (kRowWaves) {
-      wait_vmem_at_most(after * dma_n);  // at most 3 x 3
-    } else {
-      if (after >= 3) __builtin_amdgcn_s_waitcnt(vmcnt_only(12));
-      else if (after == 2) __builtin_amdgcn_s_waitcnt(vmcnt_only(8));
-      else if (after == 1) __builtin_amdgcn_s_waitcnt(vmcnt_only(4));
-      else __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
-    }
+    if (after >= 3) __builtin_amdgcn_s_waitcnt(vmcnt_only(12));
+    else if (after == 2) __builtin_amdgcn_s_waitcnt(vmcnt_only(8));
+    else if (after == 1) __builtin_amdgcn_s_waitcnt(vmcnt_only(4));
+    else __builtin_amdgcn_s_waitcnt(vmcnt_only(0));
     // After the barrier every wave's part of k-unit u is in LDS (each wave waited for its own
     // copies above) and slot (u - 1) % kDwSlots is free (each wave consumed its LDS reads of it
     // in the MFMAs of iteration u - 1).  A plain s_barrier with compiler-only memory barriers:
@@ -1327,34 +1291,20 @@ __global__ __launch_bounds__(64 * kDwWaves) void mlp_dw_kernel(DwArgs a) {
       dma_unit(pb + (u + kDwSlots - 1) * KPTS, ring + ((u + kDwSlots - 1) % kDwSlots) * kDwSlot);
     if (busy) {
       const uint8_t* fr = ring + (u % kDwSlots) * kDwSlot;
-      // No branch between the MFMAs (a branch after every FP32 MFMA doubled the products' time).
-      // Narrow tiling: the valid row and column tiles are prefixes (nmv, nnv, uniform over the
-      // wave), so the products run as one unguarded block per count of valid columns, chosen once
-      // per k-unit.  Wide tilings: every tile's product runs (a tile past the job's rows multiplies
-      // the re-read first row tile; the epilogue stores only the valid tiles), since a second,
-      // unguarded copy of their products spills.
+      // No branch between the MFMAs (a branch after every FP32 MFMA doubled the products' time): every
+      // tile's product runs (a tile past the job's rows multiplies the re-read first row tile; the
+      // epilogue stores only the valid tiles), since a second, guarded copy of the products spills.
       f32x4 av[RM], bv[NC];
 #pragma unroll
       for (int i = 0; i < RM; ++i) av[i] = *reinterpret_cast<const f32x4*>(fr + (qm + i) * 1024 + lane * 16);
 #pragma unroll
       for (int k = 0; k < NC; ++k) bv[k] = *reinterpret_cast<const f32x4*>(fr + (16 + qn + k) * 1024 + lane * 16);
-      auto prod = [&](auto NRI, auto NVI) SRF_AI {
-        constexpr int NR = decltype(NRI)::value, NV = decltype(NVI)::value;
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
+      for (int q = 0; q < 4; ++q)
 #pragma unroll
-          for (int i = 0; i < NR; ++i)
+        for (int i = 0; i < RM; ++i)
 #pragma unroll
-            for (int k = 0; k < NV; ++k) acc[i][k] = mfma32(av[i][q], bv[k][q], acc[i][k]);
-      };
-      if constexpr (kRowWaves) {
-        if (nmv == RM)
-          static_for<1, NC + 1>([&](auto VI) SRF_AI {
-            if (nnv == decltype(VI)::value) prod(std::integral_constant<int, RM>{}, VI);
-          });
-      } else {
-        prod(std::integral_constant<int, RM>{}, std::integral_constant<int, NC>{});
-      }
+          for (int k = 0; k < NC; ++k) acc[i][k] = mfma32(av[i][q], bv[k][q], acc[i][k]);
       if (do_db)
 #pragma unroll
         for (int i = 0; i < RM; ++i) rs[i] += (av[i][0] + av[i][1]) + (av[i][2] + av[i][3]);
@@ -1545,9 +1495,9 @@ int launch_bwd(const BwdArgs& a, hipStream_t s) {
   return launch_status();
 }
 
-template <int P, int RM = 4, int NC = 8>
+template <int P>
 int launch_dw(const DwArgs& d, hipStream_t s) {
-  hipLaunchKernelGGL((mlp_dw_kernel<P, RM, NC>), dim3(d.total_work), dim3(64 * kDwWaves), 0, s, d);
+  hipLaunchKernelGGL(mlp_dw_kernel<P>, dim3(d.total_work), dim3(64 * kDwWaves), 0, s, d);
   return launch_status();
 }
 
@@ -1562,7 +1512,6 @@ int fwd_f16(const FwdArgs& a, bool vd, bool tr, hipStream_t s);
 int bwd_f32(const BwdArgs& a, bool vd, hipStream_t s);
 int bwd_bf16(const BwdArgs& a, bool vd, hipStream_t s);
 int dw_f32(const DwArgs& d, hipStream_t s);
-int dw_f32_narrow(const DwArgs& d, hipStream_t s);  // 128 x 160 tiles (kDwNarrowRows x kDwNarrowCols)
 int fwd_bf16s(const FwdArgs& a, bool vd, bool tr, hipStream_t s);  // split BF16 (mlp_bf16s.hip)
 int bwd_bf16s(const BwdArgs& a, bool vd, hipStream_t s);
 int dw_bf16s(const DwArgs& d, hipStream_t s);  // mlp_dw_split_kernel
