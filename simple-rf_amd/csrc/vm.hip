@@ -13,10 +13,13 @@
 // axis innermost).  A bilinear tap then reads c_p contiguous floats.
 //
 // Mapping.  The channels of the three planes are cut into 4-channel quads (c_p % 4 == 0) and
-// concatenated, Q quads in all.  A group of G lanes (G = next power of two >= Q) owns one
-// sample; lane j of the group handles quads j, j + G, ...  Every tap of a group is thus one
-// contiguous 16 B x (quads of that plane) read, appearance rows are written as coalesced
-// 16 B stores, and the density sum over channels is a butterfly inside the group.
+// concatenated, Q quads in all.
+//   Forward: a wave owns 64 samples.  Each lane prepares one (validity, cell, weights, into LDS),
+//   then groups of G = 4 or 8 lanes read the factors of the prepared samples, lane j of a group the
+//   quads j, j + G, ...: a tap of a group is one contiguous 16 B x G read, appearance rows are
+//   written as 16 B stores, and the density sum over channels is a butterfly inside the group.
+//   Backward: a group of lanes owns a run of samples, lane j the quads j, j + G, ... (G = next power
+//   of two >= Q).
 //
 // Arithmetic follows grid_sample's op order: source index ((x + 1) / 2) * (size - 1), corner
 // weights as products of the opposite distances, taps accumulated nw, ne, sw, se; the file is
@@ -157,19 +160,149 @@ __device__ __forceinline__ QuadSite quad_site(const VmArgs& a, int q, const floa
   return s;
 }
 
+// Sum of the taps v of weights w; a tap that is not ok adds nothing (whatever its value and weight).  The
+// loads come before (a branch per tap would serialise them); a wave without a corner outside the factor,
+// as all samples inside the box are, takes no select.
+template <int N>
+__device__ __forceinline__ float4 tap_sum(const float4 (&v)[N], const float (&w)[N], bool clean, const bool (&ok)[N]) {
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (__ballot(!clean) == 0) {
+#pragma unroll
+    for (int t = 0; t < N; ++t) s = madd4(s, v[t], w[t]);
+  } else {
+#pragma unroll
+    for (int t = 0; t < N; ++t) {
+      const float4 n = madd4(s, v[t], w[t]);
+      s = make_float4(ok[t] ? n.x : s.x, ok[t] ? n.y : s.y, ok[t] ? n.z : s.z, ok[t] ? n.w : s.w);
+    }
+  }
+  return s;
+}
+
 // Bilinear plane value and linear line value of the 4 components of a quad.
 __device__ __forceinline__ void quad_values(const VmArgs& a, const QuadSite& s, float4& pv, float4& lv) {
   const int C = sel3(s.p, a.comp[0], a.comp[1], a.comp[2]);
   const float* P = sel3(s.p, a.plane[0], a.plane[1], a.plane[2]);
   const float* L = sel3(s.p, a.line[0], a.line[1], a.line[2]);
-  pv = make_float4(0.f, 0.f, 0.f, 0.f);
+  float4 v[4], l[2];
+  bool ok[4], okl[2];
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
-    if (s.pt.idx[t] >= 0) pv = madd4(pv, ld4(P + (int64_t)s.pt.idx[t] * C + s.c), s.pt.w[t]);
-  lv = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int t = 0; t < 4; ++t) {
+    ok[t] = s.pt.idx[t] >= 0;
+    v[t] = ld4(P + (int64_t)max(s.pt.idx[t], 0) * C + s.c);
+  }
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
-    if (s.lt.idx[t] >= 0) lv = madd4(lv, ld4(L + (int64_t)s.lt.idx[t] * C + s.c), s.lt.w[t]);
+  for (int t = 0; t < 2; ++t) {
+    okl[t] = s.lt.idx[t] >= 0;
+    l[t] = ld4(L + (int64_t)max(s.lt.idx[t], 0) * C + s.c);
+  }
+  const bool clean = ok[0] && ok[1] && ok[2] && ok[3] && okl[0] && okl[1];
+  pv = tap_sum(v, s.pt.w, clean, ok);
+  lv = tap_sum(l, s.lt.w, clean, okl);
+}
+
+// ----- prepared sites of the forward kernels
+// Plane p's cell and line interval of one sample, as a lane of the wave prepares them for the groups: the
+// fractions of the coordinates within their cells (the weight of the upper corner; the lower one's is
+// 1 - f, the same number as x1 - x for every size that FP32 coordinates resolve), the first corner inside
+// the factor and which corners are (kTap bits: nw, ne, sw, se, lower, upper; kDx, kDy, kDl: the second
+// corner of the axis is another texel).
+constexpr int kTapAll = 63, kDx = 64, kDy = 128, kDl = 256;
+
+struct WaveSites {
+  float4 frac[kPlanes][SRF_WAVE];  // fx, fy, fl, flags
+  int2 at[kPlanes][SRF_WAVE];      // texel of the plane, of the line
+};
+
+__device__ __forceinline__ void prepare_sites(const VmArgs& a, const float pn[3], WaveSites& ws, int slot) {
+  auto axis = [](float x, int size, float& f, int& first, int& in) {
+    const float ix = source_index(x, size);
+    const float x0 = floorf(ix);
+    f = __fsub_rn(ix, x0);
+    const int xi = (int)x0;
+    const bool in0 = xi >= 0 && xi < size, in1 = xi + 1 >= 0 && xi + 1 < size;
+    first = in0 ? xi : (in1 ? xi + 1 : 0);
+    in = (in0 ? 1 : 0) | (in1 ? 2 : 0);
+  };
+#pragma unroll
+  for (int p = 0; p < kPlanes; ++p) {
+    if (a.comp[p] == 0) continue;  // uniform
+    float4 fr;
+    int xc, yc, lc, xin, yin, lin;
+    axis(pn[axis_a0(p)], a.pw[p], fr.x, xc, xin);
+    axis(pn[axis_a1(p)], a.ph[p], fr.y, yc, yin);
+    axis(pn[axis_v(p)], a.ll[p], fr.z, lc, lin);
+    const int flags = ((yin & 1) ? xin : 0) | ((yin & 2) ? xin << 2 : 0) | (lin << 4) | (xin == 3 ? kDx : 0) |
+                      (yin == 3 ? kDy : 0) | (lin == 3 ? kDl : 0);
+    fr.w = __int_as_float(flags);
+    ws.frac[p][slot] = fr;
+    ws.at[p][slot] = make_int2(yc * a.pw[p] + xc, lc);
+  }
+}
+
+// LDS written by lanes of this wave is read by others of it: LDS operations of a wave are performed in
+// order, so only the compiler has to keep them so.
+__device__ __forceinline__ void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
+
+// Products plane x line of the quads q0, q0 + G, ... (T of them, clamped to the last) of the site in `slot`,
+// with all 6 T loads in flight at once.  kUniform: a step's quads lie in one plane.
+template <int G, int T, bool kUniform>
+__device__ __forceinline__ void quad_products(const VmArgs& a, const WaveSites& ws, int slot, int q0, float4 (&out)[T],
+                                              int (&pl)[T]) {
+  float4 v[T][4], l[T][2], fr[T];
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+    const int q = kUniform ? q0 + G * t : min(q0 + G * t, a.n_quads - 1);
+    const int p = kUniform ? __builtin_amdgcn_readfirstlane(quad_plane(a, q)) : quad_plane(a, q);
+    pl[t] = p;
+    const int c = 4 * (q - sel3(p, a.qoff[0], a.qoff[1], a.qoff[2]));
+    const int C = sel3(p, a.comp[0], a.comp[1], a.comp[2]);
+    const int64_t row = (int64_t)sel3(p, a.pw[0], a.pw[1], a.pw[2]) * C;
+    fr[t] = ws.frac[p][slot];
+    const int2 at = ws.at[p][slot];
+    const int flags = __float_as_int(fr[t].w);
+    const float* P = sel3(p, a.plane[0], a.plane[1], a.plane[2]) + (int64_t)at.x * C + c;
+    const float* L = sel3(p, a.line[0], a.line[1], a.line[2]) + (int64_t)at.y * C + c;
+    const int dx = (flags & kDx) ? C : 0, dl = (flags & kDl) ? C : 0;
+    const float* P1 = P + ((flags & kDy) ? row : 0);
+    v[t][0] = ld4(P);
+    v[t][1] = ld4(P + dx);
+    v[t][2] = ld4(P1);
+    v[t][3] = ld4(P1 + dx);
+    l[t][0] = ld4(L);
+    l[t][1] = ld4(L + dl);
+  }
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+    const int flags = __float_as_int(fr[t].w);
+    const float x1 = fr[t].x, x0 = __fsub_rn(1.0f, x1), y1 = fr[t].y, y0 = __fsub_rn(1.0f, y1);
+    const float w[4] = {__fmul_rn(x0, y0), __fmul_rn(x1, y0), __fmul_rn(x0, y1), __fmul_rn(x1, y1)};
+    const float wl[2] = {__fsub_rn(1.0f, fr[t].z), fr[t].z};
+    const bool ok[4] = {(flags & 1) != 0, (flags & 2) != 0, (flags & 4) != 0, (flags & 8) != 0};
+    const bool okl[2] = {(flags & 16) != 0, (flags & 32) != 0};
+    const bool clean = (flags & kTapAll) == kTapAll;
+    out[t] = mul4(tap_sum(v[t], w, clean, ok), tap_sum(l[t], wl, clean, okl));
+  }
+}
+
+// f(products, planes, first step) over all steps of a group, three at a time while there are that many.
+template <int G, bool kUniform, typename F>
+__device__ __forceinline__ void for_quads(const VmArgs& a, const WaveSites& ws, int slot, int ql, F&& f) {
+  const int steps = (a.n_quads + G - 1) / G;
+  int st = 0;
+  for (; st + 3 <= steps; st += 3) {
+    float4 o[3];
+    int pl[3];
+    quad_products<G, 3, kUniform>(a, ws, slot, ql + G * st, o, pl);
+#pragma unroll
+    for (int t = 0; t < 3; ++t) f(o[t], pl[t], ql + G * (st + t));
+  }
+  for (; st < steps; ++st) {
+    float4 o[1];
+    int pl[1];
+    quad_products<G, 1, kUniform>(a, ws, slot, ql + G * st, o, pl);
+    f(o[0], pl[0], ql + G * st);
+  }
 }
 
 // Trilinear grid_sample of the alpha volume (align_corners=True, zero padding); corners
@@ -185,19 +318,21 @@ __device__ float alpha_value(const AlphaArgs& m, const float p[3]) {
   const float wy[2] = {__fsub_rn(y1, iy), __fsub_rn(iy, y0)};
   const float wz[2] = {__fsub_rn(z1, iz), __fsub_rn(iz, z0)};
   const int xi = (int)x0, yi = (int)y0, zi = (int)z0;
+  // all eight loads before the sum (a branch per corner would serialise them); a corner outside adds nothing
+  float v[8];
+  bool ok[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const int X = xi + (k & 1), Y = yi + ((k >> 1) & 1), Z = zi + (k >> 2);
+    ok[k] = X >= 0 && X < m.w && Y >= 0 && Y < m.h && Z >= 0 && Z < m.d;
+    v[k] = m.vol[ok[k] ? ((int64_t)Z * m.h + Y) * m.w + X : 0];
+  }
   float out = 0.f;
 #pragma unroll
-  for (int dz = 0; dz < 2; ++dz)
-#pragma unroll
-    for (int dy = 0; dy < 2; ++dy)
-#pragma unroll
-      for (int dx = 0; dx < 2; ++dx) {
-        const int X = xi + dx, Y = yi + dy, Z = zi + dz;
-        if (X >= 0 && X < m.w && Y >= 0 && Y < m.h && Z >= 0 && Z < m.d) {
-          const float w = __fmul_rn(__fmul_rn(wx[dx], wy[dy]), wz[dz]);
-          out = __fadd_rn(out, __fmul_rn(m.vol[((int64_t)Z * m.h + Y) * m.w + X], w));
-        }
-      }
+  for (int k = 0; k < 8; ++k) {
+    const float w = __fmul_rn(__fmul_rn(wx[k & 1], wy[(k >> 1) & 1]), wz[k >> 2]);
+    out = ok[k] ? __fadd_rn(out, __fmul_rn(v[k], w)) : out;
+  }
   return out;
 }
 
@@ -247,41 +382,59 @@ __device__ __forceinline__ GroupPos group_pos() {
 
 // --------------------------------------------------------------------------- kernels
 
-template <int G>
+// What bounded the forwards was the vector ALU: every lane of a group of 16 (or 64) repeated the sample's
+// divisions, its eight-voxel alpha test and the cells of its quad, a quarter (or nearly half) of the lanes
+// had no quad, and a branch per tap put its six loads one after the other.  Now a lane prepares one sample,
+// only the valid ones are packed for the groups, and a group is small enough that its lanes have several
+// quads (with G = 4 in the equal configurations all lanes work).  3.6M samples of 3 x 16 components under an
+// alpha mask: 658 -> 164 us; 1.45M rows of 3 x 48: 707 -> 372 us (of which 835 MB of rows written).
+constexpr int kFwdWaves = 256 / SRF_WAVE;
+
+template <int G, bool kUniform>
 __global__ __launch_bounds__(256) void density_fwd_kernel(VmArgs a, AlphaArgs m, int64_t n,
                                                           const float* __restrict__ pts, int kind,
                                                           float offset, float* __restrict__ sigma,
                                                           float* __restrict__ feat_out,
                                                           uint8_t* __restrict__ valid_out) {
-  const GroupPos gp = group_pos<G>();
-  // all lanes of a group share i, so the group stays converged for its butterfly
-  for (int64_t i = gp.first; i < n; i += gp.stride) {
+  __shared__ WaveSites sites[kFwdWaves];
+  __shared__ float feats[kFwdWaves][SRF_WAVE];
+  const int lane = threadIdx.x & (SRF_WAVE - 1), wv = threadIdx.x / SRF_WAVE;
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t base = (int64_t)blockIdx.x * blockDim.x + wv * SRF_WAVE; base < n; base += stride) {
+    const int64_t i = base + lane < n ? base + lane : n - 1;
     const float p[3] = {pts[3 * i + 0], pts[3 * i + 1], pts[3 * i + 2]};
-    bool valid = in_box(p, a.lo, a.hi);
+    bool valid = base + lane < n && in_box(p, a.lo, a.hi);
     if (valid && m.vol) valid = alpha_value(m, p) > 0.f;
-    float pn[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) pn[k] = normalize_coord(p[k], a.lo[k], a.size[k]);
-    float s[kPlanes] = {0.f, 0.f, 0.f};
+    const uint64_t mask = __ballot(valid);
+    const int count = __popcll(mask), rank = __popcll(mask & ((1ull << lane) - 1ull));
     if (valid) {
-      for (int q = gp.ql; q < a.n_quads; q += G) {
-        const QuadSite site = quad_site(a, q, pn);
-        float4 pv, lv;
-        quad_values(a, site, pv, lv);
-        const float d = sum4(mul4(pv, lv));
-        s[0] = site.p == 0 ? __fadd_rn(s[0], d) : s[0];
-        s[1] = site.p == 1 ? __fadd_rn(s[1], d) : s[1];
-        s[2] = site.p == 2 ? __fadd_rn(s[2], d) : s[2];
-      }
-    }
+      float pn[3];
 #pragma unroll
-    for (int k = 0; k < kPlanes; ++k) s[k] = group_sum<G>(s[k]);
-    if (gp.ql == 0) {
-      const float f = __fadd_rn(__fadd_rn(s[0], s[1]), s[2]);
+      for (int k = 0; k < 3; ++k) pn[k] = normalize_coord(p[k], a.lo[k], a.size[k]);
+      prepare_sites(a, pn, sites[wv], rank);
+    }
+    wave_lds_fence();
+    for (int k0 = 0; k0 < count; k0 += SRF_WAVE / G) {  // uniform: whole groups stay converged
+      const int k = k0 + lane / G;
+      float s[kPlanes] = {0.f, 0.f, 0.f};
+      for_quads<G, kUniform>(a, sites[wv], min(k, count - 1), lane % G, [&](float4 v, int pl, int q) {
+        const float d = kUniform || q < a.n_quads ? sum4(v) : 0.f;
+        s[0] = pl == 0 ? __fadd_rn(s[0], d) : s[0];
+        s[1] = pl == 1 ? __fadd_rn(s[1], d) : s[1];
+        s[2] = pl == 2 ? __fadd_rn(s[2], d) : s[2];
+      });
+#pragma unroll
+      for (int q = 0; q < kPlanes; ++q) s[q] = group_sum<G>(s[q]);
+      if (lane % G == 0 && k < count) feats[wv][k] = __fadd_rn(__fadd_rn(s[0], s[1]), s[2]);
+    }
+    wave_lds_fence();
+    if (base + lane < n) {
+      const float f = valid ? feats[wv][rank] : 0.f;
       sigma[i] = valid ? predict_density(f, kind, offset) : 0.f;
-      if (feat_out) feat_out[i] = valid ? f : 0.f;
+      if (feat_out) feat_out[i] = f;
       if (valid_out) valid_out[i] = valid ? 1 : 0;
     }
+    wave_lds_fence();
   }
 }
 
@@ -459,24 +612,33 @@ __global__ __launch_bounds__(256) void density_bwd_kernel(VmArgs a, int64_t n, i
 
 // Appearance features of the listed samples: out[j, c] = plane_c * line_c for the sample
 // idx[j] (or j when idx is null), components concatenated over the planes.
-template <int G>
+template <int G, bool kUniform>
 __global__ __launch_bounds__(256) void appearance_fwd_kernel(VmArgs a, int64_t n, const int32_t* __restrict__ n_dev,
                                                              const int32_t* __restrict__ idx,
                                                              const float* __restrict__ pts,
                                                              float* __restrict__ out) {
-  const GroupPos gp = group_pos<G>();
+  __shared__ WaveSites sites[kFwdWaves];
+  const int lane = threadIdx.x & (SRF_WAVE - 1), wv = threadIdx.x / SRF_WAVE;
   if (n_dev) n = min(n, (int64_t)*n_dev);  // device-side row count (n is the capacity)
-  for (int64_t j = gp.first; j < n; j += gp.stride) {
-    const int64_t i = idx ? (int64_t)idx[j] : j;
-    float pn[3];
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t base = (int64_t)blockIdx.x * blockDim.x + wv * SRF_WAVE; base < n; base += stride) {
+    const int count = (int)min((int64_t)SRF_WAVE, n - base);
+    if (lane < count) {
+      const int64_t i = idx ? (int64_t)idx[base + lane] : base + lane;
+      float pn[3];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) pn[k] = normalize_coord(pts[3 * i + k], a.lo[k], a.size[k]);
-    for (int q = gp.ql; q < a.n_quads; q += G) {
-      const QuadSite site = quad_site(a, q, pn);
-      float4 pv, lv;
-      quad_values(a, site, pv, lv);
-      *reinterpret_cast<float4*>(out + j * a.total_comp + 4 * q) = mul4(pv, lv);
+      for (int k = 0; k < 3; ++k) pn[k] = normalize_coord(pts[3 * i + k], a.lo[k], a.size[k]);
+      prepare_sites(a, pn, sites[wv], lane);
     }
+    wave_lds_fence();
+    for (int k0 = 0; k0 < count; k0 += SRF_WAVE / G) {
+      const int k = k0 + lane / G;
+      for_quads<G, kUniform>(a, sites[wv], min(k, count - 1), lane % G, [&](float4 v, int, int q) {
+        if (k < count && (kUniform || q < a.n_quads))
+          *reinterpret_cast<float4*>(out + (base + k) * a.total_comp + 4 * q) = v;
+      });
+    }
+    wave_lds_fence();
   }
 }
 
@@ -1184,6 +1346,16 @@ int run_length() {
     default: hipLaunchKernelGGL(KERNEL<64>, __VA_ARGS__); break;                          \
   }
 
+// Forward groups: 4 lanes where every plane's quads are a multiple of 4 (a step's quads then lie in one plane
+// and no lane idles), else 4 or 8 lanes, whichever leaves fewer lanes without a quad (8 at a tie: fewer steps).
+#define SRF_VM_FWD_DISPATCH(A_, KERNEL, ...)                                                       \
+  if ((A_).comp[0] % 16 == 0 && (A_).comp[1] % 16 == 0 && (A_).comp[2] % 16 == 0)                  \
+    hipLaunchKernelGGL((KERNEL<4, true>), __VA_ARGS__);                                            \
+  else if (((A_).n_quads + 3) / 4 * 4 < ((A_).n_quads + 7) / 8 * 8)                                \
+    hipLaunchKernelGGL((KERNEL<4, false>), __VA_ARGS__);                                           \
+  else                                                                                             \
+    hipLaunchKernelGGL((KERNEL<8, false>), __VA_ARGS__);
+
 #define SRF_VM_DISPATCH_KD(G_, KD, KERNEL, ...)                                            \
   switch (G_) {                                                                           \
     case 1: hipLaunchKernelGGL((KERNEL<1, KD>), __VA_ARGS__); break;                      \
@@ -1327,9 +1499,8 @@ extern "C" int srf_vm_density_fwd(const srf_vm_factors* factors, const float* bb
   AlphaArgs m;
   if ((st = make_alpha_args(alpha, &m)) != SRF_OK) return st;
   if (!pts || !sigma) return SRF_EINVAL;
-  const int G = next_pow2(a.n_quads);
-  SRF_VM_DISPATCH(G, density_fwd_kernel, dim3(grid_for(n_points, G)), dim3(256), 0, as_stream(stream), a, m,
-                  n_points, pts, predictor, offset, sigma, feat, valid);
+  SRF_VM_FWD_DISPATCH(a, density_fwd_kernel, dim3(grid_for(n_points, 1)), dim3(256), 0, as_stream(stream), a, m,
+                      n_points, pts, predictor, offset, sigma, feat, valid);
   return launch_status();
 }
 
@@ -1385,9 +1556,8 @@ extern "C" int srf_vm_appearance_fwd(const srf_vm_factors* factors, const float*
   int st = make_vm_args(factors, bbox, &a, true);
   if (st != SRF_OK) return st;
   if (!pts || !features) return SRF_EINVAL;
-  const int G = next_pow2(a.n_quads);
-  SRF_VM_DISPATCH(G, appearance_fwd_kernel, dim3(grid_for(n_rows, G)), dim3(256), 0, as_stream(stream), a,
-                  n_rows, row_count, idx, pts, features);
+  SRF_VM_FWD_DISPATCH(a, appearance_fwd_kernel, dim3(grid_for(n_rows, 1)), dim3(256), 0, as_stream(stream), a,
+                      n_rows, row_count, idx, pts, features);
   return launch_status();
 }
 
