@@ -287,7 +287,7 @@ size_t srf_vm_bwd_workspace_bytes(const srf_vm_factors* factors, int64_t n_rows)
  * first).  Coordinates carry no gradient (the reference detaches them, :1224-1228) -- the
  * scatter of grid_sample's backward.  With a workspace (srf_vm_bwd_workspace_bytes) the
  * contributing samples are first ordered by plane cell, so that each texel is flushed about once
- * per run of samples and the line gradients are summed in LDS; workspace NULL walks the samples in
+ * per run of samples and a line texel about once per block; workspace NULL walks the samples in
  * their own order (more atomics).  Both give the same sums up to the order of FP32 additions. */
 int srf_vm_density_bwd(const srf_vm_factors* factors, float* const* d_planes,
                        float* const* d_lines, const float* bbox, int64_t n_points,

@@ -890,6 +890,6 @@ extern "C" int srf_color_backward(const srf_color_desc* desc, const void* packed
   c.cols = w.cols;
   c.cols_dev = point_count;
   c.chunk = (int)tune_value(SRF_TUNE_COLOR_DW_CHUNK);  // the autotuned points of a block, or 0
-  c.cus = std::max(8, mlp::device_compute_units());
+  c.cus = std::max(8, device_compute_units());
   return cdw_launch(c, g.prec != SRF_PREC_F32, s);
 }

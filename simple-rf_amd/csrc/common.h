@@ -81,4 +81,13 @@ __device__ __forceinline__ float torch_norm3(float x, float y, float z) {
   return sqrtf(fmaf(z, z, fmaf(y, y, __fmul_rn(x, x))));
 }
 
+// Compute units of the current device (launch schedules; 256 if the query fails).
+inline int device_compute_units() {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    return 256;
+  return cus;
+}
+
 }  // namespace srf

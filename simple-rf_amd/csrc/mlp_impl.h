@@ -1148,16 +1148,6 @@ inline int dw_default_chunk(int cols, int nj, int cus) {
   return best;
 }
 
-// Compute units of the current device (the launch-schedule heuristics above; 256 if the query
-// fails).
-inline int device_compute_units() {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    return 256;
-  return cus;
-}
-
 struct DwArgs {
   DwJob jobs[kMaxJobs];
   int n_jobs, ldP, cols, chunk, n_chunks, total_work;

@@ -26,6 +26,7 @@
 // compiled with -ffp-contract=off so no product is fused into a sum.
 #include <string.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "common.h"
@@ -148,16 +149,21 @@ struct QuadSite {
   LineTaps lt;
 };
 
-__device__ __forceinline__ QuadSite quad_site(const VmArgs& a, int q, const float pn[3]) {
+__device__ __forceinline__ QuadSite quad_site(const VmArgs& a, int p, int c, const float pn[3]) {
   QuadSite s;
-  s.p = quad_plane(a, q);
-  s.c = 4 * (q - sel3(s.p, a.qoff[0], a.qoff[1], a.qoff[2]));
+  s.p = p;
+  s.c = c;
   const float x = sel3(s.p, pn[axis_a0(0)], pn[axis_a0(1)], pn[axis_a0(2)]);
   const float y = sel3(s.p, pn[axis_a1(0)], pn[axis_a1(1)], pn[axis_a1(2)]);
   const float v = sel3(s.p, pn[axis_v(0)], pn[axis_v(1)], pn[axis_v(2)]);
   s.pt = plane_taps(x, y, sel3(s.p, a.pw[0], a.pw[1], a.pw[2]), sel3(s.p, a.ph[0], a.ph[1], a.ph[2]));
   s.lt = line_taps(v, sel3(s.p, a.ll[0], a.ll[1], a.ll[2]));
   return s;
+}
+
+__device__ __forceinline__ QuadSite quad_site(const VmArgs& a, int q, const float pn[3]) {
+  const int p = quad_plane(a, q);
+  return quad_site(a, p, 4 * (q - sel3(p, a.qoff[0], a.qoff[1], a.qoff[2])), pn);
 }
 
 // Sum of the taps v of weights w; a tap that is not ok adds nothing (whatever its value and weight).  The
@@ -214,7 +220,7 @@ struct WaveSites {
   int2 at[kPlanes][SRF_WAVE];      // texel of the plane, of the line
 };
 
-__device__ __forceinline__ void prepare_sites(const VmArgs& a, const float pn[3], WaveSites& ws, int slot) {
+__device__ __forceinline__ void prepare_site(const VmArgs& a, int p, const float pn[3], float4& frac, int2& at) {
   auto axis = [](float x, int size, float& f, int& first, int& in) {
     const float ix = source_index(x, size);
     const float x0 = floorf(ix);
@@ -224,19 +230,25 @@ __device__ __forceinline__ void prepare_sites(const VmArgs& a, const float pn[3]
     first = in0 ? xi : (in1 ? xi + 1 : 0);
     in = (in0 ? 1 : 0) | (in1 ? 2 : 0);
   };
+  int xc, yc, lc, xin, yin, lin;
+  axis(pn[axis_a0(p)], a.pw[p], frac.x, xc, xin);
+  axis(pn[axis_a1(p)], a.ph[p], frac.y, yc, yin);
+  axis(pn[axis_v(p)], a.ll[p], frac.z, lc, lin);
+  const int flags = ((yin & 1) ? xin : 0) | ((yin & 2) ? xin << 2 : 0) | (lin << 4) | (xin == 3 ? kDx : 0) |
+                    (yin == 3 ? kDy : 0) | (lin == 3 ? kDl : 0);
+  frac.w = __int_as_float(flags);
+  at = make_int2(yc * a.pw[p] + xc, lc);
+}
+
+__device__ __forceinline__ void prepare_sites(const VmArgs& a, const float pn[3], WaveSites& ws, int slot) {
 #pragma unroll
   for (int p = 0; p < kPlanes; ++p) {
     if (a.comp[p] == 0) continue;  // uniform
-    float4 fr;
-    int xc, yc, lc, xin, yin, lin;
-    axis(pn[axis_a0(p)], a.pw[p], fr.x, xc, xin);
-    axis(pn[axis_a1(p)], a.ph[p], fr.y, yc, yin);
-    axis(pn[axis_v(p)], a.ll[p], fr.z, lc, lin);
-    const int flags = ((yin & 1) ? xin : 0) | ((yin & 2) ? xin << 2 : 0) | (lin << 4) | (xin == 3 ? kDx : 0) |
-                      (yin == 3 ? kDy : 0) | (lin == 3 ? kDl : 0);
-    fr.w = __int_as_float(flags);
-    ws.frac[p][slot] = fr;
-    ws.at[p][slot] = make_int2(yc * a.pw[p] + xc, lc);
+    float4 frac;
+    int2 at;
+    prepare_site(a, p, pn, frac, at);
+    ws.frac[p][slot] = frac;
+    ws.at[p][slot] = at;
   }
 }
 
@@ -444,21 +456,26 @@ __global__ __launch_bounds__(256) void density_fwd_kernel(VmArgs a, AlphaArgs m,
 // most contended texels drop by up to the run length.
 constexpr int kRun = 32;  // samples walked by one lane group (SRF_TUNE_GATHER_RUN overrides it)
 
+// T quads of one lane share the corners; quad t's components start at c[t] and it counts if on[t].
+template <int T>
 struct RunAcc {
   int pidx[4], lidx[2];
-  float4 pg[4], lg[2];
+  float4 pg[4][T], lg[2][T];
 };
 
-__device__ __forceinline__ void run_init(RunAcc& r) {
+template <int T>
+__device__ __forceinline__ void run_init(RunAcc<T>& r) {
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    r.pidx[t] = -1;
-    r.pg[t] = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int k = 0; k < 4; ++k) {
+    r.pidx[k] = -1;
+#pragma unroll
+    for (int t = 0; t < T; ++t) r.pg[k][t] = make_float4(0.f, 0.f, 0.f, 0.f);
   }
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    r.lidx[t] = -1;
-    r.lg[t] = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int k = 0; k < 2; ++k) {
+    r.lidx[k] = -1;
+#pragma unroll
+    for (int t = 0; t < T; ++t) r.lg[k][t] = make_float4(0.f, 0.f, 0.f, 0.f);
   }
 }
 
@@ -469,26 +486,6 @@ __device__ __forceinline__ void atomic_add4v(float* p, float4 v) {
   unsafeAtomicAdd(p + 3, v.w);
 }
 
-__device__ __forceinline__ void run_flush_plane(const VmArgs& a, int p, int c, RunAcc& r) {
-  const int C = sel3(p, a.comp[0], a.comp[1], a.comp[2]);
-  float* dP = sel3(p, a.dplane[0], a.dplane[1], a.dplane[2]);
-#pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    if (r.pidx[t] >= 0) atomic_add4v(dP + (int64_t)r.pidx[t] * C + c, r.pg[t]);
-    r.pg[t] = make_float4(0.f, 0.f, 0.f, 0.f);
-  }
-}
-
-__device__ __forceinline__ void run_flush_line(const VmArgs& a, int p, int c, RunAcc& r) {
-  const int C = sel3(p, a.comp[0], a.comp[1], a.comp[2]);
-  float* dL = sel3(p, a.dline[0], a.dline[1], a.dline[2]);
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    if (r.lidx[t] >= 0) atomic_add4v(dL + (int64_t)r.lidx[t] * C + c, r.lg[t]);
-    r.lg[t] = make_float4(0.f, 0.f, 0.f, 0.f);
-  }
-}
-
 // Per-corner run accumulation.  Slot k keeps corner role k (plane: nw, ne, sw, se; line: lower,
 // upper), so a sample whose cell is the previous one moved by one texel along an axis carries
 // the shared half of the slots over (the texel row or column both cells touch) and flushes only
@@ -496,81 +493,104 @@ __device__ __forceinline__ void run_flush_line(const VmArgs& a, int p, int c, Ru
 // A slot is carried only when its texel index equals the new corner's, so any move is handled
 // correctly (unmatched slots are flushed); index -1 marks a corner outside the factor, whose
 // slot is never flushed.  Static selects only: the slots stay in registers.
-__device__ __forceinline__ void flush_slot(float* grad, int idx, float4 acc, int C, int c) {
-  if (idx >= 0) atomic_add4v(grad + (int64_t)idx * C + c, acc);
+template <int T>
+__device__ __forceinline__ void flush_slot(float* grad, int idx, const float4 (&acc)[T], int C, const int (&c)[T],
+                                           const bool (&on)[T]) {
+  if (idx < 0) return;
+#pragma unroll
+  for (int t = 0; t < T; ++t)
+    if (on[t]) atomic_add4v(grad + (int64_t)idx * C + c[t], acc[t]);
 }
 
-// The block's LDS copy of a line (dynamic shared memory of the cell-sorted backward).  Named at
-// file scope so that every access is known to be an LDS access (ds_add_f32), not a flat one.
-extern __shared__ float g_line_lds[];
-
-__device__ __forceinline__ void flush_slot_lds(int idx, float4 acc, int C, int c) {
-  if (idx < 0) return;
-  const int o = idx * C + c;
-  atomicAdd(&g_line_lds[o + 0], acc.x);
-  atomicAdd(&g_line_lds[o + 1], acc.y);
-  atomicAdd(&g_line_lds[o + 2], acc.z);
-  atomicAdd(&g_line_lds[o + 3], acc.w);
+template <int N, int T>
+__device__ __forceinline__ void flush_slots(const int (&si)[N], const float4 (&sa)[N][T], float* grad, int C,
+                                            const int (&c)[T], const bool (&on)[T]) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) flush_slot(grad, si[k], sa[k], C, c, on);
 }
 
 __device__ __forceinline__ float4 pick4(bool b, float4 x, float4 y) {
   return make_float4(b ? x.x : y.x, b ? x.y : y.y, b ? x.z : y.z, b ? x.w : y.w);
 }
 
-__device__ __forceinline__ void plane_accum(int (&si)[4], float4 (&sa)[4], const int (&ci)[4], const float (&cw)[4],
-                                            float4 g, float* grad, int C, int c) {
+template <int T>
+__device__ __forceinline__ void plane_accum(int (&si)[4], float4 (&sa)[4][T], const int (&ci)[4], const float (&cw)[4],
+                                            const float4 (&g)[T], float* grad, int C, const int (&c)[T],
+                                            const bool (&on)[T]) {
   const bool same = ci[0] == si[0] && ci[1] == si[1] && ci[2] == si[2] && ci[3] == si[3];
-  const bool px = !same && ci[0] == si[1] && ci[2] == si[3];         // cell moved +x: nw<-ne, sw<-se
-  const bool nx = !same && !px && ci[1] == si[0] && ci[3] == si[2];  // -x: ne<-nw, se<-sw
-  const bool py = !same && !px && !nx && ci[0] == si[2] && ci[1] == si[3];          // +y: nw<-sw, ne<-se
-  const bool ny = !same && !px && !nx && !py && ci[2] == si[0] && ci[3] == si[1];  // -y: sw<-nw, se<-ne
-  if (!(same || nx || ny)) flush_slot(grad, si[0], sa[0], C, c);
-  if (!(same || px || ny)) flush_slot(grad, si[1], sa[1], C, c);
-  if (!(same || nx || py)) flush_slot(grad, si[2], sa[2], C, c);
-  if (!(same || px || py)) flush_slot(grad, si[3], sa[3], C, c);
-  const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-  const float4 n0 = pick4(same, sa[0], pick4(px, sa[1], pick4(py, sa[2], z)));
-  const float4 n1 = pick4(same, sa[1], pick4(nx, sa[0], pick4(py, sa[3], z)));
-  const float4 n2 = pick4(same, sa[2], pick4(px, sa[3], pick4(ny, sa[0], z)));
-  const float4 n3 = pick4(same, sa[3], pick4(nx, sa[2], pick4(ny, sa[1], z)));
-  sa[0] = madd4(n0, g, cw[0]);
-  sa[1] = madd4(n1, g, cw[1]);
-  sa[2] = madd4(n2, g, cw[2]);
-  sa[3] = madd4(n3, g, cw[3]);
+  if (__ballot(!same) != 0) {  // some lane's walk leaves its cell
+    const bool px = !same && ci[0] == si[1] && ci[2] == si[3];         // cell moved +x: nw<-ne, sw<-se
+    const bool nx = !same && !px && ci[1] == si[0] && ci[3] == si[2];  // -x: ne<-nw, se<-sw
+    const bool py = !same && !px && !nx && ci[0] == si[2] && ci[1] == si[3];          // +y: nw<-sw, ne<-se
+    const bool ny = !same && !px && !nx && !py && ci[2] == si[0] && ci[3] == si[1];  // -y: sw<-nw, se<-ne
+    if (!(same || nx || ny)) flush_slot(grad, si[0], sa[0], C, c, on);
+    if (!(same || px || ny)) flush_slot(grad, si[1], sa[1], C, c, on);
+    if (!(same || nx || py)) flush_slot(grad, si[2], sa[2], C, c, on);
+    if (!(same || px || py)) flush_slot(grad, si[3], sa[3], C, c, on);
+    const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-  for (int k = 0; k < 4; ++k) si[k] = ci[k];
+    for (int t = 0; t < T; ++t) {
+      const float4 n0 = pick4(same, sa[0][t], pick4(px, sa[1][t], pick4(py, sa[2][t], z)));
+      const float4 n1 = pick4(same, sa[1][t], pick4(nx, sa[0][t], pick4(py, sa[3][t], z)));
+      const float4 n2 = pick4(same, sa[2][t], pick4(px, sa[3][t], pick4(ny, sa[0][t], z)));
+      const float4 n3 = pick4(same, sa[3][t], pick4(nx, sa[2][t], pick4(ny, sa[1][t], z)));
+      sa[0][t] = n0;
+      sa[1][t] = n1;
+      sa[2][t] = n2;
+      sa[3][t] = n3;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) si[k] = ci[k];
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+#pragma unroll
+    for (int t = 0; t < T; ++t) sa[k][t] = madd4(sa[k][t], g[t], cw[k]);
 }
 
-template <bool kLds = false>
-__device__ __forceinline__ void line_accum(int (&si)[2], float4 (&sa)[2], const int (&ci)[2], const float (&cw)[2],
-                                           float4 g, float* grad, int C, int c) {
+template <int T>
+__device__ __forceinline__ void line_accum(int (&si)[2], float4 (&sa)[2][T], const int (&ci)[2], const float (&cw)[2],
+                                           const float4 (&g)[T], float* grad, int C, const int (&c)[T],
+                                           const bool (&on)[T]) {
   const bool same = ci[0] == si[0] && ci[1] == si[1];
-  const bool up = !same && ci[0] == si[1];          // lower <- upper
-  const bool down = !same && !up && ci[1] == si[0];  // upper <- lower
-  if (kLds) {  // grad unused: the slots flush into the LDS line copy
-    if (!(same || down)) flush_slot_lds(si[0], sa[0], C, c);
-    if (!(same || up)) flush_slot_lds(si[1], sa[1], C, c);
-  } else {
-    if (!(same || down)) flush_slot(grad, si[0], sa[0], C, c);
-    if (!(same || up)) flush_slot(grad, si[1], sa[1], C, c);
+  if (__ballot(!same) != 0) {
+    const bool up = !same && ci[0] == si[1];           // lower <- upper
+    const bool down = !same && !up && ci[1] == si[0];  // upper <- lower
+    if (!(same || down)) flush_slot(grad, si[0], sa[0], C, c, on);
+    if (!(same || up)) flush_slot(grad, si[1], sa[1], C, c, on);
+    const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const float4 n0 = pick4(same, sa[0][t], pick4(up, sa[1][t], z));
+      const float4 n1 = pick4(same, sa[1][t], pick4(down, sa[0][t], z));
+      sa[0][t] = n0;
+      sa[1][t] = n1;
+    }
+    si[0] = ci[0];
+    si[1] = ci[1];
   }
-  const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-  const float4 n0 = pick4(same, sa[0], pick4(up, sa[1], z));
-  const float4 n1 = pick4(same, sa[1], pick4(down, sa[0], z));
-  sa[0] = madd4(n0, g, cw[0]);
-  sa[1] = madd4(n1, g, cw[1]);
-  si[0] = ci[0];
-  si[1] = ci[1];
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+#pragma unroll
+    for (int t = 0; t < T; ++t) sa[k][t] = madd4(sa[k][t], g[t], cw[k]);
 }
 
 // Adds one sample's plane gradient gp and line gradient gl (before the corner weights).
-__device__ __forceinline__ void run_add(const VmArgs& a, const QuadSite& s, RunAcc& r, float4 gp, float4 gl) {
+__device__ __forceinline__ void run_add(const VmArgs& a, const QuadSite& s, RunAcc<1>& r, float4 gp, float4 gl) {
   const int C = sel3(s.p, a.comp[0], a.comp[1], a.comp[2]);
-  float* dP = sel3(s.p, a.dplane[0], a.dplane[1], a.dplane[2]);
-  float* dL = sel3(s.p, a.dline[0], a.dline[1], a.dline[2]);
-  const int c = s.c;
-  plane_accum(r.pidx, r.pg, s.pt.idx, s.pt.w, gp, dP, C, c);
-  line_accum(r.lidx, r.lg, s.lt.idx, s.lt.w, gl, dL, C, c);
+  const int c[1] = {s.c};
+  const bool on[1] = {true};
+  const float4 gps[1] = {gp}, gls[1] = {gl};
+  plane_accum<1>(r.pidx, r.pg, s.pt.idx, s.pt.w, gps, sel3(s.p, a.dplane[0], a.dplane[1], a.dplane[2]), C, c, on);
+  line_accum<1>(r.lidx, r.lg, s.lt.idx, s.lt.w, gls, sel3(s.p, a.dline[0], a.dline[1], a.dline[2]), C, c, on);
+}
+
+__device__ __forceinline__ void run_flush(const VmArgs& a, int p, int c0, const RunAcc<1>& r) {
+  const int C = sel3(p, a.comp[0], a.comp[1], a.comp[2]);
+  const int c[1] = {c0};
+  const bool on[1] = {true};
+  flush_slots<4, 1>(r.pidx, r.pg, sel3(p, a.dplane[0], a.dplane[1], a.dplane[2]), C, c, on);
+  flush_slots<2, 1>(r.lidx, r.lg, sel3(p, a.dline[0], a.dline[1], a.dline[2]), C, c, on);
 }
 
 // d_feat = d_sigma * predictor'(feat) on valid samples; planes receive d_feat * line and
@@ -586,7 +606,7 @@ __global__ __launch_bounds__(256) void density_bwd_kernel(VmArgs a, int64_t n, i
     const int64_t i0 = run * run_len;
     const int64_t i1 = i0 + run_len < n ? i0 + run_len : n;
     for (int q = gp.ql; q < a.n_quads; q += G) {
-      RunAcc r;
+      RunAcc<1> r;
       run_init(r);
       int p = 0, c = 0;
       for (int64_t i = i0; i < i1; ++i) {
@@ -604,8 +624,7 @@ __global__ __launch_bounds__(256) void density_bwd_kernel(VmArgs a, int64_t n, i
         p = site.p;
         c = site.c;
       }
-      run_flush_plane(a, p, c, r);
-      run_flush_line(a, p, c, r);
+      run_flush(a, p, c, r);
     }
   }
 }
@@ -654,7 +673,7 @@ __global__ __launch_bounds__(256) void appearance_bwd_kernel(VmArgs a, int64_t n
     const int64_t j0 = run * run_len;
     const int64_t j1 = j0 + run_len < n ? j0 + run_len : n;
     for (int q = gp.ql; q < a.n_quads; q += G) {
-      RunAcc r;
+      RunAcc<1> r;
       run_init(r);
       int p = 0, c = 0;
       for (int64_t j = j0; j < j1; ++j) {
@@ -670,8 +689,7 @@ __global__ __launch_bounds__(256) void appearance_bwd_kernel(VmArgs a, int64_t n
         p = site.p;
         c = site.c;
       }
-      run_flush_plane(a, p, c, r);
-      run_flush_line(a, p, c, r);
+      run_flush(a, p, c, r);
     }
   }
 }
@@ -682,8 +700,9 @@ __global__ __launch_bounds__(256) void appearance_bwd_kernel(VmArgs a, int64_t n
 // component.  With a caller workspace the backward instead orders the contributing rows by the
 // plane cell of their nw corner (a counting sort per plane: histogram, one scan, a scatter of row
 // numbers), so that a lane group walking the sorted rows meets each cell's samples in one run and
-// flushes each texel about once per run; the line gradients of the walk (the third coordinate of
-// the rows of one cell is arbitrary) go to a copy of the line in LDS, flushed once per block.
+// flushes each texel about once per run.  An order whose major axis is the coordinate of another
+// plane's line serves that line's gradients too, so every line has an order in which it stays on
+// one interval for whole rows of cells.
 // The order within a cell comes from integer atomics and varies between calls, as the order of
 // the FP32 atomics does anyway.
 struct BwdRows {
@@ -737,7 +756,14 @@ __device__ __forceinline__ void normalized_point(const VmArgs& a, const float* p
   for (int k = 0; k < 3; ++k) pn[k] = normalize_coord(pts[3 * i + k], a.lo[k], a.size[k]);
 }
 
-// Sort key of a sample for plane p: the cell of its nw corner, clamped into the plane.
+// Plane p's order also serves the line of another plane, whose coordinate is the order's major axis: z for
+// plane 1 (x, z), x for plane 0 (x, y), y for plane 2 (y, z).
+__device__ __host__ __forceinline__ constexpr int order_line(int p) { return (p + 2) % kPlanes; }
+__device__ __host__ __forceinline__ bool has_order(const VmArgs& a, int p) {
+  return a.comp[p] != 0 || a.comp[order_line(p)] != 0;
+}
+
+// Sort key of a sample for plane p: the cell of its nw corner, clamped into the plane, the major axis first.
 __device__ __forceinline__ int plane_cell(const VmArgs& a, int p, const float pn[3]) {
   const int W = sel3(p, a.pw[0], a.pw[1], a.pw[2]), H = sel3(p, a.ph[0], a.ph[1], a.ph[2]);
   const float x = sel3(p, pn[axis_a0(0)], pn[axis_a0(1)], pn[axis_a0(2)]);
@@ -745,7 +771,7 @@ __device__ __forceinline__ int plane_cell(const VmArgs& a, int p, const float pn
   int xi = (int)floorf(source_index(x, W)), yi = (int)floorf(source_index(y, H));
   xi = xi < 0 ? 0 : (xi > W - 1 ? W - 1 : xi);
   yi = yi < 0 ? 0 : (yi > H - 1 ? H - 1 : yi);
-  return yi * W + xi;
+  return p == 1 ? yi * W + xi : xi * H + yi;
 }
 
 __global__ __launch_bounds__(256) void fill_zero_kernel(int32_t* __restrict__ p, int64_t n) {
@@ -794,7 +820,7 @@ __global__ __launch_bounds__(256) void cell_count_kernel(VmArgs a, BwdRows r, So
     if (active) normalized_point(a, r.pts, i, pn);
 #pragma unroll
     for (int p = 0; p < kPlanes; ++p) {
-      if (a.comp[p] == 0) continue;  // uniform
+      if (!has_order(a, p)) continue;  // uniform
       const int key = active ? plane_cell(a, p, pn) : -1;
       const WaveRun run = wave_run(key, active);
       if (!kScatter) {
@@ -882,90 +908,288 @@ __global__ __launch_bounds__(kScanThreads) void cell_chunk_apply_kernel(SortWs w
   }
 }
 
-constexpr int kSortedThreads = 512;
-constexpr int kMaxLineLds = 160 * 1024;  // a CU's LDS
-// Component slices of the sorted backward: a line copy above kLineLdsSplit (at most two blocks per
-// CU) is split into slices of at most kLineLdsSlice.  Measured: the 512 x 64 appearance line (128 KB,
-// one block per CU) walks faster in four slices (4.42 -> 4.08 ms per uneven-batch step), while
-// splitting the 57.6 KB and 48 KB copies of the 300^2 appearance and 512^2 density lines cost more
-// (re-walked rows) than the added blocks gained.
-constexpr int kLineLdsSplit = 64 * 1024;
-constexpr int kLineLdsSlice = 32 * 1024;
+constexpr int kSortedThreads = 256;
+constexpr int kSortedPerCu = 3;   // blocks of a round per compute unit
+constexpr int kSortedLeast = 16;  // least rows of a lane group
 
-// Plane p's gradients from its cell-sorted rows: a lane group walks run_len consecutive sorted
-// rows with the corner slots of the run walk (flushing a plane texel when the walk leaves it) and
-// adds the line gradients into g_line_lds (the line copy in LDS, line_lds != 0) or, when the line is
-// too large for LDS, through the line slots of the run walk.  The plane's components are split into
-// gridDim.y slices of whole quads: a block walks its rows for one slice and keeps only that slice's
-// columns of the line in LDS (L x Cs floats), so that more blocks fit in a CU's LDS.
-template <int G, bool kDensity>
-__global__ __launch_bounds__(kSortedThreads) void sorted_bwd_kernel(VmArgs a, BwdRows r, SortWs w, int p,
-                                                                    int run_len, int line_lds) {
-  const int C = sel3(p, a.comp[0], a.comp[1], a.comp[2]);
-  const int L = sel3(p, a.ll[0], a.ll[1], a.ll[2]);
-  const int qs = C / 4 / (int)gridDim.y;           // quads of the slice
-  const int Cs = 4 * qs, cb = Cs * (int)blockIdx.y;  // its components: cb .. cb + Cs - 1
-  const int64_t m = w.total[p];
-  const int groups = kSortedThreads / G;
-  const int64_t b0 = (int64_t)blockIdx.x * groups * run_len;
-  if (b0 >= m) return;  // uniform over the block
-  if (line_lds) {
-    for (int e = threadIdx.x; e < L * Cs; e += kSortedThreads) g_line_lds[e] = 0.f;
-    __syncthreads();
+// LDS of one wave of the sorted backward: the prepared rows of its groups and a queue of texels that walks
+// have left (entry e is the sums of one group, a quad a lane, at sum[lanes e], for texel[e]).
+// A prepared row: the corner weights of plane P and of plane PL, the interval weights of their lines, the
+// texels (of plane P and line PL, where gradients go) and quad offsets (of line P and plane PL, whose values
+// are read), the flags of plane P's site and, 16 bits up, of plane PL's, and the entry's last word.
+struct WaveWalk {
+  float4 wp[SRF_WAVE], wq[SRF_WAVE], wl[SRF_WAVE];
+  int4 at[SRF_WAVE];
+  int2 word[SRF_WAVE];
+  float4 sum[4 * SRF_WAVE];
+  int texel[4 * SRF_WAVE];
+};
+
+__device__ __forceinline__ float4 corner_weights(float x1, float y1) {
+  const float x0 = __fsub_rn(1.0f, x1), y0 = __fsub_rn(1.0f, y1);
+  return make_float4(__fmul_rn(x0, y0), __fmul_rn(x1, y0), __fmul_rn(x0, y1), __fmul_rn(x1, y1));
+}
+
+__device__ __forceinline__ float4 fma4(float4 v, float w, float4 acc) {
+  return make_float4(fmaf(v.x, w, acc.x), fmaf(v.y, w, acc.y), fmaf(v.z, w, acc.z), fmaf(v.w, w, acc.w));
+}
+
+__device__ __forceinline__ float4 scale4(float4 v, float w) {
+  return make_float4(__fmul_rn(v.x, w), __fmul_rn(v.y, w), __fmul_rn(v.z, w), __fmul_rn(v.w, w));
+}
+
+// A block's sums of the line texels base .. base + kLineSums / C - 1.
+constexpr int kLineSums = 4 * 4 * kMaxQuads;
+struct BlockLine {
+  float sum[kLineSums];
+  int base, texels;
+};
+
+// Adds the queue's texels (C components each) to HBM, or those within the block's line texels in LDS, and
+// empties it.  The wave goes over them dword by dword, so that an atomic instruction covers whole cache
+// lines: device-scope adds are done line by line behind the L2, and a lane adding its own 4 components with
+// 4 instructions takes each line 4 times.
+template <bool kBlockLine>
+__device__ __forceinline__ void queue_flush(WaveWalk& f, int& count, int lanes, float* __restrict__ grad, int C,
+                                            uint32_t inv_c, BlockLine* line) {
+  const float* sums = reinterpret_cast<const float*>(f.sum);
+  wave_lds_fence();
+  for (int e = threadIdx.x & (SRF_WAVE - 1); e < count * C; e += SRF_WAVE) {
+    const int n = (int)(((uint32_t)e * inv_c) >> 20), d = e - n * C;  // e / C: e < 1024
+    const int texel = f.texel[n];
+    const float v = sums[4 * lanes * n + d];
+    if (kBlockLine && (uint32_t)(texel - line->base) < (uint32_t)line->texels)
+      atomicAdd(&line->sum[(texel - line->base) * C + d], v);
+    else
+      unsafeAtomicAdd(grad + (int64_t)texel * C + d, v);
   }
-  const int grp = threadIdx.x / G, ql = threadIdx.x % G;
-  const int64_t s0 = b0 + (int64_t)grp * run_len;
-  const int64_t s1 = s0 + run_len < m ? s0 + run_len : m;
-  const int q0 = sel3(p, a.qoff[0], a.qoff[1], a.qoff[2]);
-  float* dP = sel3(p, a.dplane[0], a.dplane[1], a.dplane[2]);
-  float* dL = sel3(p, a.dline[0], a.dline[1], a.dline[2]);
-  const float4* order = sel3(p, w.order[0], w.order[1], w.order[2]);
-  for (int q = q0 + cb / 4 + ql; q < q0 + cb / 4 + qs; q += G) {
-    RunAcc acc;
-    run_init(acc);
-    int c = 0;
-    // The next row's entry (and its output gradient) are loaded one row ahead, so that a row waits
-    // for its taps only; the look-ahead index is clamped to the last entry (always written).
-    auto grad_of = [&](const float4& e) -> float4 {
-      return kDensity ? make_float4(e.w, e.w, e.w, e.w)
-                      : ld4(r.d_out + (int64_t)__float_as_int(e.w) * a.total_comp + 4 * q);
-    };
-    float4 en = order[s0 < m ? s0 : m - 1];
-    float4 gn = grad_of(en);
-    for (int64_t s = s0; s < s1; ++s) {
-      const float4 e = en, g = gn;
-      en = order[s + 1 < m ? s + 1 : m - 1];
+  wave_lds_fence();
+  count = 0;
+}
+
+// Queues the slots k with leave[k] (the same for all lanes of a group, false in the lanes past the last whole
+// group) of every group, after a flush if they would not fit.  All lanes of the wave call it.
+template <int N, bool kBlockLine = false>
+__device__ __forceinline__ void queue_slots(WaveWalk& f, int& count, int lanes, int grp, int ql, const int (&si)[N],
+                                            const float4 (&sa)[N], const bool (&leave)[N], float* __restrict__ grad, int C,
+                                            uint32_t inv_c, BlockLine* line = nullptr) {
+  uint64_t m[N];
+  int add = 0;
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    m[k] = __ballot(leave[k] && ql == 0);
+    add += __popcll(m[k]);
+  }
+  if (add == 0) return;
+  if ((count + add) * lanes > 4 * SRF_WAVE) queue_flush<kBlockLine>(f, count, lanes, grad, C, inv_c, line);
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    if (leave[k]) {
+      const int n = count + __popcll(m[k] & ((1ull << (grp * lanes)) - 1ull));
+      f.sum[n * lanes + ql] = sa[k];
+      if (ql == 0) f.texel[n] = si[k];
+    }
+    count += __popcll(m[k]);
+  }
+}
+
+// The corners of a prepared site: texels, -1 outside the factor.
+__device__ __forceinline__ void site_corners(int i00, int flags, int W, int (&idx)[4]) {
+  const int dx = (flags & kDx) ? 1 : 0, dy = (flags & kDy) ? W : 0;
+  idx[0] = (flags & 1) ? i00 : -1;
+  idx[1] = (flags & 2) ? i00 + dx : -1;
+  idx[2] = (flags & 4) ? i00 + dy : -1;
+  idx[3] = (flags & 8) ? i00 + dy + dx : -1;
+}
+
+// One order's gradients: plane P's, and those of the line whose coordinate is the order's major axis (plane
+// PL's line).  A group of `lanes` lanes, one quad of components each, walks run_len consecutive sorted rows
+// (0: the rows that there are, over the grid's groups) and keeps the sums of the cell's four corners and of the
+// line's interval in registers until the walk leaves them.  The group's lanes prepare its next rows, one a
+// lane, as the forward does.  The line sums left at the end of the runs, of the same few texels for all groups
+// of a block, are added up in LDS and flushed once per block.
+//
+// What bounded it was the line of plane P itself, whose coordinate is arbitrary among a cell's rows and changed
+// its texel with nearly every row: its copy in LDS took 8 LDS float adds per row and quad, which run at about
+// one lane a clock and were half of the time.  With another plane's line the atomics did (each makes the loads
+// behind it wait, hence the queue), then the cells and weights that every lane repeated (hence the prepared
+// rows).  Now the appearance rows' output gradients, read twice (0.56 GB an order at 3 x 48 components and
+// 1.45M rows), and the vector ALU share the time.  Three orders of 1.45M rows of 3 x 48 components: 1.46 ->
+// 0.78 ms; of the alpha-masked samples of 3.6M at 3 x 16: 0.37 -> 0.16 ms.  Three blocks per compute unit (its
+// registers and LDS): 2 and 4 measured 0.79 and 0.78, and 0.17 and 0.20 (more runs to flush).
+template <int P, bool kDensity>
+__global__ __launch_bounds__(kSortedThreads, 3) void sorted_bwd_kernel(VmArgs a, BwdRows r, SortWs w, int lanes, int run_len) {
+  constexpr int PL = order_line(P);
+  __shared__ WaveWalk walk[kSortedThreads / SRF_WAVE];
+  __shared__ BlockLine bline;
+  const int64_t m = w.total[P];
+  const int lane = threadIdx.x & (SRF_WAVE - 1), wv = threadIdx.x / SRF_WAVE;
+  const int per_wave = SRF_WAVE / lanes;
+  const int groups = (kSortedThreads / SRF_WAVE) * per_wave;
+  const int64_t all = (int64_t)gridDim.x * groups;
+  if (run_len == 0) run_len = max(kSortedLeast, (int)((m + all - 1) / all));
+  const int grp = lane / lanes, ql = lane - grp * lanes;
+  const int64_t block0 = (int64_t)blockIdx.x * groups * run_len;
+  if (block0 >= m) return;  // uniform over the block
+  const int64_t s0 = block0 + ((int64_t)wv * per_wave + grp) * run_len;
+  // rows of this lane's group: none past the last row or in the lanes past the last whole group
+  const int rows = grp < per_wave ? (int)max((int64_t)0, min((int64_t)run_len, m - s0)) : 0;
+  const int C = a.comp[P], CL = a.comp[PL];
+  const uint32_t inv_c = C ? (1u << 20) / C + 1 : 0, inv_cl = CL ? (1u << 20) / CL + 1 : 0;
+  const float4* order = w.order[P];
+  WaveWalk& ws = walk[wv];
+  for (int e = threadIdx.x; e < kLineSums; e += kSortedThreads) bline.sum[e] = 0.f;
+  if (threadIdx.x == 0) {
+    const float4 e = order[block0];
+    const float pn[3] = {e.x, e.y, e.z};
+    float4 frac;
+    int2 at;
+    prepare_site(a, PL, pn, frac, at);
+    bline.base = at.y;
+    bline.texels = CL ? kLineSums / CL : 0;
+  }
+  __syncthreads();
+  // this lane's components of the plane and of the line; lanes past the last quad repeat the first one's
+  // and are not flushed
+  const int c = 4 * ql < C ? 4 * ql : 0, cl = 4 * ql < CL ? 4 * ql : 0;
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  int pat = 0, pflags = 0, lat = 0, lflags = 0;  // the site the slots belong to (flags 0: none)
+  float4 pg[4] = {zero, zero, zero, zero}, lg[2] = {zero, zero};
+  int queued = 0;  // the wave's
+  auto grads_of = [&](float word, float4& gp, float4& gl) {
+    if (kDensity) {
+      gp = gl = make_float4(word, word, word, word);
+    } else {
+      const float* row = r.d_out + (int64_t)__float_as_int(word) * a.total_comp;
+      gp = C ? ld4(row + 4 * a.qoff[P] + c) : zero;
+      gl = CL ? ld4(row + 4 * a.qoff[PL] + cl) : zero;
+    }
+  };
+  float4 en = order[min(s0 + ql, m - 1)];  // the next row that this lane prepares
+  for (int k0 = 0; __ballot(k0 < rows) != 0; k0 += lanes) {
+    {
+      const float4 e = en;
+      en = order[min(s0 + k0 + lanes + ql, m - 1)];
       const float pn[3] = {e.x, e.y, e.z};
-      const QuadSite site = quad_site(a, q, pn);
-      float4 pv, lv;
-      quad_values(a, site, pv, lv);
-      plane_accum(acc.pidx, acc.pg, site.pt.idx, site.pt.w, mul4(g, lv), dP, C, site.c);
-      const float4 gl = mul4(g, pv);
-      // the line slots carry a texel while consecutive rows (one ray's samples within the cell) stay
-      // on it, and flush into the LDS copy (or HBM) when the walk leaves it
-      if (line_lds)
-        line_accum<true>(acc.lidx, acc.lg, site.lt.idx, site.lt.w, gl, nullptr, Cs, site.c - cb);
-      else
-        line_accum<false>(acc.lidx, acc.lg, site.lt.idx, site.lt.w, gl, dL, C, site.c);
-      c = site.c;
-      gn = grad_of(en);
+      float4 fp, fq;
+      int2 ap, aq;
+      prepare_site(a, P, pn, fp, ap);
+      prepare_site(a, PL, pn, fq, aq);
+      ws.wp[lane] = corner_weights(fp.x, fp.y);
+      ws.wq[lane] = corner_weights(fq.x, fq.y);
+      ws.wl[lane] = make_float4(__fsub_rn(1.0f, fp.z), fp.z, __fsub_rn(1.0f, fq.z), fq.z);
+      ws.at[lane] = make_int4(ap.x, aq.y, (int)((uint32_t)ap.y * (uint32_t)(C / 4)), (int)((uint32_t)aq.x * (uint32_t)(CL / 4)));
+      ws.word[lane] = make_int2(__float_as_int(fp.w) | __float_as_int(fq.w) << 16, __float_as_int(e.w));
     }
-    run_flush_plane(a, p, c, acc);
-    for (int t = 0; t < 2; ++t) {
-      if (line_lds)
-        flush_slot_lds(acc.lidx[t], acc.lg[t], Cs, c - cb);
-      else
-        flush_slot(dL, acc.lidx[t], acc.lg[t], C, c);
+    wave_lds_fence();
+    const int slot0 = min(grp * lanes, SRF_WAVE - lanes);
+    for (int k = 0; k < lanes; ++k) {
+      const bool live = k0 + k < rows;
+      if (__ballot(live) == 0) break;
+      const int4 at = ws.at[slot0 + k];
+      const int2 fw = ws.word[slot0 + k];
+      const int fgp = fw.x & 0xffff, fgq = fw.x >> 16;
+      float4 gp, gl, lt[2] = {zero, zero}, pt[4] = {zero, zero, zero, zero};
+      if (kDensity) {
+        const float g = __int_as_float(fw.y);
+        gp = gl = make_float4(g, g, g, g);
+      } else {
+        const float* row = r.d_out + (int64_t)fw.y * a.total_comp;
+        gp = C ? ld4(row + 4 * a.qoff[P] + c) : zero;
+        gl = CL ? ld4(row + 4 * a.qoff[PL] + cl) : zero;
+      }
+      if (C) {
+        const float* L = a.line[P] + 4 * (size_t)(uint32_t)at.z + c;
+        lt[0] = ld4(L);
+        lt[1] = ld4(L + ((fgp & kDl) ? C : 0));
+      }
+      if (CL) {
+        const float* Q = a.plane[PL] + 4 * (size_t)(uint32_t)at.w + cl;
+        const int dx = (fgq & kDx) ? CL : 0;
+        const float* Q1 = Q + ((fgq & kDy) ? (int64_t)a.pw[PL] * CL : 0);
+        pt[0] = ld4(Q);
+        pt[1] = ld4(Q + dx);
+        pt[2] = ld4(Q1);
+        pt[3] = ld4(Q1 + dx);
+      }
+      {
+        const bool same = !live || (at.x == pat && ((fgp ^ pflags) & 15) == 0);
+        if (__ballot(!same) != 0) {  // some walk leaves its cell
+          // the next cell of the order, one step along the minor axis, shares two texels; any other move
+          // leaves all four
+          int o[4];
+          site_corners(pat, pflags, a.pw[P], o);
+          constexpr int kB = P == 1 ? 1 : 2;  // +minor: slot k takes slot k + kB's sums, if 0 <= o[k + kB]
+          const bool step = (fgp & pflags & 15) == 15 && at.x == o[kB];
+          const bool leave[4] = {!same && o[0] >= 0, !same && o[1] >= 0 && !(P == 1 && step),
+                                 !same && o[2] >= 0 && !(P != 1 && step), !same && o[3] >= 0 && !step};
+          queue_slots<4>(ws, queued, lanes, grp, ql, o, pg, leave, a.dplane[P], C, inv_c);
+          constexpr int kA = 3 - kB;  // slots 0 and kA are the lower ones along the minor axis
+          pg[0] = pick4(same, pg[0], pick4(step, pg[kB], zero));
+          pg[kA] = pick4(same, pg[kA], pick4(step, pg[3], zero));
+          pg[kB] = pick4(same, pg[kB], zero);
+          pg[3] = pick4(same, pg[3], zero);
+          pat = same ? pat : at.x;
+          pflags = same ? pflags : fgp;
+        }
+      }
+      {
+        const bool same = !live || (at.y == lat && ((fgq ^ lflags) & 48) == 0);
+        if (__ballot(!same) != 0) {
+          const int o[2] = {(lflags & 16) ? lat : -1, (lflags & 32) ? lat + ((lflags & kDl) ? 1 : 0) : -1};
+          const bool up = (fgq & lflags & 48) == 48 && at.y == o[1];  // lower <- upper
+          const bool leave[2] = {!same && o[0] >= 0, !same && o[1] >= 0 && !up};
+          queue_flush<false>(ws, queued, lanes, a.dplane[P], C, inv_c, nullptr);  // (rare: the queue holds one kind)
+          queue_slots<2, true>(ws, queued, lanes, grp, ql, o, lg, leave, a.dline[PL], CL, inv_cl, &bline);
+          queue_flush<true>(ws, queued, lanes, a.dline[PL], CL, inv_cl, &bline);
+          lg[0] = pick4(same, lg[0], pick4(up, lg[1], zero));
+          lg[1] = pick4(same, lg[1], zero);
+          lat = same ? lat : at.y;
+          lflags = same ? lflags : fgq;
+        }
+      }
+      const float4 wq = ws.wq[slot0 + k], wl = ws.wl[slot0 + k];
+      float4 lv, pv;
+      if (__ballot((fgp & fgq & kTapAll) != kTapAll) == 0) {
+        lv = fma4(lt[1], wl.y, scale4(lt[0], wl.x));
+        pv = fma4(pt[3], wq.w, fma4(pt[2], wq.z, fma4(pt[1], wq.y, scale4(pt[0], wq.x))));
+      } else {  // some corner lies outside its factor and adds nothing
+        const float lw[2] = {wl.x, wl.y}, qw[4] = {wq.x, wq.y, wq.z, wq.w};
+        const bool okl[2] = {(fgp & 16) != 0, (fgp & 32) != 0};
+        const bool okq[4] = {(fgq & 1) != 0, (fgq & 2) != 0, (fgq & 4) != 0, (fgq & 8) != 0};
+        lv = tap_sum(lt, lw, false, okl);
+        pv = tap_sum(pt, qw, false, okq);
+      }
+      if (live) {
+        const float4 wp = ws.wp[slot0 + k];
+        gp = mul4(gp, lv);
+        gl = mul4(gl, pv);
+        pg[0] = fma4(gp, wp.x, pg[0]);
+        pg[1] = fma4(gp, wp.y, pg[1]);
+        pg[2] = fma4(gp, wp.z, pg[2]);
+        pg[3] = fma4(gp, wp.w, pg[3]);
+        lg[0] = fma4(gl, wl.z, lg[0]);
+        lg[1] = fma4(gl, wl.w, lg[1]);
+      }
     }
+    wave_lds_fence();
   }
-  if (line_lds) {
-    __syncthreads();
-    for (int e = threadIdx.x; e < L * Cs; e += kSortedThreads) {
-      const float v = g_line_lds[e];
-      const int row = e / Cs;
-      if (v != 0.f) unsafeAtomicAdd(dL + (int64_t)row * C + cb + (e - row * Cs), v);
-    }
+  {
+    int o[4];
+    site_corners(pat, pflags, a.pw[P], o);
+    const bool leave[4] = {o[0] >= 0, o[1] >= 0, o[2] >= 0, o[3] >= 0};
+    queue_slots<4>(ws, queued, lanes, grp, ql, o, pg, leave, a.dplane[P], C, inv_c);
+    queue_flush<false>(ws, queued, lanes, a.dplane[P], C, inv_c, nullptr);
   }
+  {
+    const int o[2] = {(lflags & 16) ? lat : -1, (lflags & 32) ? lat + ((lflags & kDl) ? 1 : 0) : -1};
+    const bool leave[2] = {o[0] >= 0, o[1] >= 0};
+    queue_slots<2, true>(ws, queued, lanes, grp, ql, o, lg, leave, a.dline[PL], CL, inv_cl, &bline);
+    queue_flush<true>(ws, queued, lanes, a.dline[PL], CL, inv_cl, &bline);
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < bline.texels * CL; e += kSortedThreads)
+    if (bline.sum[e] != 0.f) unsafeAtomicAdd(a.dline[PL] + (int64_t)bline.base * CL + e, bline.sum[e]);
 }
 
 // ------------------------------------------------------------ CP decomposition (3 lines)
@@ -1008,7 +1232,7 @@ __device__ __forceinline__ float4 cp_product(const float4 v[kPlanes]) { return m
 // Run-length gradient accumulation for the three lines of one quad (as RunAcc for VM).
 struct CpRun {
   int idx[kPlanes][2];
-  float4 g[kPlanes][2];
+  float4 g[kPlanes][2][1];
 };
 
 __device__ __forceinline__ void cp_run_init(CpRun& r) {
@@ -1017,26 +1241,28 @@ __device__ __forceinline__ void cp_run_init(CpRun& r) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       r.idx[k][t] = -1;
-      r.g[k][t] = make_float4(0.f, 0.f, 0.f, 0.f);
+      r.g[k][t][0] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
 }
 
-__device__ __forceinline__ void cp_run_flush(const CpArgs& a, int k, int c, CpRun& r) {
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    if (r.idx[k][t] >= 0) atomic_add4v(a.dline[k] + (int64_t)r.idx[k][t] * a.comp + c, r.g[k][t]);
-    r.g[k][t] = make_float4(0.f, 0.f, 0.f, 0.f);
-  }
+__device__ __forceinline__ void cp_run_flush(const CpArgs& a, int k, int c0, const CpRun& r) {
+  const int c[1] = {c0};
+  const bool on[1] = {true};
+  flush_slots<2, 1>(r.idx[k], r.g[k], a.dline[k], a.comp, c, on);
 }
 
 // Adds the gradient g of the quad's component products: line k receives g times the other two
 // lines' values, spread over its two taps.
-__device__ __forceinline__ void cp_run_add(const CpArgs& a, const CpTaps& s, int c, CpRun& r, float4 g,
+__device__ __forceinline__ void cp_run_add(const CpArgs& a, const CpTaps& s, int c0, CpRun& r, float4 g,
                                            const float4 v[kPlanes]) {
   const float4 d[kPlanes] = {mul4(mul4(g, v[1]), v[2]), mul4(mul4(g, v[0]), v[2]), mul4(mul4(g, v[0]), v[1])};
+  const int c[1] = {c0};
+  const bool on[1] = {true};
 #pragma unroll
-  for (int k = 0; k < kPlanes; ++k)
-    line_accum(r.idx[k], r.g[k], s.t[k].idx, s.t[k].w, d[k], a.dline[k], a.comp, c);
+  for (int k = 0; k < kPlanes; ++k) {
+    const float4 dk[1] = {d[k]};
+    line_accum<1>(r.idx[k], r.g[k], s.t[k].idx, s.t[k].w, dk, a.dline[k], a.comp, c, on);
+  }
 }
 
 template <int G>
@@ -1356,17 +1582,6 @@ int run_length() {
   else                                                                                             \
     hipLaunchKernelGGL((KERNEL<8, false>), __VA_ARGS__);
 
-#define SRF_VM_DISPATCH_KD(G_, KD, KERNEL, ...)                                            \
-  switch (G_) {                                                                           \
-    case 1: hipLaunchKernelGGL((KERNEL<1, KD>), __VA_ARGS__); break;                      \
-    case 2: hipLaunchKernelGGL((KERNEL<2, KD>), __VA_ARGS__); break;                      \
-    case 4: hipLaunchKernelGGL((KERNEL<4, KD>), __VA_ARGS__); break;                      \
-    case 8: hipLaunchKernelGGL((KERNEL<8, KD>), __VA_ARGS__); break;                      \
-    case 16: hipLaunchKernelGGL((KERNEL<16, KD>), __VA_ARGS__); break;                    \
-    case 32: hipLaunchKernelGGL((KERNEL<32, KD>), __VA_ARGS__); break;                    \
-    default: hipLaunchKernelGGL((KERNEL<64, KD>), __VA_ARGS__); break;                    \
-  }
-
 // Workspace of the cell-sorted backward for `rows` rows (capacity), and its carving.
 size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 
@@ -1412,35 +1627,32 @@ SortWs carve_sorted_ws(const VmArgs& a, int64_t rows, void* ws) {
   return w;
 }
 
-// The dynamic LDS of the sorted kernels (the line copy) can exceed the 64 KB default: raise the
-// limit of every instantiation once per device, before any call that could be under capture.
-template <bool kDensity>
-int raise_sorted_lds_limit() {
-  constexpr int kMaxDevices = 64;
-  static std::mutex mutex;
-  static bool raised[kMaxDevices];
-  int dev = -1;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return SRF_EHIP;
-  std::lock_guard<std::mutex> lock(mutex);
-  if (raised[dev]) return SRF_OK;
-  const void* fns[] = {
-      reinterpret_cast<const void*>(&sorted_bwd_kernel<1, kDensity>),
-      reinterpret_cast<const void*>(&sorted_bwd_kernel<2, kDensity>),
-      reinterpret_cast<const void*>(&sorted_bwd_kernel<4, kDensity>),
-      reinterpret_cast<const void*>(&sorted_bwd_kernel<8, kDensity>),
-      reinterpret_cast<const void*>(&sorted_bwd_kernel<16, kDensity>),
-      reinterpret_cast<const void*>(&sorted_bwd_kernel<32, kDensity>),
-      reinterpret_cast<const void*>(&sorted_bwd_kernel<64, kDensity>)};
-  for (const void* f : fns)
-    if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLineLds) != hipSuccess)
-      return SRF_EHIP;
-  raised[dev] = true;
-  return SRF_OK;
+template <int P, bool kDensity>
+void launch_sorted_plane(const VmArgs& a, const BwdRows& r, const SortWs& w, hipStream_t s) {
+  if (!has_order(a, P)) return;
+  const int lanes = std::max(a.comp[P], a.comp[order_line(P)]) / 4;
+  const int groups = kSortedThreads / SRF_WAVE * (SRF_WAVE / lanes);
+  // as many blocks as the chip holds, which share the rows that there are; or, with the gather run knob,
+  // blocks for runs of that length over the capacity
+  const int64_t run = tune_value(SRF_TUNE_GATHER_RUN);
+  const int64_t least = run ? run : kSortedLeast;
+  const int64_t round = run ? INT32_MAX : (int64_t)device_compute_units() * kSortedPerCu;
+  const int64_t blocks = std::max<int64_t>(1, std::min(round, (r.n + groups * least - 1) / (groups * least)));
+  hipLaunchKernelGGL((sorted_bwd_kernel<P, kDensity>), dim3((unsigned)blocks), dim3(kSortedThreads), 0, s, a, r, w, lanes,
+                     (int)run);
+}
+
+// The prepared rows hold quad offsets of 32 bits (planes of up to 64 GB).
+bool sorted_addressable(const VmArgs& a) {
+  for (int p = 0; p < kPlanes; ++p)
+    if ((uint64_t)a.ph[p] * a.pw[p] * (a.comp[p] / 4) >= (1ull << 32) ||
+        (uint64_t)a.ll[p] * (a.comp[p] / 4) >= (1ull << 32))
+      return false;
+  return true;
 }
 
 template <bool kDensity>
 int launch_sorted_bwd(const VmArgs& a, const BwdRows& r, void* ws, hipStream_t s) {
-  if (const int st = raise_sorted_lds_limit<kDensity>(); st != SRF_OK) return st;
   const SortWs w = carve_sorted_ws(a, r.n, ws);
   const int64_t zb = (w.zero_count + 255) / 256;
   hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)(zb < 2048 ? zb : 2048)), dim3(256), 0, s, w.zero_begin,
@@ -1455,29 +1667,9 @@ int launch_sorted_bwd(const VmArgs& a, const BwdRows& r, void* ws, hipStream_t s
   hipLaunchKernelGGL(cell_chunk_scan_kernel, dim3(kPlanes), dim3(kScanThreads), 0, s, w);
   hipLaunchKernelGGL(cell_chunk_apply_kernel, dim3(chunks, kPlanes), dim3(kScanThreads), 0, s, w);
   hipLaunchKernelGGL((cell_count_kernel<kDensity, true>), dim3(row_blocks), dim3(256), 0, s, a, r, w);
-  for (int p = 0; p < kPlanes; ++p) {
-    if (a.comp[p] == 0) continue;
-    // component slices: halve the slice (whole quads) while its line copy exceeds kLineLdsSlice,
-    // when the whole line fits in LDS but above kLineLdsSplit
-    const int quads = a.comp[p] / 4;
-    const size_t full_line = (size_t)a.ll[p] * a.comp[p] * sizeof(float);
-    int ns = 1;
-    if (full_line <= (size_t)kMaxLineLds && full_line > (size_t)kLineLdsSplit)
-      while ((size_t)a.ll[p] * (a.comp[p] / ns) * sizeof(float) > (size_t)kLineLdsSlice && quads % (2 * ns) == 0)
-        ns *= 2;
-    const int G = next_pow2(quads / ns);
-    const int groups = kSortedThreads / G;
-    // about 1024 blocks over the capacity (fewer run when the device count is lower), unless the
-    // gather run knob sets the walk length
-    int64_t run = (r.n + 1024LL * groups - 1) / (1024LL * groups);
-    run = run < 16 ? 16 : (run > 256 ? 256 : run);
-    if (const int64_t v = tune_value(SRF_TUNE_GATHER_RUN)) run = v;
-    const int64_t blocks = (r.n + (int64_t)groups * run - 1) / ((int64_t)groups * run);
-    const size_t line_bytes = (size_t)a.ll[p] * (a.comp[p] / ns) * sizeof(float);
-    const int line_lds = line_bytes <= (size_t)kMaxLineLds ? 1 : 0;
-    SRF_VM_DISPATCH_KD(G, kDensity, sorted_bwd_kernel, dim3((unsigned)(blocks > 0 ? blocks : 1), ns),
-                       dim3(kSortedThreads), line_lds ? line_bytes : 0, s, a, r, w, p, (int)run, line_lds);
-  }
+  launch_sorted_plane<0, kDensity>(a, r, w, s);
+  launch_sorted_plane<1, kDensity>(a, r, w, s);
+  launch_sorted_plane<2, kDensity>(a, r, w, s);
   return launch_status();
 }
 
@@ -1528,7 +1720,7 @@ extern "C" int srf_vm_density_bwd(const srf_vm_factors* factors, float* const* d
     a.dplane[p] = d_planes[p];
     a.dline[p] = d_lines[p];
   }
-  if (workspace) {
+  if (workspace && sorted_addressable(a)) {
     BwdRows r;
     memset(&r, 0, sizeof(r));
     r.n = n_points;
@@ -1576,7 +1768,7 @@ extern "C" int srf_vm_appearance_bwd(const srf_vm_factors* factors, float* const
     a.dplane[p] = d_planes[p];
     a.dline[p] = d_lines[p];
   }
-  if (workspace) {
+  if (workspace && sorted_addressable(a)) {
     BwdRows r;
     memset(&r, 0, sizeof(r));
     r.n = n_rows;
