@@ -12,10 +12,13 @@ constexpr int kCdwWaves = 8;
 constexpr int kCdwRingKB = 160;
 constexpr int kCdwMaxSlots = 8;
 constexpr int kCdwLeast = 512;     // least points of a block
-// 32-point steps after which a wave adds its partial sums to the gradients and begins anew: an FP32 sum is
-// that much more exact than one over a whole range (the bias gradient of 1.4M rows was more than 1.5 times as
-// far from FP64 in ranges of 40,000 points than in 20,000).  Without it the FP32 kernel takes 1.22 ms.
-constexpr int kCdwFlush = 256;
+// 32-point steps after which a wave sets its partial sums aside and begins anew: an FP32 sum is that much more
+// exact than one over a whole range (the gradients of W3 and b3 over 1.4M rows, ranges of 40,000 points, were
+// more than 1.5 times as far from FP64 as sums over 20,000).  A wave of few tiles sets them aside in registers,
+// often; one of many, whose ranges are the shortest, adds them to the gradients.  The row sums, few numbers that
+// many points add up to, are compensated besides.
+constexpr int kCdwAside = 32;
+constexpr int kCdwFlush = 512;
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -89,8 +92,8 @@ struct Ring {
     wr = next(wr);
   }
   // load(slot byte offset of a half, operands) reads one half's operands; multiply(operands) runs its
-  // products; flush() adds the partial sums to the gradients and zeroes them.
-  template <typename Ops, typename Load, typename Mul, typename Flush>
+  // products; flush(last) sets the partial sums aside, or with last adds them all to the gradients.
+  template <int kFlush, typename Ops, typename Load, typename Mul, typename Flush>
   __device__ SRF_AI void run(Ops& o0, Ops& o1, Load&& load, Mul&& multiply, Flush&& flush) {
     wait_vmem_le(min(30, (min(slots - 1, steps) - 1) * 2 * n_mine));
     block_barrier();
@@ -109,11 +112,21 @@ struct Ring {
       load(rd, o0);  // (past the last step: a slot's old contents, unused)
       multiply(o1);
       __builtin_amdgcn_sched_barrier(0);
-      if ((st + 1) % kCdwFlush == 0 || st + 1 == steps) {
-        flush();
-        wait_vmem();  // the counted waits above are of copies alone
+      if ((st + 1) % kFlush == 0 || st + 1 == steps) {
+        flush(st + 1 == steps);
+        if (kFlush == kCdwFlush) wait_vmem();  // the counted waits above are of copies alone
       }
     }
+  }
+};
+
+// A compensated sum (Kahan).
+struct RowSum {
+  float sum = 0.f, c = 0.f;
+  __device__ SRF_AI void add(float v) {
+    const float y = v - c, t = sum + y;
+    c = (t - sum) - y;
+    sum = t;
   }
 };
 
@@ -122,15 +135,17 @@ template <int RM, int NC, int kStride>
 __device__ __forceinline__ void run_f32(const CdwJob& jb, int row0, int col0, bool sums, Ring& ring) {
   const int lane = threadIdx.x & 63, g = lane >> 4, j = lane & 15;
   struct Ops { f32x4 a[RM], b[NC]; } o0, o1;
-  f32x4 acc[RM][NC];
-  float rs[RM];
+  constexpr bool kAside = RM * NC <= 4;
+  f32x4 acc[RM][NC], aside[kAside ? RM : 1][kAside ? NC : 1];
+  RowSum rs[RM];
 #pragma unroll
-  for (int i = 0; i < RM; ++i) {
-    rs[i] = 0.f;
+  for (int i = 0; i < RM; ++i)
 #pragma unroll
-    for (int k = 0; k < NC; ++k) acc[i][k] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-  ring.run(
+    for (int k = 0; k < NC; ++k) {
+      acc[i][k] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (kAside) aside[i][k] = acc[i][k];
+    }
+  ring.run<kAside ? kCdwAside : kCdwFlush>(
       o0, o1,
       [&](uint32_t at, Ops& o) SRF_AI {
         const uint8_t* fr = ring.ring + at + lane * 16;
@@ -149,9 +164,19 @@ __device__ __forceinline__ void run_f32(const CdwJob& jb, int row0, int col0, bo
             for (int k = 0; k < NC; ++k) acc[i][k] = mfma32(o.a[i][q], o.b[k][q], acc[i][k]);
         if (sums)
 #pragma unroll
-          for (int i = 0; i < RM; ++i) rs[i] += (o.a[i][0] + o.a[i][1]) + (o.a[i][2] + o.a[i][3]);
+          for (int i = 0; i < RM; ++i) rs[i].add((o.a[i][0] + o.a[i][1]) + (o.a[i][2] + o.a[i][3]));
       },
-      [&]() SRF_AI {
+      [&](bool last) SRF_AI {
+        if constexpr (kAside) {
+#pragma unroll
+          for (int i = 0; i < RM; ++i)
+#pragma unroll
+            for (int k = 0; k < NC; ++k) {
+              aside[i][k] += acc[i][k];
+              acc[i][k] = last ? aside[i][k] : f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+          if (!last) return;
+        }
 #pragma unroll
         for (int i = 0; i < RM; ++i) {
 #pragma unroll
@@ -164,13 +189,12 @@ __device__ __forceinline__ void run_f32(const CdwJob& jb, int row0, int col0, bo
             }
             acc[i][k] = f32x4{0.f, 0.f, 0.f, 0.f};
           }
-          if (sums) {
-            float s = rs[i];
+          if (sums && last) {
+            float s = rs[i].sum;
             s += __shfl_xor(s, 16, 64);
             s += __shfl_xor(s, 32, 64);
             const int o = 16 * (row0 + i) + j;
             if (g == 0 && o < jb.M) unsafeAtomicAdd(jb.db + o, s);
-            rs[i] = 0.f;
           }
         }
       });
@@ -182,7 +206,7 @@ __device__ __forceinline__ void run_split(const CdwJob& jb, int rb, int cb0, boo
   const int lane = threadIdx.x & 63, h = lane >> 5, i32 = lane & 31;
   struct Ops { f32x4 a[2], b[NC][2]; } o0, o1;
   f32x16 acc[NC];
-  float rs = 0.f;
+  RowSum rs;
 #pragma unroll
   for (int k = 0; k < NC; ++k)
 #pragma unroll
@@ -199,7 +223,7 @@ __device__ __forceinline__ void run_split(const CdwJob& jb, int rb, int cb0, boo
     hi = u32x4{t[0][0], t[1][0], t[2][0], t[3][0]};
     lo = u32x4{t[0][1], t[1][1], t[2][1], t[3][1]};
   };
-  ring.run(
+  ring.run<kCdwFlush>(
       o0, o1,
       [&](uint32_t at, Ops& o) SRF_AI {
         const uint8_t* fr = ring.ring + at + at_lane;
@@ -226,10 +250,10 @@ __device__ __forceinline__ void run_split(const CdwJob& jb, int rb, int cb0, boo
                                                              __builtin_bit_cast(bf16x8, pr == 1 ? bl[k] : bh[k]),
                                                              acc[k], 0, 0, 0);
         if (sums)
-          rs += ((o.a[0][0] + o.a[0][1]) + (o.a[0][2] + o.a[0][3])) + ((o.a[1][0] + o.a[1][1]) + (o.a[1][2] + o.a[1][3]));
+          rs.add(((o.a[0][0] + o.a[0][1]) + (o.a[0][2] + o.a[0][3])) + ((o.a[1][0] + o.a[1][1]) + (o.a[1][2] + o.a[1][3])));
       },
       // 32x32 D layout: lane l, register r holds row 8 (r / 4) + 4 (l / 32) + (r mod 4), column l mod 32
-      [&]() SRF_AI {
+      [&](bool last) SRF_AI {
 #pragma unroll
         for (int k = 0; k < NC; ++k) {
           const int col = 32 * (cb0 + k) + i32;
@@ -240,11 +264,10 @@ __device__ __forceinline__ void run_split(const CdwJob& jb, int rb, int cb0, boo
             acc[k][r] = 0.f;
           }
         }
-        if (sums) {
-          const float s = rs + __shfl_xor(rs, 32, 64);
+        if (sums && last) {
+          const float s = rs.sum + __shfl_xor(rs.sum, 32, 64);
           const int o = 32 * rb + i32;
           if (h == 0 && o < jb.M) unsafeAtomicAdd(jb.db + o, s);
-          rs = 0.f;
         }
       });
 }
