@@ -331,27 +331,25 @@ __device__ __forceinline__ void staged_layer(f32x4 (&acc)[OUT][kCB], const float
   mlp::mma_tiles<P, NT, OUT, 0, kST>(acc, reinterpret_cast<const uint8_t*>(A), upr, 0, fin, stage);
 }
 
-// Positional-encoding input i of the first layer for one point, from its basis outputs F (LDS
-// column) and view direction (reference order: [F, sin(F), cos(F), sin(2F), ...], then the same
-// blocks of the direction).
-__device__ __forceinline__ float pe_input(const Geo& g, int i, const float* Fcol, int fstride, const float* dir) {
+// i / d for i < 1024 and d <= 64 (inv = 65536 / d + 1).
+__device__ __forceinline__ int small_div(int i, uint32_t inv) { return (int)(((uint32_t)i * inv) >> 16); }
+
+// Positional-encoding input i of the first layer for one point, from its basis outputs F and view direction
+// (LDS columns; reference order: [F, sin(F), cos(F), sin(2F), ...], then the same blocks of the direction).
+// The vector ALU evaluates 160 of these per point of the 300^2 network next to 43,500 multiply-adds, so: one
+// range reduction for whichever of sine and cosine a lane needs (the two as separate branches both run, the
+// lanes of a wave being at different i), and no integer division.
+__device__ __forceinline__ float pe_input(const Geo& g, int i, const float* Fcol, int fstride, const float* dcol,
+                                          int dstride, uint32_t inv_nb) {
   const int nf = g.NB * (2 * g.Lf + 1);
-  if (i < nf) {
-    const int b = i / g.NB, f = i - b * g.NB;
-    const float v = Fcol[f * fstride];
-    if (b == 0) return v;
-    const float x = __fmul_rn(v, (float)(1 << ((b - 1) >> 1)));
-    return (b & 1) ? sinf(x) : cosf(x);
-  }
-  if (g.view && i < g.D1) {
-    const int i2 = i - nf;
-    const int b = i2 / 3, d = i2 - 3 * b;
-    const float v = dir[d];
-    if (b == 0) return v;
-    const float x = __fmul_rn(v, (float)(1 << ((b - 1) >> 1)));
-    return (b & 1) ? sinf(x) : cosf(x);
-  }
-  return 0.f;
+  if (i >= g.D1) return 0.f;  // nf without the view directions
+  const bool feat = i < nf;
+  const int b = feat ? small_div(i, inv_nb) : small_div(i - nf, 65536 / 3 + 1);
+  const float v = feat ? Fcol[(i - b * g.NB) * fstride] : dcol[(i - nf - 3 * b) * dstride];
+  if (b == 0) return v;
+  float sn, cs;
+  sincosf(__fmul_rn(v, (float)(1 << ((b - 1) >> 1))), &sn, &cs);
+  return (b & 1) ? sn : cs;
 }
 
 struct FwdArgs {
@@ -403,8 +401,15 @@ __device__ __forceinline__ void load_tile_rows(const uint8_t* ws, size_t arr, in
   mlp::load_tile_f32(mlp::uniform_rsrc(ws + arr), blk_off(n_tiles, t, p0), v);
 }
 
+// Three waves per SIMD (51 KB of LDS a block, up to 168 registers): the products, the positional encoding and
+// the stores of different waves overlap.  1.4M rows in FP32 of the 300^2 network: 1.69 ms at two waves, 1.50 at
+// three; 300,000 rows of BF16 operands 107 and 102 us.  The split forward's stage (48 KB) allows two.
 template <int P>
-__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) void color_fwd_kernel(FwdArgs a) {
+constexpr int fwd_waves() { return P == kBFS3 ? 2 : 3; }
+
+template <int P>
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(fwd_waves<P>(), fwd_waves<P>()))) void color_fwd_kernel(
+    FwdArgs a) {
   __shared__ __attribute__((aligned(16))) uint8_t stage[stage_bytes<P>()];
   constexpr int KU = kunit<P>();
   __shared__ float sF[kWaves][kMaxB][kPW + 1];
@@ -469,15 +474,13 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2, 
     for (int cb = 0; cb < kCB; ++cb)
 #pragma unroll
       for (int r = 0; r < 4; ++r) h1[T][cb][r] = a.pk[g.b1 + 16 * T + 4 * gq + r];
+  const uint32_t inv_nb = 65536u / g.NB + 1;
   auto fin_pe = [&](int u, int cb) -> f32x4 {
     const int col = 16 * cb + j;
-    const float dir[3] = {sD[wv][0][col], sD[wv][1][col], sD[wv][2][col]};
     f32x4 b;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int i = 16 * u + 4 * gq + r;
-      b[r] = pe_input(g, i, &sF[wv][0][col], kPW + 1, dir);
-    }
+    for (int r = 0; r < 4; ++r)
+      b[r] = pe_input(g, 16 * u + 4 * gq + r, &sF[wv][0][col], kPW + 1, &sD[wv][0][col], kPW, inv_nb);
     return b;
   };
   auto keep_pe = [&](int u, const f32x4(&b)[kCB]) {
@@ -655,6 +658,7 @@ __device__ __forceinline__ void color_bwd_body(const BwdArgs& a) {
     }
   }
   const int nf = g.NB * (2 * g.Lf + 1);
+  const uint32_t inv_nb = 65536u / g.NB + 1;
   auto fin_dz1 = [&](int u, int cb) { return dz1[u][cb]; };
   auto dx_tiles = [&](auto OUTC, int T0) {
     constexpr int OUT = decltype(OUTC)::value;
@@ -670,7 +674,7 @@ __device__ __forceinline__ void color_bwd_body(const BwdArgs& a) {
       for (int r = 0; r < 4; ++r) {
         const int i = 16 * (T0 + T) + 4 * gq + r;
         if (i < nf) {
-          const int b = i / g.NB, f = i - b * g.NB;
+          const int b = small_div(i, inv_nb), f = i - b * g.NB;
 #pragma unroll
           for (int cb = 0; cb < kCB; ++cb) {
             const int col = 16 * cb + j;
@@ -691,6 +695,7 @@ __device__ __forceinline__ void color_bwd_body(const BwdArgs& a) {
   };
   int T0 = 0;
   for (; T0 + kST <= g.D1p / 16; T0 += kST) dx_tiles(std::integral_constant<int, kST>{}, T0);
+  for (; T0 + 2 <= g.D1p / 16; T0 += 2) dx_tiles(std::integral_constant<int, 2>{}, T0);
   for (; T0 < g.D1p / 16; ++T0) dx_tiles(std::integral_constant<int, 1>{}, T0);
   mlp::wave_lds_sync();  // the wave's dF rows, written by its lanes, are read across lanes below
   // 5) d_app = B^T dF (point-major, float4 per lane)
