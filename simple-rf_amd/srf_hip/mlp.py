@@ -177,8 +177,8 @@ def mlp_forward(spec: MLPSpec, weights, biases, pts: torch.Tensor, dirs: torch.T
         dirs = None
     if noise is not None:
         noise = dev_tensor(noise.reshape(-1), 'noise', (n,))
-    params = [None if spec.param_shapes()[i] is None else weights[i] for i in range(12)] + \
-             [None if spec.param_shapes()[i] is None else biases[i] for i in range(12)]
+    params = [weights[i] if spec.present(i) else None for i in range(12)] + \
+             [biases[i] if spec.present(i) else None for i in range(12)]
     train = torch.is_grad_enabled() and any(p is not None and p.requires_grad for p in params)
     return _MLPFunction.apply(spec, train, pts, dirs, noise, None, *params)
 
@@ -202,7 +202,7 @@ def mlp_forward_rays(spec: MLPSpec, weights, biases, rays_o: torch.Tensor, rays_
         view_dirs = None
     if noise is not None:
         noise = dev_tensor(noise.reshape(-1), 'noise', (r * s,))
-    params = [None if spec.param_shapes()[i] is None else weights[i] for i in range(12)] + \
-             [None if spec.param_shapes()[i] is None else biases[i] for i in range(12)]
+    params = [weights[i] if spec.present(i) else None for i in range(12)] + \
+             [biases[i] if spec.present(i) else None for i in range(12)]
     train = torch.is_grad_enabled() and any(p is not None and p.requires_grad for p in params)
     return _MLPFunction.apply(spec, train, None, view_dirs, noise, (rays_o, rays_d, z_vals), *params)
