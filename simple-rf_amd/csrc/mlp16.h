@@ -1,7 +1,7 @@
 // NeRF MLP forward and backward chain for 16-bit operands (BF16 training and inference, FP16
 // inference) on 32x32x16 MFMAs.  Plan, workspace and weight gradients are those of mlp_impl.h.
 //
-// Why 32x32: with one wave per SIMD (the accumulators take the whole AGPR file) a stream of
+// Why 32x32: with one wave per SIMD a stream of
 // independent 16x16x32 MFMAs on random operands reaches 1.40-1.50 PFLOP/s on this chip, the same
 // products as 32x32x16 MFMAs 1.79 PFLOP/s (1.58 and 2.49 on zeros: the larger shape also draws less
 // power per product).  4,096 rays x 192 samples, main model: training forward 1,705 us on 16x16x32 tiles,
@@ -677,6 +677,15 @@ template <int P, bool VD, bool TRAIN, int NB>
 int launch_fwd16(const FwdArgs& a, hipStream_t s) {
   hipLaunchKernelGGL((mlp16_fwd_kernel<P, VD, TRAIN, NB>), dim3(a.w.cols / (kWaves * 32 * NB)), dim3(64 * kWaves), 0, s, a);
   return launch_status();
+}
+
+// Inference of few points takes 128-point blocks while the compute units are enough for all of them: the call
+// takes as long as one block then (62 us for 256 points, 42 for 128; 16,384 points).  Beyond, a block streams its
+// weights for twice the points.
+template <int P, bool VD>
+int launch_infer16(const FwdArgs& a, hipStream_t s) {
+  return a.w.cols / (kWaves * 32) <= device_compute_units() ? launch_fwd16<P, VD, false, 1>(a, s)
+                                                            : launch_fwd16<P, VD, false, 2>(a, s);
 }
 
 template <int P, bool VD>

@@ -5,8 +5,8 @@ namespace srf {
 namespace mlp {
 
 int fwd_bf16(const FwdArgs& a, bool vd, bool tr, hipStream_t s) {
-  if (vd) return tr ? launch_fwd16<kBF16, true, true, 2>(a, s) : launch_fwd16<kBF16, true, false, 2>(a, s);
-  return tr ? launch_fwd16<kBF16, false, true, 2>(a, s) : launch_fwd16<kBF16, false, false, 2>(a, s);
+  if (tr) return vd ? launch_fwd16<kBF16, true, true, 2>(a, s) : launch_fwd16<kBF16, false, true, 2>(a, s);
+  return vd ? launch_infer16<kBF16, true>(a, s) : launch_infer16<kBF16, false>(a, s);
 }
 
 int bwd_bf16(const BwdArgs& a, bool vd, hipStream_t s) {

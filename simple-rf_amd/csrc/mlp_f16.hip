@@ -8,7 +8,7 @@ namespace mlp {
 
 int fwd_f16(const FwdArgs& a, bool vd, bool tr, hipStream_t s) {
   if (tr) return SRF_EUNSUPPORTED;
-  return vd ? launch_fwd16<kF16, true, false, 2>(a, s) : launch_fwd16<kF16, false, false, 2>(a, s);
+  return vd ? launch_infer16<kF16, true>(a, s) : launch_infer16<kF16, false>(a, s);
 }
 
 }  // namespace mlp

@@ -81,3 +81,19 @@ def test_gradients_add_up(cuda, variant, n, cut):
     whole, one, two = grads(slice(0, n)), grads(slice(0, cut)), grads(slice(cut, n))
     for x, y, z in zip(whole, one, two):
         assert (x - (y + z)).norm() <= n * 2.0 ** -24 * x.norm()
+
+
+@pytest.mark.parametrize('variant', list(VARIANTS))
+@pytest.mark.parametrize('prec', ['bf16', 'fp16'])
+def test_few_points_as_many(cuda, variant, prec):
+    """Inference of few points runs on 32-point waves while every block has a compute unit of its own (32,768
+    points on 256), and on 64-point waves beyond: the same values, to the bit."""
+    spec = hm.MLPSpec(prec=prec, **VARIANTS[variant]['spec'])
+    w, b = leaves(spec, cuda)
+    most = 128 * torch.cuda.get_device_properties(cuda).multi_processor_count
+    pts, dirs = (t.to(cuda) for t in points(most + 300, 26))
+    with torch.no_grad():
+        sig, rgb = hm.mlp_forward(spec, w, b, pts, dirs)
+        for n in (1, 33, 129, most - 1, most, most + 1):
+            s, c = hm.mlp_forward(spec, w, b, pts[:n], dirs[:n])
+            assert torch.equal(s, sig[:n]) and torch.equal(c, rgb[:n]), n
