@@ -297,17 +297,17 @@ __device__ __forceinline__ void quad_products(const VmArgs& a, const WaveSites& 
   }
 }
 
-// f(products, planes, first step) over all steps of a group, three at a time while there are that many.
-template <int G, bool kUniform, typename F>
+// f(products, plane, quad) over all steps of a group, kAtOnce at a time while there are that many.
+template <int G, bool kUniform, int kAtOnce, typename F>
 __device__ __forceinline__ void for_quads(const VmArgs& a, const WaveSites& ws, int slot, int ql, F&& f) {
   const int steps = (a.n_quads + G - 1) / G;
   int st = 0;
-  for (; st + 3 <= steps; st += 3) {
-    float4 o[3];
-    int pl[3];
-    quad_products<G, 3, kUniform>(a, ws, slot, ql + G * st, o, pl);
+  for (; st + kAtOnce <= steps; st += kAtOnce) {
+    float4 o[kAtOnce];
+    int pl[kAtOnce];
+    quad_products<G, kAtOnce, kUniform>(a, ws, slot, ql + G * st, o, pl);
 #pragma unroll
-    for (int t = 0; t < 3; ++t) f(o[t], pl[t], ql + G * (st + t));
+    for (int t = 0; t < kAtOnce; ++t) f(o[t], pl[t], ql + G * (st + t));
   }
   for (; st < steps; ++st) {
     float4 o[1];
@@ -399,8 +399,11 @@ __device__ __forceinline__ GroupPos group_pos() {
 // had no quad, and a branch per tap put its six loads one after the other.  Now a lane prepares one sample,
 // only the valid ones are packed for the groups, and a group is small enough that its lanes have several
 // quads (with G = 4 in the equal configurations all lanes work).  3.6M samples of 3 x 16 components under an
-// alpha mask: 658 -> 164 us; 1.45M rows of 3 x 48: 707 -> 372 us (of which 835 MB of rows written).
+// alpha mask: 658 -> 140 us; 1.45M rows of 3 x 48: 707 -> 372 us (of which 835 MB of rows written).
 constexpr int kFwdWaves = 256 / SRF_WAVE;
+// Quads of a lane at once: the density keeps more waves with one (86 registers against 136), the appearance rows, whose
+// stores wait on nothing, take three.  1, 2, 3: 140, 144, 161 us and 433, 390, 372 us at the shapes above.
+constexpr int kDensityAtOnce = 1, kAppearanceAtOnce = 3;
 
 template <int G, bool kUniform>
 __global__ __launch_bounds__(256) void density_fwd_kernel(VmArgs a, AlphaArgs m, int64_t n,
@@ -429,7 +432,7 @@ __global__ __launch_bounds__(256) void density_fwd_kernel(VmArgs a, AlphaArgs m,
     for (int k0 = 0; k0 < count; k0 += SRF_WAVE / G) {  // uniform: whole groups stay converged
       const int k = k0 + lane / G;
       float s[kPlanes] = {0.f, 0.f, 0.f};
-      for_quads<G, kUniform>(a, sites[wv], min(k, count - 1), lane % G, [&](float4 v, int pl, int q) {
+      for_quads<G, kUniform, kDensityAtOnce>(a, sites[wv], min(k, count - 1), lane % G, [&](float4 v, int pl, int q) {
         const float d = kUniform || q < a.n_quads ? sum4(v) : 0.f;
         s[0] = pl == 0 ? __fadd_rn(s[0], d) : s[0];
         s[1] = pl == 1 ? __fadd_rn(s[1], d) : s[1];
@@ -652,7 +655,7 @@ __global__ __launch_bounds__(256) void appearance_fwd_kernel(VmArgs a, int64_t n
     wave_lds_fence();
     for (int k0 = 0; k0 < count; k0 += SRF_WAVE / G) {
       const int k = k0 + lane / G;
-      for_quads<G, kUniform>(a, sites[wv], min(k, count - 1), lane % G, [&](float4 v, int, int q) {
+      for_quads<G, kUniform, kAppearanceAtOnce>(a, sites[wv], min(k, count - 1), lane % G, [&](float4 v, int, int q) {
         if (k < count && (kUniform || q < a.n_quads))
           *reinterpret_cast<float4*>(out + (base + k) * a.total_comp + 4 * q) = v;
       });
