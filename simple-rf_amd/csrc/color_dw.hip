@@ -120,12 +120,13 @@ struct Ring {
   }
 };
 
-// A compensated sum (Kahan).
+// A compensated sum (Kahan).  An infinite sum has nothing to compensate: inf - inf would turn it into NaN at the
+// next term.
 struct RowSum {
   float sum = 0.f, c = 0.f;
   __device__ SRF_AI void add(float v) {
     const float y = v - c, t = sum + y;
-    c = (t - sum) - y;
+    c = __builtin_isinf(t) ? 0.f : (t - sum) - y;
     sum = t;
   }
 };
