@@ -356,7 +356,11 @@ static int weight_grads16(const Plan& p, const Ws& w, uint8_t* ws, float* const*
   // adds 256 KB with atomics); 262,144 points 517, 523, 550; 786,432 points 1,495, 1,440, 1,436 (a second
   // round evens out the compute units).  16,384 points 87 us with 512 points a block, 79 with 1,024, 82
   // with 1,536.
-  constexpr int kStep = 6, kLeast = 1024, kLong = 20000;
+  // The running FP32 sums end earlier than a long block: those of many tiles after kSums points, in the
+  // gradients, those of few (kDwNarrow, kDwRow, whose blocks are the longest) after kAside, in registers.  The
+  // gradient of the rgb layer over 786,432 points was 2.8e-7 off the FP64 sum with sums over whole blocks, 1.4e-7
+  // with these; over 3,145,728 points 1.0e-6 and 2.3e-7.
+  constexpr int kStep = 6, kLeast = 1024, kLong = 20000, kSums = 16384, kAside = 1024;
   auto cost = [](const Dw16Job& j) { return j.n_dz + j.n_x + j.n_x2 + kStep; };
   const int64_t tuned = tune_value(SRF_TUNE_DW_CHUNK);  // points of a block of a 256 x 256 layer
   double per_block = 0.;                                // points x cost
@@ -373,6 +377,7 @@ static int weight_grads16(const Plan& p, const Ws& w, uint8_t* ws, float* const*
       j.first_block = blocks;
       j.chunk = (int)(per_block / cost(j)) / 64 * 64;
       if (j.chunk < kLeast) j.chunk = kLeast;
+      j.segment = j.kind == kDwNarrow || j.kind == kDwRow ? kAside : dw_segment(j.chunk, kSums);
       blocks += (w.cols + j.chunk - 1) / j.chunk;
     }
     // (the jobs' last, partly filled blocks: no more than whole rounds)
@@ -462,11 +467,13 @@ static int mlp_backward_impl(const srf_mlp_desc* desc, const void* packed, int n
     job(w.dz[8], 0, 16, w.h[7], 256, 4, 256, d_weights[9], 256, d_biases[9]);
   }
   d.n_jobs = nj;
-  // points per work item: whole rounds of resident blocks (dw_default_chunk), whole multiples of
-  // 256 points (so every item holds an even number of k-units), between 2048 and 262144 points
-  long long target = dw_default_chunk(w.cols, nj, device_compute_units());
-  if (const int64_t v = tune_value(SRF_TUNE_DW_CHUNK)) target = v;  // autotuned schedule
+  // points per work item (dw_schedule), whole multiples of 256 points (so every item holds an even number
+  // of k-units), between 2048 and 262144 points
+  const DwSchedule plan = dw_schedule(w.cols, nj, device_compute_units());
+  const int64_t tuned = tune_value(SRF_TUNE_DW_CHUNK);  // autotuned schedule
+  const long long target = tuned ? tuned : plan.chunk;
   d.chunk = (int)(target < 2048 ? 2048 : (target > 262144 ? 262144 : target));
+  d.segment = tuned ? dw_segment(d.chunk, plan.segment) : plan.segment;
   d.n_chunks = (w.cols + d.chunk - 1) / d.chunk;
   int work = 0;
   for (int i = 0; i < nj; ++i) {

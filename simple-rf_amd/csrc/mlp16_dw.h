@@ -46,6 +46,7 @@ struct Dw16Job {
   float* db;
   float* db_row;
   int chunk;           // points per block, a multiple of 64
+  int segment;         // points after which the block adds its sums to the gradients and begins anew (of 64)
   int first_block;
 };
 

@@ -16,7 +16,7 @@ __device__ __forceinline__ void dw16_run(const Dw16Args& a, const Dw16Job& jb, i
   const int slots = min(kDw16MaxSlots, kDw16Lds / n_frag);
   const int slot_bytes = n_frag * 1024;
   const int pb = (blockIdx.x - jb.first_block) * jb.chunk;
-  const int units = (min(pb + jb.chunk, a.cols) - pb) / 32;
+  const int units = (min(pb + jb.chunk, a.cols) - pb) / 32, seg_units = jb.segment / 32;
 
   // This wave's fragments of a unit: f = w, w + 8, ...  LDS position l of a fragment (16 B) takes chunk
   // k = (l >> 1) & 1 of record (l & 1, c) with c = 16 (unit % 2) + 8 s + 4 h' + d, where d = l >> 4, h' = (l >> 2)
@@ -50,13 +50,18 @@ __device__ __forceinline__ void dw16_run(const Dw16Args& a, const Dw16Job& jb, i
   };
   for (int u = 0; u < slots - 1 && u < units; ++u) fill();
 
-  f32x16 acc[RM][NB], row_acc;
+  // Sums of few tiles are set aside in registers, those of many added to the gradients, after jb.segment points.
+  constexpr bool kAside = RM * NB <= 2;
+  f32x16 acc[RM][NB], aside[kAside ? RM : 1][kAside ? NB : 1], row_acc;
 #pragma unroll
   for (int i = 0; i < RM; ++i)
 #pragma unroll
     for (int k = 0; k < NB; ++k)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][k][r] = 0.f;
+      for (int r = 0; r < 16; ++r) {
+        acc[i][k][r] = 0.f;
+        if constexpr (kAside) aside[i][k][r] = 0.f;
+      }
 #pragma unroll
   for (int r = 0; r < 16; ++r) row_acc[r] = 0.f;
   float rs[NA];
@@ -102,6 +107,54 @@ __device__ __forceinline__ void dw16_run(const Dw16Args& a, const Dw16Job& jb, i
       if (w == 0) add_rows(av[RM], rs[RM]);
   };
 
+  // adds the block's sums: D register r holds row 8 (r / 4) + 4 h + r % 4, column i32 of a tile
+  auto add_sums = [&](bool last) SRF_AI {
+    if constexpr (kAside) {
+#pragma unroll
+      for (int i = 0; i < RM; ++i)
+#pragma unroll
+        for (int k = 0; k < NB; ++k)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            aside[i][k][r] += acc[i][k][r];
+            acc[i][k][r] = last ? aside[i][k][r] : 0.f;
+          }
+      if (!last) return;
+    }
+    const int at = (int)lane_here(), h = at >> 5, i32 = at & 31;
+#pragma unroll
+    for (int i = 0; i < RM; ++i)
+#pragma unroll
+      for (int k = 0; k < NB; ++k) {
+        const int ct = k < NC ? col0 + k : colx + 2 * (k - NC);
+        const bool ext = k >= NC;
+        const int c = 32 * (ext ? ct - 8 : ct) + i32;
+        float* dst = ext ? jb.dw2 : jb.dw;
+        const int n = ext ? jb.N2 : jb.N;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int o = 32 * (row0 + i) + 8 * (r >> 2) + 4 * h + (r & 3);
+          if (o < jb.M && c < n) unsafeAtomicAdd(dst + (size_t)o * jb.ld + c, acc[i][k][r]);
+          acc[i][k][r] = 0.f;
+        }
+      }
+    if constexpr (ROW) {
+      if (h == 0) unsafeAtomicAdd(jb.dw_row + 32 * (col0 + row0 / 2) + i32, row_acc[0]);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) row_acc[r] = 0.f;
+    }
+    if (sums && last) {
+      const float s = rs[0] + __shfl_xor(rs[0], 32, 64);
+      const int o = 32 * (row0 + my_sum) + i32;
+      if (h == 0 && o < jb.M) unsafeAtomicAdd(jb.db + o, s);
+    }
+    if constexpr (ROW)
+      if (w == 0 && last) {
+        const float s = rs[RM] + __shfl_xor(rs[RM], 32, 64);
+        if (lane == 0) unsafeAtomicAdd(jb.db_row, s);
+      }
+  };
+
   u32x4 a0[NA], b0[NB], x0 = {0u, 0u, 0u, 0u}, a1[NA], b1[NB], x1 = {0u, 0u, 0u, 0u};
   uint32_t rd = 0;
   // unit 0 (and the others of the prologue that every wave has waited for)
@@ -109,7 +162,7 @@ __device__ __forceinline__ void dw16_run(const Dw16Args& a, const Dw16Job& jb, i
   block_barrier();
   load(0, 0, a0, b0, x0);
 #pragma unroll 1
-  for (int u = 0; u < units; ++u) {
+  for (int u = 0, stop = min(seg_units, units); u < units; ++u) {
     // unit u + 1 has landed once only the units copied after it are outstanding; the barrier makes every
     // wave's part visible and frees the slot of unit u - 1, whose operands are all in registers
     const int after = min(slots - 3, units - 2 - u);
@@ -123,36 +176,12 @@ __device__ __forceinline__ void dw16_run(const Dw16Args& a, const Dw16Job& jb, i
     load(rd, 0, a0, b0, x0);  // (past the last unit: a slot's old contents, unused)
     multiply(a1, b1, x1);
     __builtin_amdgcn_sched_barrier(0);
-  }
-
-  // add the block's sums: D register r holds row 8 (r / 4) + 4 h + r % 4, column i32 of a tile
-#pragma unroll
-  for (int i = 0; i < RM; ++i)
-#pragma unroll
-    for (int k = 0; k < NB; ++k) {
-      const int ct = k < NC ? col0 + k : colx + 2 * (k - NC);
-      const bool ext = k >= NC;
-      const int c = 32 * (ext ? ct - 8 : ct) + i32;
-      float* dst = ext ? jb.dw2 : jb.dw;
-      const int n = ext ? jb.N2 : jb.N;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int o = 32 * (row0 + i) + 8 * (r >> 2) + 4 * h + (r & 3);
-        if (o < jb.M && c < n) unsafeAtomicAdd(dst + (size_t)o * jb.ld + c, acc[i][k][r]);
-      }
+    if (u + 1 == stop) {
+      add_sums(u + 1 == units);
+      stop = min(stop + seg_units, units);
+      if (!kAside && u + 1 < units) wait_vmem();  // the counted waits above are of copies alone
     }
-  if constexpr (ROW)
-    if (h == 0) unsafeAtomicAdd(jb.dw_row + 32 * (col0 + row0 / 2) + i32, row_acc[0]);
-  if (sums) {
-    const float s = rs[0] + __shfl_xor(rs[0], 32, 64);
-    const int o = 32 * (row0 + my_sum) + i32;
-    if (h == 0 && o < jb.M) unsafeAtomicAdd(jb.db + o, s);
   }
-  if constexpr (ROW)
-    if (w == 0) {
-      const float s = rs[RM] + __shfl_xor(rs[RM], 32, 64);
-      if (lane == 0) unsafeAtomicAdd(jb.db_row, s);
-    }
 }
 
 __global__ __launch_bounds__(64 * kDwWaves) void mlp16_dw_kernel(Dw16Args a) {

@@ -1127,21 +1127,23 @@ struct DwJob {
 // multiples of 256 points, at least 2048.  One block (160 KB of LDS) is resident per CU, so a
 // launch costs about (rounds of `cus` blocks) x (per-block time), and a last, partly filled round
 // costs as much as a full one.  The per-block time is modelled as the chunk plus a fixed
-// overhead worth kDwBlockOverhead points (the tile's FP32 atomics and the ring's fill); the
-// chunk minimising rounds x that time over 1..8 rounds is chosen.  The blocks of a launch take about equally
-// long (every tile's products run, valid or not), so one round wastes nothing: backwards of 93,391 points in
-// split BF16 1.07 ms from 3 rounds on, 1.02 from 1 on; 60,000 points in FP32 1.87 and 1.72; 262,144 the same.
+// overhead worth kDwBlockOverhead points for each part of it (the tile's FP32 atomics and the ring's
+// fill); the chunk minimising rounds x that time over first..last rounds is chosen.
 constexpr int kDwBlockOverhead = 640;
-inline int dw_default_chunk(int cols, int nj, int cus) {
+inline long long dw_cost(int cols, int nj, int cus, int chunk, int parts) {
+  const long long blocks = (long long)nj * ((cols + chunk - 1) / chunk);
+  return (blocks + cus - 1) / cus * (chunk + (long long)parts * kDwBlockOverhead);
+}
+inline int dw_parts(int chunk, int longest) { return (chunk + longest - 1) / longest; }
+inline int dw_chunk(int cols, int nj, int cus, int first, int last, int longest) {
   long long best_cost = -1;
   int best = 2048;
-  for (int rounds = 1; rounds <= 8; ++rounds) {
+  for (int rounds = first; rounds <= last; ++rounds) {
     const int max_chunks = rounds * cus / (nj > 0 ? nj : 1);
     if (max_chunks < 1) continue;
     int chunk = round_up((cols + max_chunks - 1) / max_chunks, 256);
     if (chunk < 2048) chunk = 2048;
-    const long long blocks = (long long)nj * ((cols + chunk - 1) / chunk);
-    const long long cost = (blocks + cus - 1) / cus * (long long)(chunk + kDwBlockOverhead);
+    const long long cost = dw_cost(cols, nj, cus, chunk, dw_parts(chunk, longest));
     if (best_cost < 0 || cost < best_cost) {
       best_cost = cost;
       best = chunk;
@@ -1150,9 +1152,35 @@ inline int dw_default_chunk(int cols, int nj, int cus) {
   return best;
 }
 
+// A block's chunk is long where whole rounds of blocks ask for it, its running FP32 sums are not: a block of
+// more than `longest` points adds its sums to the gradients after equal parts of at most that many (multiples
+// of 64) and begins anew.
+inline int dw_segment(int chunk, int longest) {
+  const int parts = dw_parts(chunk, longest);
+  return round_up((chunk + parts - 1) / parts, 64);
+}
+
+// Chunk and segment of the FP32 and split-BF16 kernels.  The running sums are as long as the chunk of three or
+// more rounds is; the blocks take about equally long (every tile's products run, valid or not), so one or two
+// rounds of longer blocks waste nothing where they cost less.  Running sums over whole blocks of one round were up
+// to three times as far from FP64: the weight gradients of 262,144 points of the main model 3.3e-7 in FP32 and
+// 3.9e-7 in split BF16, 1.6e-7 and 1.7e-7 with segments.  Backward of 60,000 points in FP32, three rounds, one of
+// whole blocks, one of segments: 1.80, 1.65, 1.70 ms; of 93,391 in split BF16 1.06, 1.01, 1.04.
+struct DwSchedule {
+  int chunk, segment;
+};
+inline DwSchedule dw_schedule(int cols, int nj, int cus) {
+  const int longest = dw_chunk(cols, nj, cus, 3, 8, cols);
+  const int chunk = dw_chunk(cols, nj, cus, 1, 2, longest);
+  return dw_cost(cols, nj, cus, chunk, dw_parts(chunk, longest)) <= dw_cost(cols, nj, cus, longest, 1)
+             ? DwSchedule{chunk, dw_segment(chunk, longest)}
+             : DwSchedule{longest, longest};
+}
+
 struct DwArgs {
   DwJob jobs[kMaxJobs];
   int n_jobs, ldP, cols, chunk, n_chunks, total_work;
+  int segment;  // points after which a block adds its sums to the gradients and begins anew
   // dZ / X layout: 0 plain feature-major rows; 1 the paired tile blocks of store_tile
   int paired;
   // optional device-side point count: only the columns below it, rounded up to whole 256-point
@@ -1207,16 +1235,6 @@ __global__ __launch_bounds__(64 * kDwWaves) void mlp_dw_kernel(DwArgs a) {
   constexpr int ELEM = 4;
   constexpr int KPTS = 16;  // points per k-unit
   const int qm = RM * (w >> 1), qn = NC * (w & 1);
-  bool mv[RM], nv[NC];
-#pragma unroll
-  for (int i = 0; i < RM; ++i) mv[i] = m0 + 16 * (qm + i) < jb.dz_rows;
-#pragma unroll
-  for (int k = 0; k < NC; ++k) nv[k] = n0 + 16 * (qn + k) < jb.x_rows;
-  bool any_m = false, any_n = false;
-#pragma unroll
-  for (int i = 0; i < RM; ++i) any_m |= mv[i];
-#pragma unroll
-  for (int k = 0; k < NC; ++k) any_n |= nv[k];
   // DMA of the 32 fragments of the k-unit at point p into a ring slot: fragment f < 16 is dZ row
   // tile f, f >= 16 is X row tile f - 16; wave w copies f = w, w + 8, w + 16, w + 24.  Every wave
   // issues exactly four loads per k-unit (a tile beyond the job's rows re-reads its first row
@@ -1256,14 +1274,37 @@ __global__ __launch_bounds__(64 * kDwWaves) void mlp_dw_kernel(DwArgs a) {
     for (int k = 0; k < NC; ++k) acc[i][k] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   const bool do_db = jb.db != nullptr && n0 == 0 && qn == 0;
-  const bool busy = any_m && (any_n || do_db);
-  const int n_units = (pe - pb) / KPTS;
+  const bool busy = m0 + 16 * qm < jb.dz_rows && (n0 + 16 * qn < jb.x_rows || do_db);  // any tile inside the job
+  const int n_units = (pe - pb) / KPTS, seg_units = a.segment / KPTS;
+  auto add_sums = [&](bool last) SRF_AI {
+    const int at = (int)lane_here(), g = at >> 4, j = at & 15;
+#pragma unroll
+    for (int i = 0; i < RM; ++i) {
+#pragma unroll
+      for (int k = 0; k < NC; ++k) {
+        const int c = n0 + 16 * (qn + k) + j;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int o = m0 + 16 * (qm + i) + 4 * g + r;
+          if (o < jb.M && c < jb.N) unsafeAtomicAdd(jb.dw + (size_t)o * jb.ld_dw + c, acc[i][k][r]);
+        }
+        acc[i][k] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+      if (do_db && last) {
+        float sr = rs[i];
+        sr += __shfl_xor(sr, 16, 64);
+        sr += __shfl_xor(sr, 32, 64);
+        const int o = m0 + 16 * (qm + i) + j;
+        if (g == 0 && o < jb.M) unsafeAtomicAdd(jb.db + o, sr);
+      }
+    }
+  };
   // prologue: k-units 0 .. kDwSlots - 2 in flight
 #pragma unroll
   for (int u = 0; u < kDwSlots - 1; ++u)
     if (u < n_units) dma_unit(pb + u * KPTS, ring + u * kDwSlot);
 #pragma unroll 1
-  for (int u = 0; u < n_units; ++u) {
+  for (int u = 0, stop = min(seg_units, n_units); u < n_units; ++u) {
     // k-unit u has landed once at most (issued after it) k-units' loads are outstanding
     const int after = min(kDwSlots - 2, n_units - 1 - u);
     static_assert(kDwSlots <= 5, "waits below cover up to three k-units in flight after u");
@@ -1301,26 +1342,10 @@ __global__ __launch_bounds__(64 * kDwWaves) void mlp_dw_kernel(DwArgs a) {
 #pragma unroll
         for (int i = 0; i < RM; ++i) rs[i] += (av[i][0] + av[i][1]) + (av[i][2] + av[i][3]);
     }
-  }
-#pragma unroll
-  for (int i = 0; i < RM; ++i) {
-    if (!mv[i]) continue;
-#pragma unroll
-    for (int k = 0; k < NC; ++k) {
-      if (!nv[k]) continue;
-      const int c = n0 + 16 * (qn + k) + j;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int o = m0 + 16 * (qm + i) + 4 * g + r;
-        if (o < jb.M && c < jb.N) unsafeAtomicAdd(jb.dw + (size_t)o * jb.ld_dw + c, acc[i][k][r]);
-      }
-    }
-    if (do_db) {
-      float sr = rs[i];
-      sr += __shfl_xor(sr, 16, 64);
-      sr += __shfl_xor(sr, 32, 64);
-      const int o = m0 + 16 * (qm + i) + j;
-      if (g == 0 && o < jb.M) unsafeAtomicAdd(jb.db + o, sr);
+    if (u + 1 == stop) {
+      add_sums(u + 1 == n_units);
+      stop = min(stop + seg_units, n_units);
+      if (u + 1 < n_units) wait_vmem();  // the counted waits above are of copies alone
     }
   }
 }
@@ -1358,11 +1383,6 @@ __global__ __launch_bounds__(64 * kDwWaves) void mlp_dw_split_kernel(DwArgs a) {
   const size_t ldP = a.ldP;
   constexpr int KPTS = 16;
   const int qm = 4 * (w >> 1), qn = 8 * (w & 1);  // first 16-row / 16-column tile of the wave
-  bool mv[2], nv[4];  // 32-row / 32-column blocks with data (their first 16-row tile inside the job)
-#pragma unroll
-  for (int b = 0; b < 2; ++b) mv[b] = m0 + 16 * (qm + 2 * b) < jb.dz_rows;
-#pragma unroll
-  for (int b = 0; b < 4; ++b) nv[b] = n0 + 16 * (qn + 2 * b) < jb.x_rows;
   // DMA of one 16-point unit: the 16 dZ and 16 X fragments of the tile, as in mlp_dw_kernel (a row
   // tile beyond the job's rows re-reads its first tile, so every wave issues four loads per unit)
   auto dma_unit = [&](int p, uint8_t* buf) SRF_AI {
@@ -1390,11 +1410,8 @@ __global__ __launch_bounds__(64 * kDwWaves) void mlp_dw_split_kernel(DwArgs a) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[rb][cb][r] = 0.f;
   const bool do_db = jb.db != nullptr && n0 == 0 && qn == 0;
-  bool any_m = mv[0] || mv[1], any_n = false;
-#pragma unroll
-  for (int b = 0; b < 4; ++b) any_n |= nv[b];
-  const bool busy = any_m && (any_n || do_db);
-  const int n_units = (pe - pb) / KPTS;
+  const bool busy = m0 + 16 * qm < jb.dz_rows && (n0 + 16 * qn < jb.x_rows || do_db);  // any block inside the job
+  const int n_units = (pe - pb) / KPTS, seg_units = a.segment / KPTS;
   // two BF16 planes of the eight FP32 values lane (h, i) takes from fragment f: records 2h, 2h + 1
   // of its lane group pair
   auto planes = [&](const uint8_t* fr, int f, u32x4& hi, u32x4& lo, float* sum) SRF_AI {
@@ -1410,11 +1427,32 @@ __global__ __launch_bounds__(64 * kDwWaves) void mlp_dw_split_kernel(DwArgs a) {
     lo = u32x4{t[0][1], t[1][1], t[2][1], t[3][1]};
     if (sum) *sum += ((v0[0] + v0[1]) + (v0[2] + v0[3])) + ((v1[0] + v1[1]) + (v1[2] + v1[3]));
   };
+  auto add_sums = [&](bool last) SRF_AI {
+    const int at = (int)lane_here(), h = at >> 5, i32 = at & 31;
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb) {
+#pragma unroll
+      for (int cb = 0; cb < 4; ++cb) {
+        const int c = n0 + 16 * qn + 32 * cb + i32;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int o = m0 + 16 * qm + 32 * rb + 8 * (r >> 2) + 4 * h + (r & 3);
+          if (o < jb.M && c < jb.N) unsafeAtomicAdd(jb.dw + (size_t)o * jb.ld_dw + c, acc[rb][cb][r]);
+          acc[rb][cb][r] = 0.f;
+        }
+      }
+      if (do_db && last) {
+        const float sr = rs[rb] + __shfl_xor(rs[rb], 32, 64);
+        const int o = m0 + 16 * qm + 32 * rb + i32;
+        if (h == 0 && o < jb.M) unsafeAtomicAdd(jb.db + o, sr);
+      }
+    }
+  };
 #pragma unroll
   for (int u = 0; u < kDwSlots - 1; ++u)
     if (u < n_units) dma_unit(pb + u * KPTS, ring + u * kDwSlot);
 #pragma unroll 1
-  for (int u = 0; u < n_units; ++u) {
+  for (int u = 0, stop = min(seg_units, n_units); u < n_units; ++u) {
     const int after = min(kDwSlots - 2, n_units - 1 - u);
     if (after >= 3) __builtin_amdgcn_s_waitcnt(vmcnt_only(12));
     else if (after == 2) __builtin_amdgcn_s_waitcnt(vmcnt_only(8));
@@ -1446,24 +1484,10 @@ __global__ __launch_bounds__(64 * kDwWaves) void mlp_dw_split_kernel(DwArgs a) {
                 __builtin_bit_cast(bf16x8, pr == 0 ? al[rb] : ah[rb]),
                 __builtin_bit_cast(bf16x8, pr == 1 ? bl[cb] : bh[cb]), acc[rb][cb], 0, 0, 0);
     }
-  }
-#pragma unroll
-  for (int rb = 0; rb < 2; ++rb) {
-    if (!mv[rb]) continue;
-#pragma unroll
-    for (int cb = 0; cb < 4; ++cb) {
-      if (!nv[cb]) continue;
-      const int c = n0 + 16 * qn + 32 * cb + i32;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int o = m0 + 16 * qm + 32 * rb + 8 * (r >> 2) + 4 * h + (r & 3);
-        if (o < jb.M && c < jb.N) unsafeAtomicAdd(jb.dw + (size_t)o * jb.ld_dw + c, acc[rb][cb][r]);
-      }
-    }
-    if (do_db) {
-      const float sr = rs[rb] + __shfl_xor(rs[rb], 32, 64);
-      const int o = m0 + 16 * qm + 32 * rb + i32;
-      if (h == 0 && o < jb.M) unsafeAtomicAdd(jb.db + o, sr);
+    if (u + 1 == stop) {  // as in mlp_dw_kernel
+      add_sums(u + 1 == n_units);
+      stop = min(stop + seg_units, n_units);
+      if (u + 1 < n_units) wait_vmem();
     }
   }
 }
