@@ -42,6 +42,33 @@ struct CdwArgs {
   const int32_t* cols_dev;
 };
 
+// Tiles that each wave of a block multiplies, of 16 x 16 (FP32) or 32 x 32 entries (split).  At most two row
+// tiles: the eight waves share the columns, column tile w + 8 k or column block w going to wave w.  More: waves
+// 2 r and 2 r + 1 (FP32) or r and r + 4 (split) take row tiles 2 r, 2 r + 1 or row block r, and half of the
+// columns each.  The kernel has exactly these forms, each without a branch between its products, and the costs
+// below are theirs.  (With FP32 forms of 4, 5 and 8 column tiles alone, whatever the product had, but costs of
+// its own, the first layer of the network without encoding, two tiles, was charged 800 cycles per 16 points and
+// took 2,250, and set the launch's time.  Backward of 1.4M rows of 72 components: 3.05 ms then,
+// 2.44 before there were costs, 1.77 here.)
+struct CdwForm {
+  int rows, cols;
+};
+template <bool SPLIT>
+__host__ __device__ constexpr CdwForm cdw_form(int nA, int nB) {
+  if (nA <= 2) return SPLIT ? CdwForm{1, 1} : CdwForm{nA, (nB + 7) / 8};
+  return SPLIT ? CdwForm{1, (nB + 3) / 4} : CdwForm{2, (nB + 1) / 2};
+}
+
+// Cost of 16 points to a block, in cycles: the MFMAs of its busiest SIMD (two waves) or the reads, and the
+// step itself.  The reads' share and the step's were swept (1.4M rows FP32, 300,000 rows split, us):
+// 104 / 200 1306, 205; 80 / 200 1252, 204; 60 / 200 1215, 208; 60 / 50 1258, 211; 40 / 100 1219, 225.
+template <bool SPLIT>
+__host__ __device__ constexpr int cdw_cost(int nA, int nB) {
+  const CdwForm f = cdw_form<SPLIT>(nA, nB);
+  const int mfma = (SPLIT ? 512 : 256) * f.rows * f.cols, reads = (SPLIT ? 90 : 60) * (nA + nB);
+  return (mfma > reads ? mfma : reads) + 200;
+}
+
 int cdw_launch(const CdwArgs& a, bool split, hipStream_t s);
 
 }  // namespace color

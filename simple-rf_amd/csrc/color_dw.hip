@@ -22,17 +22,6 @@ constexpr int kCdwFlush = 512;
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-// Cost of 16 points to a block, in cycles: the MFMAs of its busiest SIMD (two waves) or the reads, and the
-// step itself.  The reads' share and the step's were swept (1.4M rows FP32, 300,000 rows split, us):
-// 104 / 200 1306, 205; 80 / 200 1252, 204; 60 / 200 1215, 208; 60 / 50 1258, 211; 40 / 100 1219, 225.
-template <bool SPLIT>
-__device__ __forceinline__ int job_cost(int nA, int nB) {
-  const int thin = nA <= 2;
-  const int tiles = SPLIT ? (thin ? 1 : (nB + 3) / 4) : (thin ? (nB > 8 ? 2 : 1) : (nB + 1) / 2);
-  const int mfma = SPLIT ? 512 * tiles : (thin && nA == 1 ? 256 : 512) * tiles;
-  return max(mfma, (SPLIT ? 90 : 60) * (nA + nB)) + 200;
-}
-
 // s_waitcnt vmcnt(n) for a wave-uniform n, at most 47.
 __device__ __forceinline__ void wait_vmem_le(int n) {
   switch (n) {
@@ -279,43 +268,59 @@ __global__ __launch_bounds__(64 * kCdwWaves) void color_dw_kernel(CdwArgs a) {
   const int cols = a.cols_dev ? min(a.cols, (*a.cols_dev + 255) / 256 * 256) : a.cols;
   // the block's product and range of points: product by product, each cut into ranges of equal cost
   int total = 0;
-  for (int i = 0; i < a.n_jobs; ++i) total += job_cost<SPLIT>(a.jobs[i].nA, a.jobs[i].nB);
+  for (int i = 0; i < a.n_jobs; ++i) total += cdw_cost<SPLIT>(a.jobs[i].nA, a.jobs[i].nB);
   const float per_block = (float)cols * (float)total / (float)(a.cus - a.n_jobs);
   int ji = 0, b = blockIdx.x, chunk = 0;
 #pragma unroll 1
   for (; ji < a.n_jobs; ++ji) {
-    chunk = a.chunk ? a.chunk : max(kCdwLeast, ((int)(per_block / (float)job_cost<SPLIT>(a.jobs[ji].nA, a.jobs[ji].nB)) + 31) / 32 * 32);
+    chunk = a.chunk ? a.chunk : max(kCdwLeast, ((int)(per_block / (float)cdw_cost<SPLIT>(a.jobs[ji].nA, a.jobs[ji].nB)) + 31) / 32 * 32);
     const int n = (cols + chunk - 1) / chunk;
     if (b < n) break;
     b -= n;
   }
   if (ji == a.n_jobs) return;  // uniform over the block
+  // (the ranges come from vector instructions; scalar from here on)
+  ji = __builtin_amdgcn_readfirstlane(ji);
+  b = __builtin_amdgcn_readfirstlane(b);
+  chunk = __builtin_amdgcn_readfirstlane(chunk);
   const CdwJob& jb = a.jobs[ji];
   const int pb = b * chunk, steps = (min(pb + chunk, cols) - pb) / 32;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   Ring ring(jb, pb, steps, lds);
-  if constexpr (SPLIT) {
-    if (jb.nA <= 2) {
-      run_split<1>(jb, 0, w, jb.db && w == 0, ring);
+  const CdwForm form = cdw_form<SPLIT>(jb.nA, jb.nB);
+  if (jb.nA <= 2) {
+    const bool sums = jb.db && w == 0;
+    if constexpr (SPLIT) {
+      run_split<1>(jb, 0, w, sums, ring);
     } else {
-      const int rb = w & 3, half = w >> 2, nc = (jb.nB + 3) / 4;
-      const bool sums = jb.db && half == 0;
-      if (nc <= 2) run_split<2>(jb, rb, 2 * half, sums, ring);
-      else if (nc == 3) run_split<3>(jb, rb, 3 * half, sums, ring);
-      else run_split<4>(jb, rb, 4 * half, sums, ring);
+      switch (2 * form.rows + form.cols) {
+        case 3: run_f32<1, 1, 8>(jb, 0, w, sums, ring); break;
+        case 4: run_f32<1, 2, 8>(jb, 0, w, sums, ring); break;
+        case 5: run_f32<2, 1, 8>(jb, 0, w, sums, ring); break;
+        default: run_f32<2, 2, 8>(jb, 0, w, sums, ring); break;
+      }
+    }
+  } else if constexpr (SPLIT) {
+    const int rb = w & 3, half = w >> 2, col0 = form.cols * half;
+    const bool sums = jb.db && half == 0;
+    switch (form.cols) {
+      case 1: run_split<1>(jb, rb, col0, sums, ring); break;
+      case 2: run_split<2>(jb, rb, col0, sums, ring); break;
+      case 3: run_split<3>(jb, rb, col0, sums, ring); break;
+      default: run_split<4>(jb, rb, col0, sums, ring); break;
     }
   } else {
-    if (jb.nA <= 2) {
-      const bool sums = jb.db && w == 0;
-      if (jb.nA == 1 && jb.nB <= 8) run_f32<1, 1, 8>(jb, 0, w, sums, ring);
-      else if (jb.nB <= 8) run_f32<2, 1, 8>(jb, 0, w, sums, ring);
-      else run_f32<2, 2, 8>(jb, 0, w, sums, ring);
-    } else {
-      const int row0 = 2 * (w >> 1), half = w & 1, nc = (jb.nB + 1) / 2;
-      const bool sums = jb.db && half == 0;
-      if (nc <= 4) run_f32<2, 4, 1>(jb, row0, 4 * half, sums, ring);
-      else if (nc == 5) run_f32<2, 5, 1>(jb, row0, 5 * half, sums, ring);
-      else run_f32<2, 8, 1>(jb, row0, 8 * half, sums, ring);
+    const int row0 = 2 * (w >> 1), half = w & 1, col0 = form.cols * half;
+    const bool sums = jb.db && half == 0;
+    switch (form.cols) {
+      case 1: run_f32<2, 1, 1>(jb, row0, col0, sums, ring); break;
+      case 2: run_f32<2, 2, 1>(jb, row0, col0, sums, ring); break;
+      case 3: run_f32<2, 3, 1>(jb, row0, col0, sums, ring); break;
+      case 4: run_f32<2, 4, 1>(jb, row0, col0, sums, ring); break;
+      case 5: run_f32<2, 5, 1>(jb, row0, col0, sums, ring); break;
+      case 6: run_f32<2, 6, 1>(jb, row0, col0, sums, ring); break;
+      case 7: run_f32<2, 7, 1>(jb, row0, col0, sums, ring); break;
+      default: run_f32<2, 8, 1>(jb, row0, col0, sums, ring); break;
     }
   }
 }

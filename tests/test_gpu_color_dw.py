@@ -94,3 +94,38 @@ def test_many_rows_and_counts(cuda, prec, tuned):
             close(grads(spec, prm, app, vd, gout, cuda, count), grads(spec, prm, app[:m], vd[:m], gout[:m], cuda))
     finally:
         autotune.set_knob('color_dw_chunk', old)
+
+
+# --- every number of column tiles of the first layer (1 .. 15) and of the basis (1 .. 16): D1 inputs by the basis
+# outputs and encodings, C components; bar and rows as in test_column_tiles
+WIDTHS = [(4, 14, 0, False), (16, 27, 0, True), (33 * 4, 20, 1, False), (48, 16, 1, False), (200, 27, 1, False),
+          (80, 16, 2, False), (176, 32, 1, True), (96, 27, 2, False), (112, 29, 2, False), (240, 24, 2, False),
+          (208, 24, 3, False), (224, 27, 3, False), (60, 29, 3, False), (64, 32, 3, False), (256, 26, 4, False)]
+
+
+@pytest.mark.parametrize('prec', ['fp32', 'bf16_split'])
+@pytest.mark.parametrize('i', range(len(WIDTHS)))
+def test_every_width(cuda, i, prec):
+    C, nb, Lf, view = WIDTHS[i]
+    spec = color.ColorSpec(n_features=C, basis_dim=nb, features_pe=Lf, use_view_dirs=view, views_pe=0, prec=prec)
+    if not spec.supported():
+        pytest.skip('more than 240 inputs once padded to the BF16 k-unit')
+    g = torch.Generator().manual_seed(60 + i)
+    d1 = nb * (2 * Lf + 1) + (3 if view else 0)
+    lin = lambda o, k: ((torch.rand(o, k, generator=g) * 2 - 1) / k ** 0.5, (torch.rand(o, generator=g) * 2 - 1) * 0.1)
+    prm = [(torch.rand(nb, C, generator=g) * 2 - 1) / C ** 0.5, *lin(128, d1), *lin(128, 128), *lin(3, 128)]
+    app = torch.randn(2600, C, generator=g) * 0.3
+    vd = F.normalize(torch.randn(2600, 3, generator=g), dim=-1)
+    basis, w1, b1, w2, b2, _, _ = [t.double() for t in prm]
+    x1 = _pe(app.double() @ basis.T, Lf)
+    if view:
+        x1 = torch.cat([x1, vd.double()], -1)
+    z1 = x1 @ w1.T + b1
+    z2 = z1.clamp_min(0) @ w2.T + b2
+    keep = (torch.cat([z1, z2], -1).abs().min(-1)[0] > 1e-4).nonzero()[:, 0][:600]
+    app, vd = app[keep], vd[keep]
+    gout = torch.randn(len(keep), 3, generator=g)
+    p64 = [t.double().requires_grad_(True) for t in prm]
+    (oracle(dict(Lf=Lf, Lv=0, view=view), p64, app.double(), vd.double()) * gout.double()).sum().backward()
+    got = grads(spec, prm, app.to(cuda), vd.to(cuda), gout.to(cuda), cuda)
+    close(got, [p.grad for p in p64])
