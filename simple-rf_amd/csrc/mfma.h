@@ -155,12 +155,15 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t (&out)[NP]
 // read that follows the builtin wait for all vector-memory operations (it cannot tell the buffers of a
 // stage or ring apart), which undoes a copy ahead of its use and drains the stores behind it.  The caller
 // waits for the copy (s_waitcnt vmcnt) and synchronises before it is read.
-// The compiler does not look for hazards in written-out instructions either, so their wait states are here: one
-// between the write of M0 and the copy, and five between a vector instruction that wrote the scalar address
-// (v_readfirstlane, v_readlane of a spilled one) and the copy; s_mov and s_nop 3 are these five.
+// The compiler does not look for hazards in written-out instructions either: one wait state belongs between the
+// write of M0 and the copy, and five between a vector instruction that wrote the copy's scalar address
+// (v_readfirstlane, v_readlane of a spilled one) and the copy.  The address is therefore copied by a scalar
+// instruction first, which the hardware keeps in order on both sides and which is M0's wait state (s_nop 3 in its
+// place cost the colour network's backward one percent).
 __device__ __forceinline__ void lds_dma_1k_ahead(const uint8_t* src, uint32_t lds_offset, uint32_t lane16) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2"
-               :
+  const uint8_t* at;
+  asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0"
+               : "=&s"(at)
                : "s"(lds_offset), "v"(lane16), "s"(src)
                : "memory", "m0");
 }
