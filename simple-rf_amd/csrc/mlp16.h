@@ -109,7 +109,10 @@ struct Stream16 {
 };
 
 // A value in an accumulation register (the MFMAs read their operands from there; vector operations
-// cannot).  No MFMA of these kernels writes accumulation registers.
+// cannot).  Its output is not an operand that the register also holds before, as push_nonzero's are (the register
+// pressure of that spills hundreds of values), so it may be any accumulation register: what makes that safe is
+// that no MFMA of these kernels writes one (-amdgpu-mfma-vgpr-form) and that a tile's quads are read a unit or more
+// after they are written.  tests/test_written_out_instructions.py reads both off the built code.
 __device__ __forceinline__ uint32_t to_agpr(uint32_t x) {
   uint32_t r;
   asm("v_accvgpr_write_b32 %0, %1" : "=a"(r) : "v"(x));
