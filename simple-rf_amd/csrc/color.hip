@@ -560,16 +560,6 @@ struct BwdArgs {
   uint8_t* ws;
 };
 
-// One element (feature f, point p) of a tile-block array of n_tiles tiles (the record of
-// mlp::store_tile holding it: chunk f & 1 of record 16 (fl / 4) + 2 (jj / 2) + (fl / 2) % 2, at
-// position 2 cb + jj % 2, fl = f mod 16, point p = 32 q + 16 cb + jj).
-__device__ __forceinline__ float load_elem(const uint8_t* base, size_t arr, int n_tiles, int f, int p) {
-  const int fl = f & 15, q = p & 31, jj = q & 15;
-  const int rec = 16 * (fl >> 2) + 2 * (jj >> 1) + ((fl >> 1) & 1);
-  const uint32_t off = blk_off(n_tiles, f >> 4, p) + 1024u * (fl & 1) + 16u * rec + 4u * (2 * (q >> 4) + (jj & 1));
-  return *reinterpret_cast<const float*>(base + arr + off);
-}
-
 template <int P>
 __device__ __forceinline__ void color_bwd_body(const BwdArgs& a) {
   __shared__ __attribute__((aligned(16))) uint8_t stage[stage_bytes<P>()];

@@ -34,9 +34,7 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // kBFS1: one plane, i.e. BF16 operands rounded from FP32 activations and weights (FP32 storage).
 enum Prec { kF32 = 0, kBF16 = 1, kF16 = 2, kBFS3 = 3, kBFS2 = 4, kBFS1 = 5 };
 
-template <int P>
-__host__ __device__ constexpr bool f32_layout() { return P == kF32 || P == kBFS3 || P == kBFS2 || P == kBFS1; }
-// BF16 operand planes of the FP32-layout precisions
+// BF16 operand planes of the precisions with FP32 activations
 template <int P>
 __host__ __device__ constexpr bool split_prec() { return P == kBFS3 || P == kBFS2 || P == kBFS1; }
 template <int P>

@@ -367,7 +367,6 @@ __device__ __forceinline__ void static_for(F&& f) {
 // of chunk c; every wave then reads the fragments it needs from LDS.  This divides the weight
 // traffic out of L2 by the number of waves per block and hides its latency.
 constexpr int kKC = 2;
-constexpr int kStageBytes = 16 * kKC * 1024;
 // Split-BF16 operands: a k-unit's fragment is one 1 KB plane per BF16 plane (3 KB forward, 2 KB
 // backward), and a chunk holds one k-unit when there are three planes, so that one buffer of the
 // stage is 48 KB (forward) or 64 KB (backward, two k-units).
@@ -1181,18 +1180,7 @@ struct DwArgs {
   DwJob jobs[kMaxJobs];
   int n_jobs, ldP, cols, chunk, n_chunks, total_work;
   int segment;  // points after which a block adds its sums to the gradients and begins anew
-  // dZ / X layout: 0 plain feature-major rows; 1 the paired tile blocks of store_tile
-  int paired;
-  // optional device-side point count: only the columns below it, rounded up to whole 256-point
-  // blocks, are reduced (the chunks past it exit); the columns up to that bound must hold finite
-  // values with dZ = 0 beyond the count, as the forward and backward kernels leave them
-  const int32_t* cols_dev;
 };
-
-// Columns of a weight-gradient launch: a.cols, or fewer when a device-side count is given.
-__device__ __forceinline__ int dw_cols(const DwArgs& a) {
-  return a.cols_dev ? min(a.cols, (*a.cols_dev + 255) / 256 * 256) : a.cols;
-}
 
 // One block of 8 waves reduces a 256 x 256 tile of dW = dZ X^T (a whole layer of the MLP) over a
 // chunk of points, so every dZ and X row of the chunk is read from HBM once; the reduction over
@@ -1228,8 +1216,7 @@ __global__ __launch_bounds__(64 * kDwWaves) void mlp_dw_kernel(DwArgs a) {
   const int tile = local % nblk, chunk = local / nblk;
   const int m0 = kTM * (tile % jb.mblocks), n0 = kTN * (tile / jb.mblocks);
   const int pb = chunk * a.chunk;
-  const int pe = min(pb + a.chunk, dw_cols(a));
-  if (pb >= pe) return;  // the chunk lies past the device-side count (uniform over the block)
+  const int pe = min(pb + a.chunk, a.cols);
   const size_t ldP = a.ldP;
   static_assert(P == kF32, "16-bit operands: mlp16_dw.h; split BF16: mlp_dw_split_kernel");
   constexpr int ELEM = 4;
@@ -1248,19 +1235,13 @@ __global__ __launch_bounds__(64 * kDwWaves) void mlp_dw_kernel(DwArgs a) {
       int row0 = (is_a ? m0 : n0) + 16 * rt;
       if (row0 >= (is_a ? jb.dz_rows : jb.x_rows)) row0 = is_a ? m0 : n0;
       const uint8_t* base = is_a ? jb.dz : jb.x;
-      const uint8_t* src;
-      if (a.paired) {
-        // lane (g, j) takes feature j's chunk of the record pair m = 4 u + g of the 2 KB block of
-        // the points' wave (see store_tile): record (j >> 2, 2 m + ((j >> 1) & 1)), chunk j & 1
-        constexpr int PPW = 32;  // points per stored wave block
-        const int wb = p / PPW, u = (p % PPW) / KPTS;
-        const int rec = 16 * (j >> 2) + 2 * (4 * u + g) + ((j >> 1) & 1);
-        // tile-major blocks: tile t's blocks span 16 rows of ldP points
-        const size_t blk = (size_t)row0 * ldP * ELEM + (size_t)wb * 2048;
-        src = base + blk + (j & 1) * 1024 + rec * 16;
-      } else {
-        src = base + (((size_t)(row0 + j)) * ldP + p + 4 * g) * ELEM;
-      }
+      // lane (g, j) takes feature j's chunk of the record pair m = 4 u + g of the 2 KB block of
+      // the points' wave (see store_tile): record (j >> 2, 2 m + ((j >> 1) & 1)), chunk j & 1;
+      // tile-major blocks: tile t's blocks span 16 rows of ldP points
+      constexpr int PPW = 32;  // points per stored wave block
+      const int wb = p / PPW, u = (p % PPW) / KPTS;
+      const int rec = 16 * (j >> 2) + 2 * (4 * u + g) + ((j >> 1) & 1);
+      const uint8_t* src = base + (size_t)row0 * ldP * ELEM + (size_t)wb * 2048 + (j & 1) * 1024 + rec * 16;
       __builtin_amdgcn_global_load_lds((const void*)src,
                                        (__attribute__((address_space(3))) void*)(buf + f * 1024), 16, 0, 0);
     }
@@ -1378,8 +1359,7 @@ __global__ __launch_bounds__(64 * kDwWaves) void mlp_dw_split_kernel(DwArgs a) {
   const int tile = local % nblk, chunk = local / nblk;
   const int m0 = kDwTile * (tile % jb.mblocks), n0 = kDwTile * (tile / jb.mblocks);
   const int pb = chunk * a.chunk;
-  const int pe = min(pb + a.chunk, dw_cols(a));
-  if (pb >= pe) return;  // the chunk lies past the device-side count (uniform over the block)
+  const int pe = min(pb + a.chunk, a.cols);
   const size_t ldP = a.ldP;
   constexpr int KPTS = 16;
   const int qm = 4 * (w >> 1), qn = 8 * (w & 1);  // first 16-row / 16-column tile of the wave

@@ -149,21 +149,16 @@ struct QuadSite {
   LineTaps lt;
 };
 
-__device__ __forceinline__ QuadSite quad_site(const VmArgs& a, int p, int c, const float pn[3]) {
+__device__ __forceinline__ QuadSite quad_site(const VmArgs& a, int q, const float pn[3]) {
   QuadSite s;
-  s.p = p;
-  s.c = c;
+  s.p = quad_plane(a, q);
+  s.c = 4 * (q - sel3(s.p, a.qoff[0], a.qoff[1], a.qoff[2]));
   const float x = sel3(s.p, pn[axis_a0(0)], pn[axis_a0(1)], pn[axis_a0(2)]);
   const float y = sel3(s.p, pn[axis_a1(0)], pn[axis_a1(1)], pn[axis_a1(2)]);
   const float v = sel3(s.p, pn[axis_v(0)], pn[axis_v(1)], pn[axis_v(2)]);
   s.pt = plane_taps(x, y, sel3(s.p, a.pw[0], a.pw[1], a.pw[2]), sel3(s.p, a.ph[0], a.ph[1], a.ph[2]));
   s.lt = line_taps(v, sel3(s.p, a.ll[0], a.ll[1], a.ll[2]));
   return s;
-}
-
-__device__ __forceinline__ QuadSite quad_site(const VmArgs& a, int q, const float pn[3]) {
-  const int p = quad_plane(a, q);
-  return quad_site(a, p, 4 * (q - sel3(p, a.qoff[0], a.qoff[1], a.qoff[2])), pn);
 }
 
 // Sum of the taps v of weights w; a tap that is not ok adds nothing (whatever its value and weight).  The
@@ -459,26 +454,21 @@ __global__ __launch_bounds__(256) void density_fwd_kernel(VmArgs a, AlphaArgs m,
 // most contended texels drop by up to the run length.
 constexpr int kRun = 32;  // samples walked by one lane group (SRF_TUNE_GATHER_RUN overrides it)
 
-// T quads of one lane share the corners; quad t's components start at c[t] and it counts if on[t].
-template <int T>
 struct RunAcc {
   int pidx[4], lidx[2];
-  float4 pg[4][T], lg[2][T];
+  float4 pg[4], lg[2];
 };
 
-template <int T>
-__device__ __forceinline__ void run_init(RunAcc<T>& r) {
+__device__ __forceinline__ void run_init(RunAcc& r) {
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     r.pidx[k] = -1;
-#pragma unroll
-    for (int t = 0; t < T; ++t) r.pg[k][t] = make_float4(0.f, 0.f, 0.f, 0.f);
+    r.pg[k] = make_float4(0.f, 0.f, 0.f, 0.f);
   }
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
     r.lidx[k] = -1;
-#pragma unroll
-    for (int t = 0; t < T; ++t) r.lg[k][t] = make_float4(0.f, 0.f, 0.f, 0.f);
+    r.lg[k] = make_float4(0.f, 0.f, 0.f, 0.f);
   }
 }
 
@@ -496,104 +486,79 @@ __device__ __forceinline__ void atomic_add4v(float* p, float4 v) {
 // A slot is carried only when its texel index equals the new corner's, so any move is handled
 // correctly (unmatched slots are flushed); index -1 marks a corner outside the factor, whose
 // slot is never flushed.  Static selects only: the slots stay in registers.
-template <int T>
-__device__ __forceinline__ void flush_slot(float* grad, int idx, const float4 (&acc)[T], int C, const int (&c)[T],
-                                           const bool (&on)[T]) {
-  if (idx < 0) return;
-#pragma unroll
-  for (int t = 0; t < T; ++t)
-    if (on[t]) atomic_add4v(grad + (int64_t)idx * C + c[t], acc[t]);
+__device__ __forceinline__ void flush_slot(float* grad, int idx, float4 acc, int C, int c) {
+  if (idx >= 0) atomic_add4v(grad + (int64_t)idx * C + c, acc);
 }
 
-template <int N, int T>
-__device__ __forceinline__ void flush_slots(const int (&si)[N], const float4 (&sa)[N][T], float* grad, int C,
-                                            const int (&c)[T], const bool (&on)[T]) {
+template <int N>
+__device__ __forceinline__ void flush_slots(const int (&si)[N], const float4 (&sa)[N], float* grad, int C, int c) {
 #pragma unroll
-  for (int k = 0; k < N; ++k) flush_slot(grad, si[k], sa[k], C, c, on);
+  for (int k = 0; k < N; ++k) flush_slot(grad, si[k], sa[k], C, c);
 }
 
 __device__ __forceinline__ float4 pick4(bool b, float4 x, float4 y) {
   return make_float4(b ? x.x : y.x, b ? x.y : y.y, b ? x.z : y.z, b ? x.w : y.w);
 }
 
-template <int T>
-__device__ __forceinline__ void plane_accum(int (&si)[4], float4 (&sa)[4][T], const int (&ci)[4], const float (&cw)[4],
-                                            const float4 (&g)[T], float* grad, int C, const int (&c)[T],
-                                            const bool (&on)[T]) {
+__device__ __forceinline__ void plane_accum(int (&si)[4], float4 (&sa)[4], const int (&ci)[4], const float (&cw)[4], float4 g,
+                                            float* grad, int C, int c) {
   const bool same = ci[0] == si[0] && ci[1] == si[1] && ci[2] == si[2] && ci[3] == si[3];
   if (__ballot(!same) != 0) {  // some lane's walk leaves its cell
     const bool px = !same && ci[0] == si[1] && ci[2] == si[3];         // cell moved +x: nw<-ne, sw<-se
     const bool nx = !same && !px && ci[1] == si[0] && ci[3] == si[2];  // -x: ne<-nw, se<-sw
     const bool py = !same && !px && !nx && ci[0] == si[2] && ci[1] == si[3];          // +y: nw<-sw, ne<-se
     const bool ny = !same && !px && !nx && !py && ci[2] == si[0] && ci[3] == si[1];  // -y: sw<-nw, se<-ne
-    if (!(same || nx || ny)) flush_slot(grad, si[0], sa[0], C, c, on);
-    if (!(same || px || ny)) flush_slot(grad, si[1], sa[1], C, c, on);
-    if (!(same || nx || py)) flush_slot(grad, si[2], sa[2], C, c, on);
-    if (!(same || px || py)) flush_slot(grad, si[3], sa[3], C, c, on);
+    if (!(same || nx || ny)) flush_slot(grad, si[0], sa[0], C, c);
+    if (!(same || px || ny)) flush_slot(grad, si[1], sa[1], C, c);
+    if (!(same || nx || py)) flush_slot(grad, si[2], sa[2], C, c);
+    if (!(same || px || py)) flush_slot(grad, si[3], sa[3], C, c);
     const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-      const float4 n0 = pick4(same, sa[0][t], pick4(px, sa[1][t], pick4(py, sa[2][t], z)));
-      const float4 n1 = pick4(same, sa[1][t], pick4(nx, sa[0][t], pick4(py, sa[3][t], z)));
-      const float4 n2 = pick4(same, sa[2][t], pick4(px, sa[3][t], pick4(ny, sa[0][t], z)));
-      const float4 n3 = pick4(same, sa[3][t], pick4(nx, sa[2][t], pick4(ny, sa[1][t], z)));
-      sa[0][t] = n0;
-      sa[1][t] = n1;
-      sa[2][t] = n2;
-      sa[3][t] = n3;
-    }
+    const float4 n0 = pick4(same, sa[0], pick4(px, sa[1], pick4(py, sa[2], z)));
+    const float4 n1 = pick4(same, sa[1], pick4(nx, sa[0], pick4(py, sa[3], z)));
+    const float4 n2 = pick4(same, sa[2], pick4(px, sa[3], pick4(ny, sa[0], z)));
+    const float4 n3 = pick4(same, sa[3], pick4(nx, sa[2], pick4(ny, sa[1], z)));
+    sa[0] = n0;
+    sa[1] = n1;
+    sa[2] = n2;
+    sa[3] = n3;
 #pragma unroll
     for (int k = 0; k < 4; ++k) si[k] = ci[k];
   }
 #pragma unroll
-  for (int k = 0; k < 4; ++k)
-#pragma unroll
-    for (int t = 0; t < T; ++t) sa[k][t] = madd4(sa[k][t], g[t], cw[k]);
+  for (int k = 0; k < 4; ++k) sa[k] = madd4(sa[k], g, cw[k]);
 }
 
-template <int T>
-__device__ __forceinline__ void line_accum(int (&si)[2], float4 (&sa)[2][T], const int (&ci)[2], const float (&cw)[2],
-                                           const float4 (&g)[T], float* grad, int C, const int (&c)[T],
-                                           const bool (&on)[T]) {
+__device__ __forceinline__ void line_accum(int (&si)[2], float4 (&sa)[2], const int (&ci)[2], const float (&cw)[2], float4 g,
+                                           float* grad, int C, int c) {
   const bool same = ci[0] == si[0] && ci[1] == si[1];
   if (__ballot(!same) != 0) {
     const bool up = !same && ci[0] == si[1];           // lower <- upper
     const bool down = !same && !up && ci[1] == si[0];  // upper <- lower
-    if (!(same || down)) flush_slot(grad, si[0], sa[0], C, c, on);
-    if (!(same || up)) flush_slot(grad, si[1], sa[1], C, c, on);
+    if (!(same || down)) flush_slot(grad, si[0], sa[0], C, c);
+    if (!(same || up)) flush_slot(grad, si[1], sa[1], C, c);
     const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-      const float4 n0 = pick4(same, sa[0][t], pick4(up, sa[1][t], z));
-      const float4 n1 = pick4(same, sa[1][t], pick4(down, sa[0][t], z));
-      sa[0][t] = n0;
-      sa[1][t] = n1;
-    }
+    const float4 n0 = pick4(same, sa[0], pick4(up, sa[1], z));
+    const float4 n1 = pick4(same, sa[1], pick4(down, sa[0], z));
+    sa[0] = n0;
+    sa[1] = n1;
     si[0] = ci[0];
     si[1] = ci[1];
   }
 #pragma unroll
-  for (int k = 0; k < 2; ++k)
-#pragma unroll
-    for (int t = 0; t < T; ++t) sa[k][t] = madd4(sa[k][t], g[t], cw[k]);
+  for (int k = 0; k < 2; ++k) sa[k] = madd4(sa[k], g, cw[k]);
 }
 
 // Adds one sample's plane gradient gp and line gradient gl (before the corner weights).
-__device__ __forceinline__ void run_add(const VmArgs& a, const QuadSite& s, RunAcc<1>& r, float4 gp, float4 gl) {
+__device__ __forceinline__ void run_add(const VmArgs& a, const QuadSite& s, RunAcc& r, float4 gp, float4 gl) {
   const int C = sel3(s.p, a.comp[0], a.comp[1], a.comp[2]);
-  const int c[1] = {s.c};
-  const bool on[1] = {true};
-  const float4 gps[1] = {gp}, gls[1] = {gl};
-  plane_accum<1>(r.pidx, r.pg, s.pt.idx, s.pt.w, gps, sel3(s.p, a.dplane[0], a.dplane[1], a.dplane[2]), C, c, on);
-  line_accum<1>(r.lidx, r.lg, s.lt.idx, s.lt.w, gls, sel3(s.p, a.dline[0], a.dline[1], a.dline[2]), C, c, on);
+  plane_accum(r.pidx, r.pg, s.pt.idx, s.pt.w, gp, sel3(s.p, a.dplane[0], a.dplane[1], a.dplane[2]), C, s.c);
+  line_accum(r.lidx, r.lg, s.lt.idx, s.lt.w, gl, sel3(s.p, a.dline[0], a.dline[1], a.dline[2]), C, s.c);
 }
 
-__device__ __forceinline__ void run_flush(const VmArgs& a, int p, int c0, const RunAcc<1>& r) {
+__device__ __forceinline__ void run_flush(const VmArgs& a, int p, int c, const RunAcc& r) {
   const int C = sel3(p, a.comp[0], a.comp[1], a.comp[2]);
-  const int c[1] = {c0};
-  const bool on[1] = {true};
-  flush_slots<4, 1>(r.pidx, r.pg, sel3(p, a.dplane[0], a.dplane[1], a.dplane[2]), C, c, on);
-  flush_slots<2, 1>(r.lidx, r.lg, sel3(p, a.dline[0], a.dline[1], a.dline[2]), C, c, on);
+  flush_slots(r.pidx, r.pg, sel3(p, a.dplane[0], a.dplane[1], a.dplane[2]), C, c);
+  flush_slots(r.lidx, r.lg, sel3(p, a.dline[0], a.dline[1], a.dline[2]), C, c);
 }
 
 // d_feat = d_sigma * predictor'(feat) on valid samples; planes receive d_feat * line and
@@ -609,7 +574,7 @@ __global__ __launch_bounds__(256) void density_bwd_kernel(VmArgs a, int64_t n, i
     const int64_t i0 = run * run_len;
     const int64_t i1 = i0 + run_len < n ? i0 + run_len : n;
     for (int q = gp.ql; q < a.n_quads; q += G) {
-      RunAcc<1> r;
+      RunAcc r;
       run_init(r);
       int p = 0, c = 0;
       for (int64_t i = i0; i < i1; ++i) {
@@ -676,7 +641,7 @@ __global__ __launch_bounds__(256) void appearance_bwd_kernel(VmArgs a, int64_t n
     const int64_t j0 = run * run_len;
     const int64_t j1 = j0 + run_len < n ? j0 + run_len : n;
     for (int q = gp.ql; q < a.n_quads; q += G) {
-      RunAcc<1> r;
+      RunAcc r;
       run_init(r);
       int p = 0, c = 0;
       for (int64_t j = j0; j < j1; ++j) {
@@ -1071,15 +1036,6 @@ __global__ __launch_bounds__(kSortedThreads, 3) void sorted_bwd_kernel(VmArgs a,
   int pat = 0, pflags = 0, lat = 0, lflags = 0;  // the site the slots belong to (flags 0: none)
   float4 pg[4] = {zero, zero, zero, zero}, lg[2] = {zero, zero};
   int queued = 0;  // the wave's
-  auto grads_of = [&](float word, float4& gp, float4& gl) {
-    if (kDensity) {
-      gp = gl = make_float4(word, word, word, word);
-    } else {
-      const float* row = r.d_out + (int64_t)__float_as_int(word) * a.total_comp;
-      gp = C ? ld4(row + 4 * a.qoff[P] + c) : zero;
-      gl = CL ? ld4(row + 4 * a.qoff[PL] + cl) : zero;
-    }
-  };
   float4 en = order[min(s0 + ql, m - 1)];  // the next row that this lane prepares
   for (int k0 = 0; __ballot(k0 < rows) != 0; k0 += lanes) {
     {
@@ -1247,7 +1203,7 @@ __device__ __forceinline__ float4 cp_product(const float4 v[kPlanes]) { return m
 // Run-length gradient accumulation for the three lines of one quad (as RunAcc for VM).
 struct CpRun {
   int idx[kPlanes][2];
-  float4 g[kPlanes][2][1];
+  float4 g[kPlanes][2];
 };
 
 __device__ __forceinline__ void cp_run_init(CpRun& r) {
@@ -1256,28 +1212,21 @@ __device__ __forceinline__ void cp_run_init(CpRun& r) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       r.idx[k][t] = -1;
-      r.g[k][t][0] = make_float4(0.f, 0.f, 0.f, 0.f);
+      r.g[k][t] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
 }
 
-__device__ __forceinline__ void cp_run_flush(const CpArgs& a, int k, int c0, const CpRun& r) {
-  const int c[1] = {c0};
-  const bool on[1] = {true};
-  flush_slots<2, 1>(r.idx[k], r.g[k], a.dline[k], a.comp, c, on);
+__device__ __forceinline__ void cp_run_flush(const CpArgs& a, int k, int c, const CpRun& r) {
+  flush_slots(r.idx[k], r.g[k], a.dline[k], a.comp, c);
 }
 
 // Adds the gradient g of the quad's component products: line k receives g times the other two
 // lines' values, spread over its two taps.
-__device__ __forceinline__ void cp_run_add(const CpArgs& a, const CpTaps& s, int c0, CpRun& r, float4 g,
+__device__ __forceinline__ void cp_run_add(const CpArgs& a, const CpTaps& s, int c, CpRun& r, float4 g,
                                            const float4 v[kPlanes]) {
   const float4 d[kPlanes] = {mul4(mul4(g, v[1]), v[2]), mul4(mul4(g, v[0]), v[2]), mul4(mul4(g, v[0]), v[1])};
-  const int c[1] = {c0};
-  const bool on[1] = {true};
 #pragma unroll
-  for (int k = 0; k < kPlanes; ++k) {
-    const float4 dk[1] = {d[k]};
-    line_accum<1>(r.idx[k], r.g[k], s.t[k].idx, s.t[k].w, dk, a.dline[k], a.comp, c, on);
-  }
+  for (int k = 0; k < kPlanes; ++k) line_accum(r.idx[k], r.g[k], s.t[k].idx, s.t[k].w, d[k], a.dline[k], a.comp, c);
 }
 
 template <int G>
