@@ -154,14 +154,13 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t (&out)[NP]
 // stage or ring apart), which undoes a copy ahead of its use and drains the stores behind it.  The caller
 // waits for the copy (s_waitcnt vmcnt) and synchronises before it is read.
 // The compiler does not look for hazards in written-out instructions either: one wait state belongs between the
-// write of M0 and the copy, and five between a vector instruction that wrote the copy's scalar address
-// (v_readfirstlane, v_readlane of a spilled one) and the copy.  The address is therefore copied by a scalar
-// instruction first, which the hardware keeps in order on both sides and which is M0's wait state (s_nop 3 in its
-// place cost the colour network's backward one percent).
+// write of M0 and the copy (s_nop 0), and five between a vector instruction that wrote the copy's scalar address
+// (v_readfirstlane, v_readlane of a spilled one) and the copy.  Here src is an address that scalar instructions
+// step from copy to copy; tests/test_written_out_instructions.py checks the five states for every copy of the
+// built library.
 __device__ __forceinline__ void lds_dma_1k_ahead(const uint8_t* src, uint32_t lds_offset, uint32_t lane16) {
-  const uint8_t* at;
-  asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0"
-               : "=&s"(at)
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :
                : "s"(lds_offset), "v"(lane16), "s"(src)
                : "memory", "m0");
 }
@@ -169,12 +168,18 @@ __device__ __forceinline__ void lds_dma_1k_ahead(const uint8_t* src, uint32_t ld
 __device__ __forceinline__ uint32_t lds_offset(const void* p) {
   return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)p);
 }
-// The same for a fragment that lies in lane order at src.
+// The same for a fragment that lies in lane order at any wave-uniform src.  A vector instruction may have made the
+// address just before, so a scalar one copies it first, which the hardware keeps in order on both sides and which
+// is M0's wait state (s_nop 3 in its place cost the colour network's backward one percent).
 __device__ __forceinline__ void lds_dma_1k(const uint8_t* src, uint8_t* lds_base) {
   const uint64_t v = reinterpret_cast<uint64_t>(src);
   const uint64_t u = (uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(v >> 32)) << 32 |
                      (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)v);
-  lds_dma_1k_ahead(reinterpret_cast<const uint8_t*>(u), lds_offset(lds_base), (threadIdx.x & 63) * 16);
+  uint64_t at;
+  asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0"
+               : "=&s"(at)
+               : "s"(lds_offset(lds_base)), "v"((threadIdx.x & 63) * 16), "s"(u)
+               : "memory", "m0");
 }
 
 // A block barrier that waits for no memory operation (__syncthreads would drain the copies in flight).
