@@ -297,26 +297,26 @@ __global__ __launch_bounds__(64 * kCdwWaves) void color_dw_kernel(CdwArgs a) {
       }
     }
   } else if constexpr (SPLIT) {
-    const int rb = w & 3, half = w >> 2, col0 = form.cols * half;
+    const int rb = w & 3, half = w >> 2;
     const bool sums = jb.db && half == 0;
     switch (form.cols) {
-      case 1: run_split<1>(jb, rb, col0, sums, ring); break;
-      case 2: run_split<2>(jb, rb, col0, sums, ring); break;
-      case 3: run_split<3>(jb, rb, col0, sums, ring); break;
-      default: run_split<4>(jb, rb, col0, sums, ring); break;
+      case 1: run_split<1>(jb, rb, 1 * half, sums, ring); break;
+      case 2: run_split<2>(jb, rb, 2 * half, sums, ring); break;
+      case 3: run_split<3>(jb, rb, 3 * half, sums, ring); break;
+      default: run_split<4>(jb, rb, 4 * half, sums, ring); break;
     }
   } else {
-    const int row0 = 2 * (w >> 1), half = w & 1, col0 = form.cols * half;
+    const int row0 = 2 * (w >> 1), half = w & 1;
     const bool sums = jb.db && half == 0;
     switch (form.cols) {
-      case 1: run_f32<2, 1, 1>(jb, row0, col0, sums, ring); break;
-      case 2: run_f32<2, 2, 1>(jb, row0, col0, sums, ring); break;
-      case 3: run_f32<2, 3, 1>(jb, row0, col0, sums, ring); break;
-      case 4: run_f32<2, 4, 1>(jb, row0, col0, sums, ring); break;
-      case 5: run_f32<2, 5, 1>(jb, row0, col0, sums, ring); break;
-      case 6: run_f32<2, 6, 1>(jb, row0, col0, sums, ring); break;
-      case 7: run_f32<2, 7, 1>(jb, row0, col0, sums, ring); break;
-      default: run_f32<2, 8, 1>(jb, row0, col0, sums, ring); break;
+      case 1: run_f32<2, 1, 1>(jb, row0, 1 * half, sums, ring); break;
+      case 2: run_f32<2, 2, 1>(jb, row0, 2 * half, sums, ring); break;
+      case 3: run_f32<2, 3, 1>(jb, row0, 3 * half, sums, ring); break;
+      case 4: run_f32<2, 4, 1>(jb, row0, 4 * half, sums, ring); break;
+      case 5: run_f32<2, 5, 1>(jb, row0, 5 * half, sums, ring); break;
+      case 6: run_f32<2, 6, 1>(jb, row0, 6 * half, sums, ring); break;
+      case 7: run_f32<2, 7, 1>(jb, row0, 7 * half, sums, ring); break;
+      default: run_f32<2, 8, 1>(jb, row0, 8 * half, sums, ring); break;
     }
   }
 }
