@@ -486,7 +486,9 @@ int srf_adam_step(int n_tensors, float* const* params, const float* const* grads
 #define SRF_TUNE_GATHER_BLOCKS 2  /* grid cap of the factor-gather kernels (srf_vm_*, srf_cp_*): 0 = 8192;
                                      else 256..65536 blocks of 256 threads */
 #define SRF_TUNE_GATHER_RUN 3     /* consecutive samples one lane group walks in the gather backwards, summing
-                                     equal-corner gradients before the atomics: 0 = 32; else 1..256 */
+                                     equal-corner gradients before the atomics: 0 = built-in (cell-sorted
+                                     backwards: the rows that there are over the lane groups of one round,
+                                     at least 16; in sample order: 32); else 1..256 */
 #define SRF_TUNE_KNOBS 4
 
 /* Sets knob to value (SRF_EINVAL for an unknown knob or a value outside its range). */

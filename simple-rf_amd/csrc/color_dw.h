@@ -9,7 +9,7 @@
 // own size, and a wave reads the operands of 16 points while the MFMAs of the previous 16 run.  The ranges
 // are cut in the kernel, from the device-side count, so that every block costs about the same and one round
 // of the compute units does it (two rounds measure the same).  1.4M rows of the 144-component network in
-// FP32: 1.25 ms (2.15 ms by equal chunks of the MLP's FP32 kernel, which read a unit's operands after its
+// FP32: 1.28 ms (2.15 ms by equal chunks of the MLP's FP32 kernel, which read a unit's operands after its
 // barrier and kept two waves of eight busy on the basis and one on W3); 300,000 rows of the 72-component
 // one, split: 0.21 ms or 4.7 TB/s (0.46 ms in chunks of 3,840, whose second round was nearly empty).
 #pragma once
@@ -60,8 +60,9 @@ __host__ __device__ constexpr CdwForm cdw_form(int nA, int nB) {
 }
 
 // Cost of 16 points to a block, in cycles: the MFMAs of its busiest SIMD (two waves) or the reads, and the
-// step itself.  The reads' share and the step's were swept (1.4M rows FP32, 300,000 rows split, us):
-// 104 / 200 1306, 205; 80 / 200 1252, 204; 60 / 200 1215, 208; 60 / 50 1258, 211; 40 / 100 1219, 225.
+// step itself.  The reads' share and the step's were swept (the kernel on 1.4M rows of 144 components and of 72 without
+// encoding in FP32, and on 300,000 of 72 split, us): 104 / 200 1370, 993, 212; 80 / 200 1307, 895, 214; 60 / 200
+// 1295, 904, 200; 60 / 50 1296, 952, 218; 40 / 100 1406, 988, 208; 60 (split 90) / 200 1280, 897, 208.
 template <bool SPLIT>
 __host__ __device__ constexpr int cdw_cost(int nA, int nB) {
   const CdwForm f = cdw_form<SPLIT>(nA, nB);

@@ -21,7 +21,7 @@ constexpr int kCdwAside = 32;
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-// s_waitcnt vmcnt(n) for a wave-uniform n, at most 47.
+// s_waitcnt vmcnt(n) for a wave-uniform n of at most 30.
 __device__ __forceinline__ void wait_vmem_le(int n) {
   switch (n) {
 #define SRF_WAIT_CASE(k) case k: __builtin_amdgcn_s_waitcnt(mlp::vmcnt_only(k)); break;

@@ -1,11 +1,12 @@
 // NeRF MLP forward and backward chain for 16-bit operands (BF16 training and inference, FP16
-// inference) on 32x32x16 MFMAs.  Plan, workspace and weight gradients are those of mlp_impl.h.
+// inference) on 32x32x16 MFMAs.  Plan and workspace are those of mlp_impl.h; the weight gradients are in
+// mlp16_dw.h.
 //
 // Why 32x32: with one wave per SIMD a stream of
 // independent 16x16x32 MFMAs on random operands reaches 1.40-1.50 PFLOP/s on this chip, the same
 // products as 32x32x16 MFMAs 1.79 PFLOP/s (1.58 and 2.49 on zeros: the larger shape also draws less
 // power per product).  4,096 rays x 192 samples, main model: training forward 1,705 us on 16x16x32 tiles,
-// 1,034 us here; backward chain 1,339 -> 898 us; inference of 16,384 x 192 points 3,985 -> 3,107 us.
+// 1,103 us here; backward chain 1,339 -> 894 us; inference of 16,384 x 192 points 3,985 -> 2,956 us.
 // The kernels are bound by the MFMAs (a 256 x 256 layer of 256 points: 3.5 us at the full clock, 4.8 us at
 // the clock that random operands leave), their operand reads from LDS (half of its rate) and, in training,
 // the stores (5.5 and 5.2 KB a point: 630 us at a fill's rate for 786,432 points).
@@ -165,8 +166,8 @@ __device__ __forceinline__ void all_pieces(const Epi& epi) {
   static_for<0, 4>([&](auto Q) SRF_AI { static_for<0, 4>([&](auto I) SRF_AI { epi(Q, I); }); });
 }
 
-// Stores 16-feature tile t of the wave's 64 points as the 2 KB block that the weight-gradient GEMM
-// reads (mlp_dw_kernel): record (h, c), chunk k at byte 1024 k + 16 (32 h + c), holds features 8 k + 4 h +
+// Stores 16-feature tile t of the wave's 64 points as the 2 KB block that the weight-gradient kernel
+// reads (mlp16_dw.h): record (h, c), chunk k at byte 1024 k + 16 (32 h + c), holds features 8 k + 4 h +
 // r (r = 0 .. 3, one dword each) at the lane's own points c and 32 + c.  Chunk k comes from quad k of the
 // tile's pair (its k-steps 2 (t / 2) + k) in both column blocks.  One byte permutation a dword, no lane
 // exchange, and each of the two stores writes 1 KB of whole lines.  Non-temporal, as store_tile's.

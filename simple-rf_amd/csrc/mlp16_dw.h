@@ -1,5 +1,5 @@
-// Weight gradients of the NeRF MLP for 16-bit operands (kernel in mlp16_dw.hip): dW = dZ X^T over all layers in one grouped launch,
-// K = points, on 32x32x16 MFMAs.  mlp16.h writes the operands (store_tile16).
+// Weight gradients of the NeRF MLP for 16-bit operands (kernel in mlp16_dw.hip): dW = dZ X^T over all layers in one
+// grouped launch, K = points, on 32x32x16 MFMAs.  mlp16.h writes the operands (store_tile16).
 //
 // What bounds it: every stored row is read from HBM once (10 KB a point of the main model) at 120 FLOP a
 // byte, below the chip's balance, so the reads have to stream while the matrix cores and the LDS work behind
@@ -10,7 +10,9 @@
 // operands of a k-step of 16 points while the MFMAs of the previous one run.
 //   786,432 points of the main model: 1,598 us by the 16x16x32 kernel it replaces (14 jobs, 8.9 GB: the skip's,
 // the sigma row's and the view layer's operands read again; operands read after each unit's barrier, before
-// its MFMAs), 1,440 us here: 7.9 GB at 5.5 TB/s, where a 2 GiB copy moves 4.9 TB/s.
+// its MFMAs), 1,461 us here: 7.9 GB at 5.4 TB/s, where a 2 GiB copy moves 4.9 TB/s.
+//   A block's running FP32 sums end before its range does: after jb.segment points they are added to the gradients
+// or, where a wave holds one or two tiles, set aside in registers (mlp.hip, weight_grads16).
 #pragma once
 
 #include "mlp_impl.h"

@@ -1,6 +1,6 @@
 // Fused positional encoding + NeRF MLP on gfx950 MFMA (templates shared by mlp*.hip): forward and backward
-// chain on FP32 activations (FP32 and split-BF16 operands; mlp16.h has those for 16-bit operands) and the
-// weight gradients of every precision.
+// chain on FP32 activations and their weight gradients (FP32 and split-BF16 operands).  mlp16.h and mlp16_dw.h
+// have those for 16-bit operands.
 //
 // Reference semantics: MLP.forward / get_view_independent_outputs / get_view_dependent_outputs
 // and PositionalEncoder (src/models/SimpleNeRF17.py:581-785), driven by run_network/batchify

@@ -18,8 +18,9 @@
 //   then groups of G = 4 or 8 lanes read the factors of the prepared samples, lane j of a group the
 //   quads j, j + G, ...: a tap of a group is one contiguous 16 B x G read, appearance rows are
 //   written as 16 B stores, and the density sum over channels is a butterfly inside the group.
-//   Backward: a group of lanes owns a run of samples, lane j the quads j, j + G, ... (G = next power
-//   of two >= Q).
+//   Backward: with a workspace the rows are ordered by cell and groups of as many lanes as the wider of the
+//   order's plane and line has quads walk them (sorted_bwd_kernel); without one, a group of G lanes (next power
+//   of two >= Q) owns a run of samples, lane j the quads j, j + G, ...
 //
 // Arithmetic follows grid_sample's op order: source index ((x + 1) / 2) * (size - 1), corner
 // weights as products of the opposite distances, taps accumulated nw, ne, sw, se; the file is
@@ -776,7 +777,7 @@ __device__ __forceinline__ WaveRun wave_run(int key, bool active) {
 //
 // The passes are bound by the device-scope atomics (about 9 G/s): the count pass keeps what its atomics return,
 // each row's rank within its cell, so that the scatter pass needs none.  Count and scatter of the samples of
-// 3.6M that a mask leaves: 100 + 100 -> 67 + 30 us; of 1.45M appearance rows: 140 + 190 -> 140 + 54 us.
+// 3.6M that a mask leaves: 100 + 100 -> 67 + 30 us; of 1.45M appearance rows: 140 + 190 -> 102 + 55 us.
 template <bool kDensity, bool kScatter>
 __global__ __launch_bounds__(256) void cell_count_kernel(VmArgs a, BwdRows r, SortWs w) {
   const int64_t n = bwd_rows_count(r);
